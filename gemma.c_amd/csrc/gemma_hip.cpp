@@ -368,6 +368,59 @@ int build_jobs(const char *fn, const gemma_hip_job *jobs, int njobs,
   return 0;
 }
 
+// Attention workspaces of the entry points that take device buffers, one per
+// (device, stream): launches on one stream run in order, so they can share
+// it.  Grown on demand, kept for the next call and freed by shutdown; past
+// kAttnWsKeep bytes in all, the other streams' go.  A caller holds g_attn_mu
+// from attn_workspace to its last launch, so that no other thread frees what
+// it is about to use.
+constexpr size_t kAttnWsKeep = (size_t)1 << 30;
+struct AttnWs {
+  char *p = nullptr;
+  size_t bytes = 0;
+};
+std::mutex g_attn_mu;
+std::map<std::pair<int, hipStream_t>, AttnWs> g_attn_ws;
+
+void attn_workspaces_free(const AttnWs *but) {  // hipFree waits for the device's queued work
+  for (auto it = g_attn_ws.begin(); it != g_attn_ws.end();) {
+    if (&it->second == but) {
+      ++it;
+      continue;
+    }
+    if (it->second.p != nullptr) (void)hipFree(it->second.p);
+    it = g_attn_ws.erase(it);
+  }
+}
+
+hipError_t attn_workspace(hipStream_t stream, size_t bytes, char **out) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  AttnWs &w = g_attn_ws[{dev, stream}];
+  if (w.bytes < bytes) {
+    size_t total = bytes;
+    for (const auto &kv : g_attn_ws)
+      if (&kv.second != &w) total += kv.second.bytes;
+    if (total > kAttnWsKeep) attn_workspaces_free(&w);
+    // calls already queued on the stream may still use the old buffer
+    if (w.p != nullptr &&
+        ((e = hipStreamSynchronize(stream)) != hipSuccess || (e = hipFree(w.p)) != hipSuccess))
+      return e;
+    w.p = nullptr;
+    w.bytes = 0;
+    if ((e = hipMalloc((void **)&w.p, bytes)) != hipSuccess) return e;
+    w.bytes = bytes;
+  }
+  *out = w.p;
+  return hipSuccess;
+}
+
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
 constexpr int kMaxGemvK8 = 65536;   // int8 vector staged in 64 KB of LDS
 constexpr int kMaxGemvK32 = 16384;  // fp32 vector staged in 64 KB of LDS
 
@@ -414,6 +467,10 @@ void gemma_hip_shutdown(void) {
     g_perf.on = false;
   }
   gh::release_gemm_workspaces();
+  {
+    std::lock_guard<std::mutex> hold(g_attn_mu);
+    attn_workspaces_free(nullptr);
+  }
   {
     std::lock_guard<std::mutex> guard(g.lock);
     for (auto &kv : g.regions) (void)hipFree(kv.second.device);
@@ -858,8 +915,15 @@ int gemma_hip_vision_attention(float *out, const float *qkv, const float *bias, 
   if (mode != GEMMA_HIP_ATTN_F64 && mode != GEMMA_HIP_ATTN_F32)
     return fail("gemma_hip_vision_attention: unknown mode %d", mode);
   const gh::VisAttn at{qkv, 3 * dim, bias, out, n, n_heads, dim, 1.0f / sqrtf((float)hdim)};
+  hipStream_t s = pick_stream(stream);
+  const bool f32 = mode == GEMMA_HIP_ATTN_F32;
+  char *planes = nullptr;
+  std::unique_lock<std::mutex> hold(g_attn_mu);
+  if (f32 && !capturing(s))  // a captured call can't allocate: the kernel without a workspace
+    GH_CHECK("gemma_hip_vision_attention: workspace",
+             attn_workspace(s, gh::attn_planes_bytes(hdim, n_heads, n), &planes));
   GH_CHECK("gemma_hip_vision_attention: launch",
-           gh::launch_vis_attention(at, hdim, mode == GEMMA_HIP_ATTN_F32, pick_stream(stream)));
+           gh::launch_vis_attention(at, hdim, f32, planes, g.info, s));
   return 0;
 }
 
@@ -2046,6 +2110,7 @@ struct gemma_hip_vision {
   float *img = nullptr, *patches = nullptr, *x = nullptr, *y = nullptr, *qkv = nullptr;
   float *att = nullptr, *hbuf = nullptr, *hln = nullptr, *out = nullptr, *as = nullptr;
   int8_t *a8 = nullptr;
+  char *planes = nullptr;  // the attention's packed K and V tiles
 };
 
 namespace {
@@ -2099,7 +2164,8 @@ hipError_t vision_enqueue(gemma_hip_vision *v, hipStream_t st) {
       return e;
     const gh::VisAttn at{v->qkv, 3 * dim, L.bqkv, v->att, n, c.n_heads, dim,
                          1.0f / sqrtf((float)v->hdim)};
-    if ((e = GH_OP(kOpSoftmax, gh::launch_vis_attention(at, v->hdim, v->attn_f32, st))) !=
+    if ((e = GH_OP(kOpSoftmax, gh::launch_vis_attention(at, v->hdim, v->attn_f32, v->planes,
+                                                              g.info, st))) !=
         hipSuccess)
       return e;
     // o (4563-4573), then its bias, the residual and the second layer norm
@@ -2173,7 +2239,8 @@ hipError_t vision_enqueue_f32(gemma_hip_vision *v, hipStream_t st) {
       return e;
     const gh::VisAttn at{v->qkv, 3 * dim, L.bqkv, v->att, n, c.n_heads, dim,
                          1.0f / sqrtf((float)v->hdim)};
-    if ((e = GH_OP(kOpSoftmax, gh::launch_vis_attention(at, v->hdim, v->attn_f32, st))) !=
+    if ((e = GH_OP(kOpSoftmax, gh::launch_vis_attention(at, v->hdim, v->attn_f32, v->planes,
+                                                              g.info, st))) !=
         hipSuccess)
       return e;
     if ((e = gemm(v->y, dim, L.wf[3], n, dim, v->att, dim, dim)) != hipSuccess) return e;
@@ -2316,7 +2383,8 @@ gemma_hip_vision *vision_build(const char *name, const gemma_hip_vision_config *
                o_y = cv.take(n * dim * 4), o_qkv = cv.take(n * 3 * dim * 4),
                o_att = cv.take(n * dim * 4), o_h = cv.take(n * mlp * 4),
                o_hln = cv.take(n * dim * 4), o_out = cv.take((size_t)c.img_tok * c.text_dim * 4),
-               o_a8 = cv.take(n * std::max(dim, mlp)), o_as = cv.take(n * 4);
+               o_a8 = cv.take(n * std::max(dim, mlp)), o_as = cv.take(n * 4),
+               o_pl = cv.take(gh::attn_planes_bytes(hdim, c.n_heads, v->npatch));
   hipError_t e = hipMalloc((void **)&v->mem, cv.used);
   if (e != hipSuccess) {
     hip_fail(name, e);
@@ -2366,6 +2434,7 @@ gemma_hip_vision *vision_build(const char *name, const gemma_hip_vision_config *
   v->hln = (float *)(m + o_hln);
   v->out = (float *)(m + o_out);
   v->a8 = (int8_t *)(m + o_a8);
+  v->planes = m + o_pl;
   v->as = (float *)(m + o_as);
   return v;
 }

@@ -314,6 +314,9 @@ struct PfAttn {
   int8_t *xq;
   float *xs;
 };
+// Bytes of the packed K and V tiles (attn_split.h) of `keys` keys, the tiles'
+// exponents included.
+size_t attn_planes_bytes(int hdim, int heads, int keys);
 constexpr int kPfMaxSplit = 8;
 constexpr int kPfMaxMergeHeads = 64;  // q heads the key-split merge handles
 // doubles of PfAttn::part for n rows
@@ -374,7 +377,10 @@ struct VisPool {
 hipError_t launch_vis_ln_rows(const VisLn &a, int n, hipStream_t stream);
 // head dim 16, 32, 64, 72 or 128
 // f32: on the fp32 matrix cores (otherwise fp64, rounded once)
-hipError_t launch_vis_attention(const VisAttn &a, int hdim, bool f32, hipStream_t stream);
+// planes: room for attn_planes_bytes(hdim, n_heads, n), or null (the kernel
+// that needs none runs then: slower, for callers that cannot allocate)
+hipError_t launch_vis_attention(const VisAttn &a, int hdim, bool f32, char *planes,
+                                const DeviceInfo &dev, hipStream_t stream);
 hipError_t launch_vis_gelu_quant(const float *h, const float *bias, int n, int mlp, int8_t *xq,
                                  float *xs, const WarmRegions &warm, hipStream_t stream);
 hipError_t launch_vis_pool(const VisPool &a, int ntok, hipStream_t stream);

@@ -15,6 +15,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "attn_split.h"
 #include "dec_common.h"
 
 namespace gh {
@@ -629,7 +630,8 @@ hipError_t launch_vis_ln_rows(const VisLn &a, int n, hipStream_t stream) {
   return go(std::integral_constant<int, 256>{});
 }
 
-// The fp32 mode's attention on the bf16 matrix cores: every fp32 operand x
+// The fp32 mode's attention without a workspace (calls under stream capture,
+// which can't allocate one), on the bf16 matrix cores: every fp32 operand x
 // of the two products (q, k, the probabilities p and v) is split into three
 // bf16 pieces x = x0 + x1 + x2 (each rounded to nearest from the remainder,
 // so together they hold x's 24 significant bits), and each product a.b is
@@ -904,17 +906,101 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void vis_attn_bf3_kernel(VisAttn 
   }
 }
 
-// The fp32 mode's kernel: the split bf16 one by default, the fp32-MFMA one
-// with GEMMA_HIP_VIS_ATTN=f32.  Read at every launch (one getenv per layer),
+// The fp32 mode's attention on the f16 matrix cores in split precision
+// (attn_split.h): NW waves x 32 queries of one head over tiles that
+// attn_pack_kernel made of K and V with their biases.  Bound by the matrix
+// cores at the clock that the chip holds under them: SigLIP at 896 px (4096
+// patches, 16 heads of 72) takes 30 products per 32 queries and tile, 258
+// TFLOP of f16 in 222 us (1.2 PFLOP/s; v_mfma_f32_32x32x16_f16 on random
+// registers alone sustains 1.6), packing 18 us.  The three-bf16-piece kernel
+// before it took 426 us at the same matrix rate with twice the products, and
+// its error against 64-bit sums was larger: 9.6e-7 relative, here 7.0e-7 (fewer
+// fp32 roundings per sum).  The tower's image (9 of 27 layers): 6.73 -> 4.7 ms.
+template <int HD, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, const char *planes,
+                                                                   const int2 *exps, int ntiles) {
+  typedef AttnTile<HD> G;
+  constexpr int QB = NW * 32;
+  __shared__ __attribute__((aligned(16))) char lds[2 * G::kBytes];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5;
+  // each XCD's workgroups share one head's tiles in its L2
+  const int nqb = (a.n + QB - 1) / QB, nblk = nqb * a.n_heads;
+  int blk = blockIdx.x;
+  if (nblk % 8 == 0) blk = (blk % 8) * (nblk / 8) + blk / 8;
+  const int h = blk / nqb;
+  const int qr = (blk - h * nqb) * QB + wave * 32 + (lane & 31);
+  AttnWave<HD, NW> w;
+  const int eq = w.load_q(a.qkv + (size_t)min(qr, a.n - 1) * a.stride + h * HD, a.bias + h * HD,
+                          half);
+  float c_hi, c_lo;
+  log2_scale(a.scale, eq, &c_hi, &c_lo);
+  const AttnSee see{0, a.n - 1, 0, a.n - 1};
+  w.run(planes + (size_t)h * ntiles * G::kBytes, exps + (size_t)h * ntiles, 0, ntiles - 1, see,
+        0.0f, c_hi, c_lo, 0.0f, lds, wave, lane);
+  if (qr >= a.n) return;
+  float *orow = a.out + (size_t)qr * a.dim + h * HD;
+  w.each(half, [&](int d, v4f x) {
+    *reinterpret_cast<v4f *>(orow + d) = ldexp4(x / w.l, w.e_o);
+  });
+}
+
+template <int HD>
+void launch_vis_split(const VisAttn &a, char *planes, const DeviceInfo &dev, hipStream_t stream) {
+  const int ntiles = (a.n + 31) / 32;
+  int2 *exps = reinterpret_cast<int2 *>(planes + (size_t)a.n_heads * ntiles * AttnTile<HD>::kBytes);
+  const AttnPack pk{a.qkv + a.dim, a.qkv + 2 * a.dim, (size_t)a.stride, (size_t)HD,
+                    a.bias + a.dim, a.bias + 2 * a.dim, 0, ntiles, a.n, planes, exps};
+  attn_pack_kernel<HD><<<dim3(ntiles, a.n_heads, 2), kPackThreads<HD>, 0, stream>>>(pk);
+  // 128 queries a workgroup while those have a CU each (784 patches, 16 heads:
+  // 39 us against 50 with 256; 2401 patches, 12 heads: 77 against 103), else
+  // 256, which share each tile's way to LDS (4096 patches: 243 against 250)
+  const int few = (a.n + 127) / 128 * a.n_heads;
+  if (few <= dev.cus)
+    vis_attn_split_kernel<HD, 4><<<few, 256, 0, stream>>>(a, planes, exps, ntiles);
+  else
+    vis_attn_split_kernel<HD, 8><<<(a.n + 255) / 256 * a.n_heads, 512, 0, stream>>>(a, planes, exps,
+                                                                                   ntiles);
+}
+
+// The fp32 mode's kernel: a split one by default (f16 pieces with a workspace,
+// bf16 pieces without), the fp32-MFMA one with GEMMA_HIP_VIS_ATTN=f32.  Read at every launch (one getenv per layer),
 // so that one process can time or check both.
 bool vis_attn_split() {
   const char *e = getenv("GEMMA_HIP_VIS_ATTN");
   return e == nullptr || strcmp(e, "f32") != 0;
 }
 
-hipError_t launch_vis_attention(const VisAttn &a, int hdim, bool f32, hipStream_t stream) {
+size_t attn_planes_bytes(int hdim, int heads, int keys) {
+  const size_t tiles = (size_t)heads * ((keys + 31) / 32);
+  size_t tile = 0;
+  switch (hdim) {
+    case 16: tile = AttnTile<16>::kBytes; break;
+    case 32: tile = AttnTile<32>::kBytes; break;
+    case 64: tile = AttnTile<64>::kBytes; break;
+    case 72: tile = AttnTile<72>::kBytes; break;
+    case 128: tile = AttnTile<128>::kBytes; break;
+    case 256: tile = AttnTile<256>::kBytes; break;
+  }
+  return tiles * (tile + sizeof(int2));
+}
+
+hipError_t launch_vis_attention(const VisAttn &a, int hdim, bool f32, char *planes,
+                                const DeviceInfo &dev, hipStream_t stream) {
   constexpr int NW = kVaWaves;
   const dim3 grid((a.n + NW * 16 - 1) / (NW * 16) * a.n_heads);
+  if (f32 && planes != nullptr && vis_attn_split()) {
+    switch (hdim) {
+      case 16: launch_vis_split<16>(a, planes, dev, stream); break;
+      case 32: launch_vis_split<32>(a, planes, dev, stream); break;
+      case 64: launch_vis_split<64>(a, planes, dev, stream); break;
+      case 72: launch_vis_split<72>(a, planes, dev, stream); break;
+      case 128: launch_vis_split<128>(a, planes, dev, stream); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   if (f32 && vis_attn_split()) {
     // 16-wave workgroups (256 queries share each staged and split tile):
     // SigLIP 896 px 19.24-19.39 -> 17.86-17.95 ms per image against 8 waves

@@ -486,13 +486,15 @@ int gemma_hip_vision_forward(gemma_hip_vision *vis, const float *img, float *out
  *   GEMMA_HIP_ATTN_F32 (the default) -- fp32 throughout as the reference
  *     computes it (its summation order differs), so results agree with the
  *     exact form to fp32 rounding, amplified where a later int8 quantization
- *     flips.  The patch GEMM runs on the fp32 matrix cores; the attention on
- *     the bf16 ones in split precision: each fp32 operand is the sum of three
- *     bf16 pieces and every product is summed from the six piece products
- *     down to 2^-16 of the leading one, which leaves an error per product of
- *     order 2^-23 relative, the size of an fp32 rounding, with fp32
- *     accumulation (the environment variable GEMMA_HIP_VIS_ATTN=f32, read
- *     once, selects the plain fp32 matrix-core kernel instead);
+ *     flips.  The patch GEMM runs on the bf16 matrix cores in split precision
+ *     and the attention on the f16 ones: each fp32 operand is scaled by a
+ *     power of two and split into two f16 pieces (22 significant bits), every
+ *     product is summed from three piece products in fp32, and the result is
+ *     closer to the exact one than with three bf16 pieces and six products
+ *     (fewer fp32 roundings).  gemma_hip_vision_attention on a stream under
+ *     capture, which can't allocate a workspace, takes the three-piece kernel;
+ *     the environment variable GEMMA_HIP_VIS_ATTN=f32, read at every launch,
+ *     selects the plain fp32 matrix-core kernel instead;
  *   GEMMA_HIP_ATTN_F64 -- fp64 (matrix cores for the attention), every
  *     output rounded once from the exact sum: the verification mode, equal
  *     to an fp64 evaluation of the same formulas.
