@@ -245,7 +245,7 @@ constexpr int kAttnReach = 64;        // octaves between tiles of V that one que
 // Tiles are double-buffered, one barrier each; the next tile's scores are
 // computed in the same stretch as this tile's weights, so that the vector
 // unit works while the matrix cores do.
-template <int HD, int NW>
+template <int HD, int NW, bool CAP = false>
 struct AttnWave {
   typedef AttnTile<HD> G;
   h8 q[G::KF][2];
@@ -366,19 +366,20 @@ struct AttnWave {
   // units lie below the sums' (<= 0), for the weights to carry.  A tile more
   // than kAttnReach octaves below the sums is out of their reach: it only adds
   // its weights to l, here (with the returned -1000 they vanish elsewhere).
-  __device__ __forceinline__ int refer(const v16f &x, float c1, float c2, float top2, int ev) {
+  __device__ __forceinline__ int refer(const v16f &x, float c1, float c2, float top2, int ev,
+                                       bool first) {
     if (__any(top2 > m2 + (float)kAttnTop)) {
       const float rmax = fmaxf(top2, __shfl_xor(top2, 32, 64));
       const float m_new = fmaxf(m2, ceilf(rmax) - (float)kAttnSet);
       const float alpha = __builtin_amdgcn_exp2f(m2 - m_new);  // a power of two, or 0
       m2 = m_new;
       l *= alpha;
-      scale_o(alpha);
+      if (!first) scale_o(alpha);
     }
     int df = ev - e_o;
     if (df > 0 || df < -8) {  // wave-uniform
       if (df >= -kAttnReach) {
-        scale_o(ldexpf(1.0f, max(-df, -300)));
+        if (!first) scale_o(ldexpf(1.0f, max(-df, -300)));
         e_o = ev;
         df = 0;
       } else {
@@ -440,12 +441,18 @@ struct AttnWave {
     lds_barrier();                       // every wave's did
     if (ta < tb) fetch_k(ta + 1);
     v16f sc = {};
-    each_chunk(std::integral_constant<int, kQ>{}, [&](auto I) {
-      h8 f[2];
+    {
+      const char *k0 = kbuf + (ta & 1) * (G::KFR * 1024) + loff;
       const h8 none[2][2] = {};
-      read<I>(kbuf + (ta & 1) * (G::KFR * 1024) + loff, nullptr, f);
-      product<I>(f, none, sc);
-    });
+      h8 f[kQ][2];
+      each_chunk(std::integral_constant<int, (kQ < 4 ? kQ : 4)>{}, [&](auto I) { read<I>(k0, nullptr, f[I]); });
+      __builtin_amdgcn_sched_barrier(0);
+      each_chunk(std::integral_constant<int, kQ>{}, [&](auto I) {
+        if constexpr (I + 4 < kQ) read<I + 4>(k0, nullptr, f[I + 4]);
+        product<I>(f[I], none, sc);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    }
     // The tile loop is turned so that what rarely happens (refer) lies outside
     // the inner loop: in it the value sums are touched by the matrix cores
     // alone and stay in the accumulation registers.
@@ -472,7 +479,7 @@ struct AttnWave {
       // 2^38) and would let the masked ones come up
       c1 = fmaxf(ldexpf(c_hi, ek), 0x1p-70f);
       c2 = ldexpf(c_lo, ek);
-      if (cap != 0.0f) {  // capped scores, in units of the scaled score
+      if constexpr (CAP) {  // capped scores, in units of the scaled score
         const float as = ldexpf(asc, ek);
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[r] = tanhf(sc[r] * as / cap) * cap;
@@ -496,7 +503,7 @@ struct AttnWave {
     int t = ta;
     begin(t);
     for (;;) {
-      int df = refer(sc, c1, c2, top2, ev);
+      int df = refer(sc, c1, c2, top2, ev, t == ta);
       do {
         const float m = m2 - (float)df;
         const char *kn = kbuf + ((t + 1) & 1) * (G::KFR * 1024) + loff;

@@ -946,10 +946,12 @@ int gemma_hip_prefill_attention(float *out, const float *q, int q_stride, const 
     return fail("%s: unknown mode %d", name, mode);
   hipStream_t s = pick_stream(stream);
   double *part = nullptr;
+  const size_t part_bytes = gh::pf_attn_part_doubles(n, n_heads, hdim) * sizeof(double);
   GH_CHECK("gemma_hip_prefill_attention: workspace",
-           hipMalloc(&part, gh::pf_attn_part_doubles(n, n_heads, hdim) * sizeof(double)));
+           hipMalloc(&part, part_bytes + gh::attn_planes_bytes(hdim, nkv, pos0 + n)));
   const gh::PfAttn at{q, q_stride, kc, vc, out, n_heads * hdim, n, pos0, n_heads, nkv, clen,
-                      slide, asc, sc_att, part, 0, 0, 0, dense ? 1 : 0};
+                      slide, asc, sc_att, part, 0, 0, 0, dense ? 1 : 0, nullptr, nullptr,
+                      (char *)part + part_bytes, 0};
   hipError_t e = gh::launch_pf_attention(at, hdim, mode == GEMMA_HIP_ATTN_F32, g.info, s);
   const hipError_t e2 = hipStreamSynchronize(s);
   (void)hipFree(part);
@@ -1250,6 +1252,7 @@ struct gemma_hip_decoder {
   float *pf_h = nullptr;  // normalized rows ('U': the fp32 GEMMs' input)
   int *pf_tok = nullptr;
   double *pf_part = nullptr;  // attention key-split partials
+  char *pf_planes = nullptr;  // ... and packed K and V tiles
 };
 
 namespace {
@@ -1279,7 +1282,8 @@ int prefill_reserve(gemma_hip_decoder *d, int n) {
                o_g = cv.take(rows * 2 * mlp * 4), o_a8 = cv.take(rows * kmax),
                o_as = cv.take(rows * 4), o_tok = cv.take(rows * 4),
                o_part = cv.take(gh::pf_attn_part_doubles(rows, c.n_heads, c.hdim) * 8),
-               o_h = cv.take(d->quant ? 0 : rows * dim * 4);
+               o_h = cv.take(d->quant ? 0 : rows * dim * 4),
+               o_pl = cv.take(gh::attn_planes_bytes(c.hdim, c.nkv, d->clen));
   if (d->pf_mem != nullptr) {
     (void)hipStreamSynchronize(g.stream);
     (void)hipFree(d->pf_mem);
@@ -1299,6 +1303,7 @@ int prefill_reserve(gemma_hip_decoder *d, int n) {
   d->pf_tok = (int *)(m + o_tok);
   d->pf_part = (double *)(m + o_part);
   d->pf_h = d->quant ? nullptr : (float *)(m + o_h);
+  d->pf_planes = m + o_pl;
   d->pf_rows = n;
   return 0;
 }
@@ -1360,7 +1365,7 @@ hipError_t prefill_enqueue(gemma_hip_decoder *d, int n, int pos, bool embed, boo
     const gh::PfAttn at{d->pf_qkv, stride, kc, kc + cache, d->pf_xo, q_sz, n, pos, c.n_heads,
                         c.nkv, d->clen, sliding ? c.slide : 0,
                         (float)(1.0f / sqrtf((float)c.q_scale)), c.sc_att, d->pf_part, 0, 0,
-                        0, dense ? 1 : 0, d->pf_a8, d->pf_as};
+                        0, dense ? 1 : 0, d->pf_a8, d->pf_as, d->pf_planes, 0};
     if ((e = GH_OP(kOpSoftmax, gh::launch_pf_attention(at, c.hdim, d->attn_f32, g.info, st))) !=
         hipSuccess)
       return e;
@@ -1592,7 +1597,7 @@ hipError_t prefill_enqueue_f32(gemma_hip_decoder *d, int n, int pos, bool embed,
     const gh::PfAttn at{d->pf_qkv, stride, kc, kc + cache, d->pf_xo, q_sz, n, pos, c.n_heads,
                         c.nkv, d->clen, sliding ? c.slide : 0,
                         (float)(1.0f / sqrtf((float)c.q_scale)), c.sc_att, d->pf_part, 0, 0,
-                        0, dense ? 1 : 0};
+                        0, dense ? 1 : 0, nullptr, nullptr, d->pf_planes, 0};
     if ((e = GH_OP(kOpSoftmax, gh::launch_pf_attention(at, c.hdim, d->attn_f32, g.info, st))) !=
         hipSuccess)
       return e;

@@ -313,6 +313,10 @@ struct PfAttn {
   // xo then holds only the rows the attention kernel wrote whole
   int8_t *xq;
   float *xs;
+  // fp32 mode: room for the split kernel's packed K and V tiles of keys
+  // 0 .. pos0+n-1 (attn_planes_bytes); null: the fp32-MFMA kernel only
+  char *planes;
+  int log2m;  // partials' reference maxima are base-2 logarithms (set by the launcher)
 };
 // Bytes of the packed K and V tiles (attn_split.h) of `keys` keys, the tiles'
 // exponents included.

@@ -34,6 +34,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "attn_split.h"
 #include "dec_common.h"
 
 namespace gh {
@@ -194,6 +195,7 @@ __host__ __device__ __forceinline__ PaRange pa_range(const PfAttn &a, int r0, in
 // 437 us).  A chunk is chunk_id's run of a.chunk keys of the row block's key
 // range (its first row's window start, rounded down to 32, to its last row's
 // position).
+template <int QW = 16>  // query vectors per wave
 __device__ __forceinline__ PaLane pa_lane(const PfAttn &a, int wave, int col) {
   PaLane L;
   const int hn = a.n_heads / a.nkv, qb = a.qpb / hn;
@@ -208,7 +210,7 @@ __device__ __forceinline__ PaLane pa_lane(const PfAttn &a, int wave, int col) {
   L.empty = L.chunk_id >= L.nchunks;
   L.k_lo = k_base + L.chunk_id * a.chunk;
   L.k_end = min(L.k_lo + a.chunk - 1, p_last);
-  const int v = 16 * wave + col;
+  const int v = QW * wave + col;
   L.valid = v % qb < L.rows;
   L.row = L.r0 + min(v % qb, L.rows - 1);
   L.head = L.hk * hn + v / qb;
@@ -602,190 +604,58 @@ __global__ __launch_bounds__(kNT, 2) void pf_attn_f32_kernel(PfAttn a) {
   }
 }
 
-// The same attention on the bf16 matrix cores in split precision: q, k, the
-// weights p and v each as three bf16 pieces (split3x2), every product summed
-// from its six leading piece products (v_mfma_f32_16x16x32_bf16, the small
-// ones first) with fp32 accumulation, so the error per product is of the
-// size of an fp32 rounding and the result agrees with the fp64 form to fp32
-// rounding, as pf_attn_f32_kernel's does, at ~2.5x its matrix-core rate.
-// A workgroup is kPbWaves waves x 16 query vectors (one workgroup per CU:
-// the planes below take most of the LDS).  Key tiles of 32, whose K rows go
-// by LDS DMA into an fp32 staging buffer and whose V rows (4 keys x 4 dims
-// per thread) into registers while the tile before is in use; at a tile's
-// start the workgroup splits both, once for all its waves, into three bf16
-// planes each: K [key][dim] and V^T [dim][k], where k = 8 g + 4 b + r is the
-// value product's index of key 16 b + 4 g + r -- the key whose score lane
-// (query, g) holds in element r of block b, so a lane's eight weights are
-// its operand of that product as they stand.  Lane (query col, g) holds the
-// query's dims 32 c + 8 g .. + 7 of every piece and the outputs' dims
-// 16 nb + 4 g .. + 3.  Masks, softmax and partials as pf_attn_f32_kernel.
-constexpr int kPbWaves = 8;
-constexpr int kPbQ = kPbWaves * 16;  // query vectors per workgroup
+// The fp32 mode's attention on the f16 matrix cores in split precision
+// (attn_split.h): a workgroup is kPbWaves waves x 32 query vectors (128: one kv
+// head's q heads at 128 / hn rows), and its tiles are the cache's keys packed by
+// attn_pack_kernel.  At head dim 256 a wave holds its queries' pieces and the
+// value sums in 256 registers, so each SIMD runs one wave and a CU one
+// workgroup (128 KB of LDS); the tile loop overlaps its softmax with the next
+// tile's score products by itself.  A tile of 32 keys takes 2.7 us, 2.4 of them
+// with its loads and LDS reads taken out: the 96 products of a wave at the clock
+// that the chip holds under f16 products on all CUs.  gemma-3-4b, 2048 rows,
+// window 1024: packing 11, kernel 63, merge 11 us, where three bf16 pieces with
+// six products, split in the kernel, took 111 + 11; global layers 12 + 71 + 11
+// against 135 + 11.  Error against 64-bit sums 4.0e-7 -> 3.3e-7 relative.
+constexpr int kPbWaves = 4;
+constexpr int kPbQ = kPbWaves * 32;  // query vectors per workgroup
 
-template <int HD>
-__global__ __launch_bounds__(kPbWaves * 64) void pf_attn_bf3_kernel(PfAttn a) {
-  constexpr int NT = kPbWaves * 64;
-  constexpr int TK = 32;          // keys per tile
-  constexpr int CH = HD / 32;     // 32-dim chunks of the score product
-  constexpr int NB = HD / 16;     // 16-dim output blocks
-  constexpr int C4 = HD / 4;      // float4 per key row
-  constexpr int RK = HD + 8;      // K plane row (bf16): 8 rows in distinct banks
-  constexpr int RV = TK + 8;      // V^T plane row (bf16)
-  constexpr int SG = TK * C4;     // float4 of a K tile
-  constexpr int NIW = SG / 64 / kPbWaves;  // K DMA instructions per wave and tile
-  constexpr int PF = (SG + NT - 1) / NT;   // K float4 split per thread
-  constexpr int VB = 8 * C4;               // V blocks (4 keys x 4 dims) per tile
-  static_assert(HD % 64 == 0 && TK == kPaKeys && NIW * 64 * kPbWaves == SG && VB <= NT,
-                "tile staging");
-  __shared__ __attribute__((aligned(16))) __bf16 kt[3][TK * RK];
-  __shared__ __attribute__((aligned(16))) __bf16 vt[3][HD * RV];
-  __shared__ v4f stg[SG];
-
+template <int HD, bool CAP>
+__global__ __launch_bounds__(kPbWaves * 64, HD == 256 ? 1 : 2) void pf_attn_split_kernel(
+    PfAttn a, const int2 *exps, int tile0, int ntiles) {
+  typedef AttnTile<HD> G;
+  __shared__ __attribute__((aligned(16))) char lds[2 * G::kBytes];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 15, grp = lane >> 4;
-  const PaLane L = pa_lane(a, wave, col);
+  const int col = lane & 31, half = lane >> 5;
+  const PaLane L = pa_lane<32>(a, wave, col);
   if (L.empty) return;  // the whole block: before any barrier
-  bf8 qa[3][CH];
-  {
-    const float *qrow = a.qkv + (size_t)L.row * a.stride + L.head * HD + 8 * grp;
+  AttnSee see{L.ws, L.p_top, L.valid ? L.ws : 0, L.valid ? L.p_top : INT_MAX};
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      u4 w0, w1, w2;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const v4f q4 = *reinterpret_cast<const v4f *>(qrow + 32 * c + 4 * h);
-#pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          const Bf3x2 sp = split3x2(q4[e], q4[e + 1]);
-          w0[2 * h + e / 2] = sp.q0;
-          w1[2 * h + e / 2] = sp.q1;
-          w2[2 * h + e / 2] = sp.q2;
-        }
-      }
-      qa[0][c] = as_bf8(w0);
-      qa[1][c] = as_bf8(w1);
-      qa[2][c] = as_bf8(w2);
-    }
+  for (int off = 1; off < 32; off <<= 1) {
+    see.f_lo = max(see.f_lo, __shfl_xor(see.f_lo, off, 64));
+    see.f_hi = min(see.f_hi, __shfl_xor(see.f_hi, off, 64));
   }
-  v4f o[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) o[nb] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m_ref = kPaFloorF, l_part = 0.0f;
-  const float *kc = a.kc + (size_t)L.hk * a.clen * HD;
-  const float *vc = a.vc + (size_t)L.hk * a.clen * HD;
-
-  // rows past the chunk's last key repeat it: their weights are exactly 0
-  const int vtq = tid % 8, vc4 = tid / 8;  // this thread's V block (tid < VB)
-  v4f vr[4];
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int j = 0; j < NIW; ++j) {
-      const int i = wave * NIW + j;  // wave-uniform
-      const int ch = 64 * i + lane, t = ch / C4;
-      lds_dma16(kc + (size_t)min(t0 + t, L.k_end) * HD + 4 * (ch - t * C4),
-                reinterpret_cast<float *>(&stg[64 * i]));
-    }
-    if (tid < VB) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        vr[u] = *reinterpret_cast<const v4f *>(vc + (size_t)min(t0 + 4 * vtq + u, L.k_end) * HD +
-                                               4 * vc4);
-    }
-  };
-  fetch(L.k_lo);
-  for (int t0 = L.k_lo; t0 <= L.k_end; t0 += TK) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's K DMAs and V rows are in
-    lds_barrier();  // every wave's DMAs landed, every wave is done with the planes
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-      const int i = tid + j * NT;
-      if (i >= SG) break;
-      const int t = i / C4, c4 = i - t * C4;
-      const v4f kv = stg[i];
-      const Bf3x2 lo = split3x2(kv[0], kv[1]), hi = split3x2(kv[2], kv[3]);
-      *reinterpret_cast<u2 *>(&kt[0][t * RK + 4 * c4]) = u2{lo.q0, hi.q0};
-      *reinterpret_cast<u2 *>(&kt[1][t * RK + 4 * c4]) = u2{lo.q1, hi.q1};
-      *reinterpret_cast<u2 *>(&kt[2][t * RK + 4 * c4]) = u2{lo.q2, hi.q2};
-    }
-    if (tid < VB) {
-      const int k0i = 8 * (vtq % 4) + 4 * (vtq / 4);  // the value product's k of key 4 vtq
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const Bf3x2 lo = split3x2(vr[0][e], vr[1][e]), hi = split3x2(vr[2][e], vr[3][e]);
-        const int at = (4 * vc4 + e) * RV + k0i;
-        *reinterpret_cast<u2 *>(&vt[0][at]) = u2{lo.q0, hi.q0};
-        *reinterpret_cast<u2 *>(&vt[1][at]) = u2{lo.q1, hi.q1};
-        *reinterpret_cast<u2 *>(&vt[2][at]) = u2{lo.q2, hi.q2};
-      }
-    }
-    lds_barrier();  // the planes are complete; the staging buffer is free
-    if (t0 + TK <= L.k_end) fetch(t0 + TK);
-
-    if (t0 > L.w_hi || t0 + TK - 1 < L.w_lo) continue;  // wave-uniform
-    v4f sc[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      sc[b] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const int at = (16 * b + col) * RK + 32 * c + 8 * grp;
-        const bf8 k0 = *reinterpret_cast<const bf8 *>(&kt[0][at]);
-        const bf8 k1 = *reinterpret_cast<const bf8 *>(&kt[1][at]);
-        const bf8 k2 = *reinterpret_cast<const bf8 *>(&kt[2][at]);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qa[0][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qa[1][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[2][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qa[0][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[1][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[0][c], sc[b], 0, 0, 0);
-      }
-    }
-    pa_softmax_f32<NB, 2>(a, L, sc, t0, grp, m_ref, l_part, o);
-    u4 w0, w1, w2;  // weight k = 4 b + r of the lane's eight is dword 2 b + r / 2
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const Bf3x2 sp = split3x2(sc[b][r], sc[b][r + 1]);
-        w0[2 * b + r / 2] = sp.q0;
-        w1[2 * b + r / 2] = sp.q1;
-        w2[2 * b + r / 2] = sp.q2;
-      }
-    const bf8 p0 = as_bf8(w0), p1 = as_bf8(w1), p2 = as_bf8(w2);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int at = (16 * nb + col) * RV + 8 * grp;
-      const bf8 v0 = *reinterpret_cast<const bf8 *>(&vt[0][at]);
-      const bf8 v1 = *reinterpret_cast<const bf8 *>(&vt[1][at]);
-      const bf8 v2 = *reinterpret_cast<const bf8 *>(&vt[2][at]);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v2, p0, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, p1, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p2, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, p0, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p1, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p0, o[nb], 0, 0, 0);
-    }
-  }
-  float l = l_part + __shfl_xor(l_part, 16, 64);
-  l = l + __shfl_xor(l, 32, 64);
+  see.f_lo = __builtin_amdgcn_readfirstlane(see.f_lo);
+  see.f_hi = __builtin_amdgcn_readfirstlane(see.f_hi);
+  AttnWave<HD, kPbWaves, CAP> w;
+  const int eq = w.load_q(a.qkv + (size_t)L.row * a.stride + L.head * HD, nullptr, half);
+  float c_hi, c_lo;
+  log2_scale(a.asc, eq, &c_hi, &c_lo);
+  const size_t first = (size_t)L.hk * ntiles;
+  w.run(a.planes + first * G::kBytes - (size_t)tile0 * G::kBytes, exps + first - tile0,
+        L.k_lo / kPaKeys, L.k_end / kPaKeys, see, ldexpf(a.asc, eq), c_hi, c_lo, a.sc_att, lds,
+        wave, lane);
   if (!L.valid) return;
-  // dims 16 nb + 4 grp .. + 3 are o[nb]
-  if (L.nchunks == 1) {
-    float *orow = a.xo + (size_t)L.row * a.q_sz + L.head * HD + 4 * grp;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<v4f *>(orow + 16 * nb) = o[nb] / l;
-    return;
-  }
   float *pf = reinterpret_cast<float *>(a.part);
   const size_t at = (size_t)L.chunk_id * a.n + L.row;
-  float *prow = pf + at * a.q_sz + L.head * HD + 4 * grp;
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<v4f *>(prow + 16 * nb) = o[nb];
-  if (grp == 0) {
+  const bool one = L.nchunks == 1;
+  float *prow = (one ? a.xo + (size_t)L.row * a.q_sz : pf + at * a.q_sz) + L.head * HD;
+  const float f = one ? 1.0f / w.l : 1.0f;
+  w.each(half, [&](int d, v4f x) { *reinterpret_cast<v4f *>(prow + d) = ldexp4(x * f, w.e_o); });
+  if (!one && half == 0) {
     float *ml = pf + (size_t)kPfMaxSplit * a.n * a.q_sz + (at * a.n_heads + L.head) * 2;
-    ml[0] = m_ref;
-    ml[1] = l;
+    ml[0] = w.m2;
+    ml[1] = w.l;
   }
 }
 
@@ -968,7 +838,8 @@ __global__ __launch_bounds__(kNT) void pf_attn_merge_kernel(PfAttn a, int hdim) 
       double den = 0.0;
       for (int c = 0; c < nchunks; ++c) {
         const size_t at = ((size_t)c * a.n + row) * a.n_heads + h;
-        const double w = exp((double)ml[at * 2] - m);
+        const double d = (double)ml[at * 2] - m;
+        const double w = a.log2m ? exp2(d) : exp(d);
         wt[h][c] = w;
         den += w * (double)ml[at * 2 + 1];
       }
@@ -1151,20 +1022,19 @@ int pf_chunk(int kmax, int split) {
   return ((kmax + split - 1) / split + kPaKeys - 1) / kPaKeys * kPaKeys;
 }
 
-// The key split for the split-bf16 kernel, which runs one workgroup per CU:
-// each candidate split's blocks are dealt, in launch order (pa_lane's block
-// order), to the CU that frees first, each costing its chunk's tiles plus a
-// fixed prologue and epilogue of about two tiles (empty blocks next to
-// nothing), and the merge pass reads and writes the partials once per chunk.
-// Measured at the gemma-3-4b prefill (2048 rows, 8 q heads on 4 kv heads):
-// sliding layers 147 -> 124 us with two chunks instead of seven, global
-// layers 182 -> 146 us with three instead of eight (kernel + merge); this
-// model ranks the splits as the measurements do.
+// The key split for the split-f16 kernel, which runs one workgroup per CU (head
+// dim 256): each candidate split's blocks are dealt, in launch order (pa_lane's
+// block order), to the CU of their XCD that frees first, each costing its chunk's tiles plus
+// a fixed prologue and epilogue of about four tiles, and the merge pass reads and writes the partials once per chunk.
+// Measured, kernel + merge, 8 q heads on 4 kv heads: 2048 rows in a 1024-key
+// window 75 us in two chunks (one 96, three 98), global 80 in three (two 99,
+// four 115), 1024 global rows 47 in four (two 59, seven 61); this model ranks
+// the splits as the measurements do.
 // The plan is a host computation of a few thousand heap operations, and a
 // decoder asks for the same few shapes at every layer: the last plans are
 // kept (per thread).
-int pf_bf3_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int cus);
-int pf_bf3_split(const PfAttn &b, int hdim, int qb, int nrb, int kmax, int cus) {
+int pf_key_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int cus);
+int pf_key_split(const PfAttn &b, int hdim, int qb, int nrb, int kmax, int cus) {
   struct Key {
     int n, pos0, n_heads, nkv, q_sz, slide, dense, hdim, cus;
     bool operator==(const Key &o) const {
@@ -1179,7 +1049,7 @@ int pf_bf3_split(const PfAttn &b, int hdim, int qb, int nrb, int kmax, int cus) 
   const Key key{b.n, b.pos0, b.n_heads, b.nkv, b.q_sz, b.slide, b.dense, hdim, cus};
   for (int i = 0; i < used; ++i)
     if (keys[i] == key) return plans[i];
-  const int split = pf_bf3_split_plan(b, hdim, qb, nrb, kmax, cus);
+  const int split = pf_key_split_plan(b, hdim, qb, nrb, kmax, cus);
   keys[next] = key;
   plans[next] = split;
   next = (next + 1) % kKeep;
@@ -1187,14 +1057,15 @@ int pf_bf3_split(const PfAttn &b, int hdim, int qb, int nrb, int kmax, int cus) 
   return split;
 }
 
-int pf_bf3_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int cus) {
-  const double tile_us = 6.0 * hdim / 256.0, fixed_tiles = 2.0;
+int pf_key_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int cus) {
+  const double tile_us = 2.75 * hdim / 256.0, fixed_tiles = 4.0;
   const double merge_us = 0.143e-6 * 4.0 * (double)b0.n * b0.q_sz;  // per chunk
   const int max_split = std::min(kPfMaxSplit, (kmax + kPaKeys - 1) / kPaKeys);
   int best = 1, last_nsplit = 0;
   double best_cost = 0.0;
-  // free_at: a min-heap of the CUs' busy-until times
-  std::vector<double> free_at((size_t)std::max(cus, 1));
+  // free_at: a min-heap of the CUs' busy-until times per XCD (block b goes to
+  // XCD b % 8)
+  std::vector<double> free_at[8];
   const auto later = [](double x, double y) { return x > y; };
   for (int s = 1; s <= max_split; ++s) {
     PfAttn b = b0;
@@ -1202,7 +1073,7 @@ int pf_bf3_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int
     b.nsplit = (kmax + b.chunk - 1) / b.chunk;
     if (b.nsplit == last_nsplit) continue;
     last_nsplit = b.nsplit;
-    std::fill(free_at.begin(), free_at.end(), 0.0);
+    for (auto &f : free_at) f.assign((size_t)std::max(cus / 8, 1), 0.0);
     double makespan = 0.0;
     const int blocks = nrb * b.nsplit * b.nkv;
     for (int blk = 0; blk < blocks; ++blk) {
@@ -1212,15 +1083,16 @@ int pf_bf3_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int
       const int r0 = (nrb - 1 - blk / b.nkv / b.nsplit) * qb;
       const PaRange r = pa_range(b, r0, std::min(qb, b.n - r0));
       const int nch = (r.p_last - r.k_base + b.chunk) / b.chunk;
-      double cost = 0.05;
+      double cost = 3.0;  // an empty block's way onto a CU and off it
       if (cid < nch) {
         const int lo = r.k_base + cid * b.chunk, hi = std::min(lo + b.chunk - 1, r.p_last);
         cost = (hi - lo + kPaKeys) / kPaKeys + fixed_tiles;
       }
-      std::pop_heap(free_at.begin(), free_at.end(), later);
-      free_at.back() += cost;
-      makespan = std::max(makespan, free_at.back());
-      std::push_heap(free_at.begin(), free_at.end(), later);
+      auto &f = free_at[blk % 8];
+      std::pop_heap(f.begin(), f.end(), later);
+      f.back() += cost;
+      makespan = std::max(makespan, f.back());
+      std::push_heap(f.begin(), f.end(), later);
     }
     const double us = makespan * tile_us + merge_us * b.nsplit;
     if (s == 1 || us < best_cost) {
@@ -1232,17 +1104,31 @@ int pf_bf3_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int
 }
 
 // The fp32 mode's kernel, read at every launch so that one process can time
-// or check both: GEMMA_HIP_PF_ATTN=f32 the fp32-MFMA one, =bf3 the split-bf16
-// one; unset, the split-bf16 one unless the pass is so small that it would
-// have fewer than kPbMinBlocks workgroups, where the fp32-MFMA kernel's
-// smaller workgroups, two per CU, finish first (gemma-3-270m, 32 rows: one
-// split-bf16 workgroup, 19.8 us per layer against 13.5).
-constexpr int kPbMinBlocks = 32;
-enum PfKind { kPfF32, kPfBf3, kPfAuto };
+// or check both: GEMMA_HIP_PF_ATTN=f32 the fp32-MFMA one, =bf3 the split-f16
+// one; unset, the split-f16 one from kPbMinFlops of score and value products
+// on.  Below, its packing launch and its longer prologue (about 15 us together)
+// outweigh its rate, 2.5 times the other's: whole prompt passes, fp32-MFMA
+// against split, gemma-3-270m (6 layers) at 512 rows (0.8 GFLOP a layer) 611
+// against 660 us, 700 rows 679 / 694; gemma-3-4b (2 layers) at 400 rows (0.66)
+// 578 / 592, 512 (1.07) 640 / 639, 700 (2.0) 669 / 652.
+constexpr double kPbMinFlops = 1.1e9;  // at head dim 256; in proportion below
+enum PfKind { kPfF32, kPfSplit, kPfAuto };
 PfKind pf_attn_kind() {
   const char *e = getenv("GEMMA_HIP_PF_ATTN");
   if (e == nullptr) return kPfAuto;
-  return strcmp(e, "f32") == 0 ? kPfF32 : strcmp(e, "bf3") == 0 ? kPfBf3 : kPfAuto;
+  return strcmp(e, "f32") == 0 ? kPfF32 : strcmp(e, "bf3") == 0 ? kPfSplit : kPfAuto;
+}
+
+// Score and value products of the n rows: 4 hdim flops per head and (row, key)
+// pair that the row sees.
+double pa_flops(const PfAttn &a, int hdim) {
+  const double n = a.n, first = a.pos0 + 1.0, last = a.pos0 + n, w = a.slide;
+  double pairs = n * (first + last) / 2;
+  if (a.dense)
+    pairs = n * last;
+  else if (a.slide > 0 && last > w)  // rows past the window's length see w keys
+    pairs = first >= w ? n * w : (w - first) * (first + w) / 2 + (last - w + 1) * w;
+  return 4.0 * hdim * a.n_heads * pairs;
 }
 
 // Row blocks of qpb query vectors and the longest key range among them.
@@ -1267,25 +1153,23 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
   if (hn <= 0 || kPbQ % hn != 0 || kPaQ % hn != 0 || kPaQPair % hn != 0 || a.n <= 0 ||
       a.part == nullptr || a.n_heads > kPfMaxMergeHeads)
     return hipErrorInvalidValue;
-  bool bf3 = false;
+  bool splitk = false;  // the split-f16 kernel
   PaGeo geo{};
-  if (f32) {
+  if (f32 && a.planes != nullptr) {
     const PfKind kind = pf_attn_kind();
     if (kind != kPfF32) {
       geo = pa_geo(a, kPbQ);
-      const int most = geo.nrb * a.nkv *
-                       std::min(kPfMaxSplit, (geo.kmax + kPaKeys - 1) / kPaKeys);
-      bf3 = kind == kPfBf3 || most >= kPbMinBlocks;
+      splitk = kind == kPfSplit || pa_flops(a, hdim) >= kPbMinFlops * hdim / 256;
     }
   }
-  const int qpb = bf3 ? kPbQ : f32 ? kPaQ : hdim == 256 ? kPaQPair : kPaQ;
-  if (!bf3) geo = pa_geo(a, qpb);
+  const int qpb = splitk ? kPbQ : f32 ? kPaQ : hdim == 256 ? kPaQPair : kPaQ;
+  if (!splitk) geo = pa_geo(a, qpb);
   const int qb = geo.qb, nrb = geo.nrb, kmax = geo.kmax;
   // GEMMA_HIP_PF_BLOCKS (a tuning knob, read once): split the key ranges
   // until there are about that many blocks.  Otherwise the fp32-MFMA and fp64
   // kernels (two workgroups per CU) take about 2048 blocks (half of them
-  // empty for causal rows), and the split-bf16 kernel the split of
-  // pf_bf3_split.
+  // empty for causal rows), and the split-f16 kernel the split of
+  // pf_key_split.
   static const int knob = [] {
     const char *e = getenv("GEMMA_HIP_PF_BLOCKS");
     const int v = e != nullptr ? atoi(e) : 0;
@@ -1293,9 +1177,10 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
   }();
   PfAttn b = a;
   b.qpb = qpb;
+  b.log2m = splitk ? 1 : 0;
   int split;
-  if (bf3 && knob == 0) {
-    split = pf_bf3_split(b, hdim, qb, nrb, kmax, dev.cus);
+  if (splitk && knob == 0) {
+    split = pf_key_split(b, hdim, qb, nrb, kmax, dev.cus);
   } else {
     const int target = knob > 0 ? knob : 2048;
     const int want = (target + nrb * a.nkv - 1) / (nrb * a.nkv);
@@ -1304,10 +1189,25 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
   b.chunk = pf_chunk(kmax, split);
   b.nsplit = (kmax + b.chunk - 1) / b.chunk;
   const dim3 grid(nrb * b.nsplit * a.nkv);
-  if (bf3) {
+  if (splitk) {
+    // the keys that some row sees: from the first row's window start on
+    const int keys = a.pos0 + a.n;
+    const int tile0 = pa_range(b, 0, 1).k_base / kPaKeys;
+    const int ntiles = (keys + kPaKeys - 1) / kPaKeys - tile0;
+    auto go = [&](auto hd) {
+      constexpr int HD = decltype(hd)::value;
+      int2 *exps = reinterpret_cast<int2 *>(a.planes + (size_t)a.nkv * ntiles * AttnTile<HD>::kBytes);
+      const AttnPack pk{a.kc, a.vc, (size_t)HD, (size_t)a.clen * HD, nullptr, nullptr,
+                        tile0, ntiles, keys, a.planes, exps};
+      attn_pack_kernel<HD><<<dim3(ntiles, a.nkv, 2), kPackThreads<HD>, 0, stream>>>(pk);
+      if (a.sc_att != 0.0f)
+        pf_attn_split_kernel<HD, true><<<grid, kPbWaves * 64, 0, stream>>>(b, exps, tile0, ntiles);
+      else
+        pf_attn_split_kernel<HD, false><<<grid, kPbWaves * 64, 0, stream>>>(b, exps, tile0, ntiles);
+    };
     switch (hdim) {
-      case 128: pf_attn_bf3_kernel<128><<<grid, kPbWaves * 64, 0, stream>>>(b); break;
-      case 256: pf_attn_bf3_kernel<256><<<grid, kPbWaves * 64, 0, stream>>>(b); break;
+      case 128: go(std::integral_constant<int, 128>{}); break;
+      case 256: go(std::integral_constant<int, 256>{}); break;
       default: return hipErrorInvalidValue;
     }
   } else if (f32) {

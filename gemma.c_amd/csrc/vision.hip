@@ -911,7 +911,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void vis_attn_bf3_kernel(VisAttn 
 // attn_pack_kernel made of K and V with their biases.  Bound by the matrix
 // cores at the clock that the chip holds under them: SigLIP at 896 px (4096
 // patches, 16 heads of 72) takes 30 products per 32 queries and tile, 258
-// TFLOP of f16 in 222 us (1.2 PFLOP/s; v_mfma_f32_32x32x16_f16 on random
+// TFLOP of f16 in 215 us (1.2 PFLOP/s; v_mfma_f32_32x32x16_f16 on random
 // registers alone sustains 1.6), packing 18 us.  The three-bf16-piece kernel
 // before it took 426 us at the same matrix rate with twice the products, and
 // its error against 64-bit sums was larger: 9.6e-7 relative, here 7.0e-7 (fewer
@@ -941,9 +941,8 @@ __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, c
         0.0f, c_hi, c_lo, 0.0f, lds, wave, lane);
   if (qr >= a.n) return;
   float *orow = a.out + (size_t)qr * a.dim + h * HD;
-  w.each(half, [&](int d, v4f x) {
-    *reinterpret_cast<v4f *>(orow + d) = ldexp4(x / w.l, w.e_o);
-  });
+  const float f = 1.0f / w.l;
+  w.each(half, [&](int d, v4f x) { *reinterpret_cast<v4f *>(orow + d) = ldexp4(x * f, w.e_o); });
 }
 
 template <int HD>

@@ -158,3 +158,99 @@ def test_vision_attention_under_capture(gh):
         torch.cuda.synchronize()
         _close(out.cpu().numpy(), want)
         _close(_vision(gh, qkv, bias, heads, dim), want)
+
+
+def _prefill_want(q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense):
+    ctx = pos0 + n
+    pos = pos0 + np.arange(n)
+    j = np.arange(ctx)[None, :]
+    live = np.ones((n, ctx), bool) if dense else j <= pos[:, None]
+    if slide and not dense:
+        live = live & (j > pos[:, None] - slide)
+    out = []
+    for h in range(nh):
+        s = q[:, h * hd:(h + 1) * hd].astype(F64) @ kc[h // (nh // nkv), :ctx].astype(F64).T
+        s = s / np.sqrt(F64(hd))
+        if cap:
+            s = np.tanh(s / cap) * cap
+        out.append(_softmax_av(np.where(live, s, -np.inf), vc[h // (nh // nkv), :ctx].astype(F64)))
+    return np.concatenate(out, axis=1)
+
+
+def _prefill(gh, q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense):
+    import torch
+
+    dq, dk, dv = (torch.from_numpy(a).cuda() for a in (q, kc, vc))
+    out = torch.full((n + 1, nh * hd), float("nan"), device="cuda")
+    gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, pos0, nh, nkv, hd, kc.shape[1], slide,
+                         np.float32(1.0) / np.sqrt(np.float32(hd)), cap, dense, 1,
+                         stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.isnan(got[n]).all()
+    return got[:n]
+
+
+def _prefill_inputs(n, pos0, nh, nkv, hd, seed):
+    rng = np.random.default_rng(seed)
+    q = rng.standard_normal((n, nh * hd + 8)).astype(np.float32)  # a padded row stride
+    kc = rng.standard_normal((nkv, pos0 + n + 5, hd)).astype(np.float32)
+    vc = rng.standard_normal((nkv, pos0 + n + 5, hd)).astype(np.float32)
+    kc[:, pos0 + n:] = np.nan  # never read
+    vc[:, pos0 + n:] = np.nan
+    return q, kc, vc
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,pos0,nh,nkv,hd,slide,cap,dense", [
+    (1, 0, 4, 1, 256, 0, 0.0, False), (33, 0, 4, 1, 256, 0, 0.0, False),
+    (32, 31, 2, 1, 256, 0, 0.0, False), (65, 127, 8, 4, 256, 40, 0.0, False),
+    (129, 0, 4, 2, 128, 33, 0.0, False), (64, 1, 4, 1, 128, 1, 0.0, False),
+    (97, 300, 32, 1, 128, 64, 0.0, False), (40, 500, 4, 1, 256, 100, 30.0, False),
+    (70, 26, 2, 2, 128, 16, 5.0, True), (257, 11, 8, 4, 256, 0, 0.0, True)])
+def test_prefill_tile_edges(gh, monkeypatch, n, pos0, nh, nkv, hd, slide, cap, dense):
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")  # the split kernel at every size
+    q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=n + hd)
+    args = (n, pos0, nh, nkv, hd, slide, cap, dense)
+    _close(_prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [128, 256])
+def test_prefill_tiles_of_any_magnitude(gh, monkeypatch, hd):
+    """Tiles of V at magnitudes far apart, a window that hides the largest
+    from some rows (held to their own largest output), masked keys with
+    infinities in their rows' place in the window."""
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
+    n, pos0, nh, nkv, slide = 150, 200, 4, 2, 90
+    q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=3)
+    ctx = pos0 + n
+    vc[:, :ctx] *= _tile_scales(ctx, (0, 12, -12, 30)).astype(np.float32)
+    q *= np.exp2(np.random.default_rng(4).integers(-20, 20, n))[:, None].astype(np.float32)
+    kc[:, :ctx] *= np.float32(2.0 ** -20)
+    args = (n, pos0, nh, nkv, hd, slide, 0.0, False)
+    got, want = _prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args)
+    for i in range(n):
+        _close(got[i], want[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["gemma-3-4b", "test-hd128"])
+def test_prefill_kernel_choice_agrees(gh, monkeypatch, model):
+    """Either side of the size where the split kernel takes over, the default
+    is one of the two forced kernels' results, and both agree."""
+    import model_bin
+
+    c = model_bin.CONFIGS[model]
+    nh, nkv, hd = c["n_heads"], c["nkv"], c["hdim"]
+    least = 1.1e9 * hd / 256  # flops: 4 hd nh pairs
+    edge = int((least / (2 * hd * nh)) ** 0.5)
+    for n in (edge - 8, edge + 8):
+        q, kc, vc = _prefill_inputs(n, 0, nh, nkv, hd, seed=5)
+        args = (n, 0, nh, nkv, hd, 0, 0.0, False)
+        outs = {}
+        for kind in ("f32", "bf3", ""):
+            monkeypatch.setenv("GEMMA_HIP_PF_ATTN", kind)
+            outs[kind] = _prefill(gh, q, kc, vc, *args)
+        _close(outs["bf3"], outs["f32"])
+        assert np.array_equal(outs[""], outs["bf3" if n > edge else "f32"]), n
