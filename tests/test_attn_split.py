@@ -254,3 +254,39 @@ def test_prefill_kernel_choice_agrees(gh, monkeypatch, model):
             outs[kind] = _prefill(gh, q, kc, vc, *args)
         _close(outs["bf3"], outs["f32"])
         assert np.array_equal(outs[""], outs["bf3" if n > edge else "f32"]), n
+
+
+@pytest.mark.gpu
+def test_attention_workspaces_by_stream(gh):
+    """The kept workspaces: calls of different sizes and both entry points in
+    turn on two streams at once, no call waited for, each with its own inputs;
+    and a captured call of the prompt's entry point, refused."""
+    import torch
+
+    from gemma_hip import GemmaHipError
+
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    hd, nh, nkv, jobs = 128, 4, 2, []
+    for i, n in enumerate((40, 300, 90, 500, 64, 400)):
+        q, kc, vc = _prefill_inputs(n, 0, nh, nkv, hd, seed=20 + i)
+        qkv = np.random.default_rng(i).standard_normal((n, 3 * 72)).astype(np.float32)
+        jobs.append((n, q, kc, vc, qkv, *(torch.from_numpy(a).cuda() for a in (q, kc, vc, qkv)),
+                     torch.zeros((n, nh * hd), device="cuda"), torch.zeros((n, 72), device="cuda")))
+    bias = torch.zeros(3 * 72, device="cuda")
+    torch.cuda.synchronize()
+    asc = np.float32(1.0) / np.sqrt(np.float32(hd))
+    for i, (n, q, kc, vc, qkv, dq, dk, dv, dqkv, out, vout) in enumerate(jobs):
+        s = streams[i % 2].cuda_stream
+        gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, 0, nh, nkv, hd, kc.shape[1], 0, asc,
+                             0.0, False, 1, stream=s)
+        gh.vision_attention(vout, dqkv, bias, n, 1, 72, 1, stream=s)
+    torch.cuda.synchronize()
+    for n, q, kc, vc, qkv, dq, dk, dv, dqkv, out, vout in jobs:
+        _close(out.cpu().numpy(), _prefill_want(q, kc, vc, n, 0, nh, nkv, hd, 0, 0.0, False))
+        _close(vout.cpu().numpy(), _vision_want(qkv, np.zeros(216, np.float32), 1, 72))
+    n, q, kc, dq, dk, dv, out = (jobs[0][i] for i in (0, 1, 2, 5, 6, 7, 9))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        with pytest.raises(GemmaHipError, match="captured"):
+            gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, 0, nh, nkv, hd, kc.shape[1], 0,
+                                 asc, 0.0, False, 1, stream=streams[0].cuda_stream)
