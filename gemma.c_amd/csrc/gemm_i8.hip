@@ -23,7 +23,7 @@
 //    kernel start and buffer stores whose out-of-range cells are dropped.
 //  - gemm_i8_kernel: register-staged loads into a padded LDS double buffer;
 //    used when an operand is too large for 32-bit buffer offsets.
-//  - gemm_i8_generic_kernel: one thread per output, any shape/alignment.
+//  - gemm_i8_kernel with ANY: any k, rows at any address.
 // Tile choice and the measurements behind it are in launch_gemm_i8.
 #include <algorithm>
 #include <cstdio>
@@ -77,11 +77,32 @@ __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n,
   *tn = in_group / gsize;
 }
 
-// Requirement (checked by the launcher): k % 16 == 0 and every row 16-byte
-// aligned; rows/columns beyond m/n and K beyond k load as zeros.
+// Sixteen bytes at any address (global loads need no alignment on this target:
+// the compiler makes one load of the copy), and the last ones of a row, kb ..
+// k - 1, with zeros in the place of those past its end, which are not read.
+__device__ __forceinline__ v4i load16(const int8_t *p) {
+  v4i v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+__device__ __forceinline__ v4i load16_tail(const int8_t *row, int kb, int k) {
+  uint64_t lo = 0, hi = 0;
+#pragma unroll 1
+  for (int e = min(16, k - kb) - 1; e >= 0; --e) {
+    hi = hi << 8 | lo >> 56;
+    lo = lo << 8 | (uint8_t)row[kb + e];
+  }
+  return v4i{(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
+}
+
+// Rows/columns beyond m/n and K beyond k load as zeros.  With ANY, rows at any
+// address and any k (odd widths; the DMA kernels need 16-byte rows): one thread
+// per output, byte by byte, took 9.5 ms at 1064 x 10240 x 7089, here 0.1.
+// Without (checked by the launcher) k % 16 == 0 and every row 16-byte aligned:
+// operands beyond 32-bit offsets.
 // WM x WN: each wave's sub-tile in 32x32 MFMA tiles; waves form a 2x2 grid,
 // so the block tile is (64*WM) x (64*WN).
-template <int WM, int WN, bool HEADS>
+template <int WM, int WN, bool HEADS, bool ANY>
 __global__ __launch_bounds__(kThreads) void gemm_i8_kernel(
     float *__restrict__ dst, int dstr, int hdim, const int8_t *__restrict__ mat,
     int mstr, const float *__restrict__ matsc, const int8_t *__restrict__ src,
@@ -109,6 +130,27 @@ __global__ __launch_bounds__(kThreads) void gemm_i8_kernel(
   v4i ra[WM], rb[WN];
   auto load_tiles = [&](int kt) {
     const int kb = kt * kBK + ld_chunk * 16;
+    if constexpr (ANY) {  // rows past the last are the last one again: not stored
+      const int8_t *arow[WM], *brow[WN];
+#pragma unroll
+      for (int h = 0; h < WM; ++h)
+        arow[h] = src + (size_t)min(m0 + ld_row + 64 * h, m - 1) * sstr;
+#pragma unroll
+      for (int h = 0; h < WN; ++h)
+        brow[h] = mat + (size_t)min(n0 + ld_row + 64 * h, n - 1) * mstr;
+      if ((kt + 1) * kBK <= k) {
+#pragma unroll
+        for (int h = 0; h < WM; ++h) ra[h] = load16(arow[h] + kb);
+#pragma unroll
+        for (int h = 0; h < WN; ++h) rb[h] = load16(brow[h] + kb);
+      } else {
+#pragma unroll
+        for (int h = 0; h < WM; ++h) ra[h] = load16_tail(arow[h], kb, k);
+#pragma unroll
+        for (int h = 0; h < WN; ++h) rb[h] = load16_tail(brow[h], kb, k);
+      }
+      return;
+    }
 #pragma unroll
     for (int h = 0; h < WM; ++h) {
       const int gm = m0 + ld_row + 64 * h;
@@ -885,27 +927,6 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_pp_kernel(
     finish(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
 }
 
-// Any shape, any alignment: one thread per output, byte loads.  Used only
-// when k % 16 != 0 or a row is not 16-byte aligned.
-template <bool HEADS>
-__global__ __launch_bounds__(kThreads) void gemm_i8_generic_kernel(
-    float *__restrict__ dst, int dstr, int hdim, const int8_t *__restrict__ mat,
-    int mstr, const float *__restrict__ matsc, const int8_t *__restrict__ src,
-    int sstr, const float *__restrict__ ssc, int m, int n, int k) {
-  const int col = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int row = blockIdx.y * 4 + (threadIdx.x >> 6);
-  if (row >= m || col >= n) return;
-  const int8_t *a = src + (size_t)row * sstr;
-  const int8_t *b = mat + (size_t)col * mstr;
-  int32_t acc = 0;
-  for (int l = 0; l < k; ++l) acc += (int32_t)a[l] * (int32_t)b[l];
-  const float y = rescale(acc, ssc[row], matsc[col]);
-  if (HEADS)
-    dst[((size_t)(col / hdim) * m + row) * hdim + col % hdim] = y;
-  else
-    dst[(size_t)row * dstr + col] = y;
-}
-
 // Tile shape: GEMMA_HIP_GEMM_TILE=WMxWN (register-staged kernel), WMxWNxS
 // (LDS-DMA kernel, S stages of 64-byte K) or WMxWNxSx128 (128-byte K stages)
 // overrides the choice below (a launch-shape knob like the reference's
@@ -1266,17 +1287,17 @@ void launch_dma(bool heads, hipStream_t stream, float *dst, int dstr, int hdim,
                                   k);
 }
 
-template <int WM, int WN>
+template <int WM, int WN, bool ANY = false>
 void launch_tiled(bool heads, hipStream_t stream, float *dst, int dstr, int hdim,
                   const int8_t *mat, int mstr, const float *matsc,
                   const int8_t *src, int sstr, const float *ssc, int m, int n,
                   int k) {
   const int tiles = ((m + 64 * WM - 1) / (64 * WM)) * ((n + 64 * WN - 1) / (64 * WN));
   if (heads)
-    gemm_i8_kernel<WM, WN, true><<<tiles, kThreads, 0, stream>>>(
+    gemm_i8_kernel<WM, WN, true, ANY><<<tiles, kThreads, 0, stream>>>(
         dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
   else
-    gemm_i8_kernel<WM, WN, false><<<tiles, kThreads, 0, stream>>>(
+    gemm_i8_kernel<WM, WN, false, ANY><<<tiles, kThreads, 0, stream>>>(
         dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
 }
 
@@ -1353,13 +1374,14 @@ hipError_t launch_gemm_i8(float *dst, int dstr, int hdim, const int8_t *mat,
       default: launch_tiled<2, 2>(heads, stream, dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k); break;
     }
   } else {
-    const dim3 grid((n + 63) / 64, (m + 3) / 4);
-    if (heads)
-      gemm_i8_generic_kernel<true><<<grid, kThreads, 0, stream>>>(
-          dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
+    // rows or a K that are not whole 16-byte chunks, tiles as narrow_tile's
+    const int tile = narrow_tile(m, n, dev);
+    if (tile == 2221)
+      launch_tiled<2, 2, true>(heads, stream, dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
+    else if (tile == 214)
+      launch_tiled<2, 1, true>(heads, stream, dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
     else
-      gemm_i8_generic_kernel<false><<<grid, kThreads, 0, stream>>>(
-          dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
+      launch_tiled<1, 1, true>(heads, stream, dst, dstr, hdim, mat, mstr, matsc, src, sstr, ssc, m, n, k);
   }
   return hipGetLastError();
 }

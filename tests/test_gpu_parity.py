@@ -280,6 +280,42 @@ def test_gemm_vs_oracle(gh, oracle, label, m, n, k):
     assert_same(host(dst), oracle.gemm_int8_full(B, bs, qo, so))
 
 
+@pytest.mark.parametrize("m,n,k,off", [
+    (2, 3, 1, 0), (5, 70, 15, 1), (65, 64, 17, 3), (64, 129, 63, 0), (130, 65, 65, 7),
+    (33, 200, 127, 1), (129, 300, 1001, 5), (200, 1000, 48, 1), (2100, 2050, 33, 1),
+    (4100, 4097, 50, 2)])
+def test_gemm_any_rows(gh, oracle, m, n, k, off):
+    """K that is not whole 16-byte chunks and rows at any address: every tile
+    shape of the register-staged kernel, the last chunk of a row that ends its
+    buffer, row-major (strided) and head-major outputs."""
+    rng = np.random.default_rng(m + n + k)
+    A = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    B = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    sa = rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    sb = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
+    want = oracle.gemm_int8_full(B, sb, A, sa)
+
+    def at(x, stride):  # rows `stride` apart from an address `off` past an aligned one
+        flat = np.full(off + (x.shape[0] - 1) * stride + k, 77, np.int8)
+        for i, r in enumerate(x):
+            flat[off + i * stride:off + i * stride + k] = r
+        t = dev(flat)
+        return t, t.data_ptr() + off
+
+    (ta, pa), (tb, pb) = at(A, k + 3), at(B, k)
+    dst = torch.full((m, n + 5), 7.0, dtype=torch.float32, device="cuda")
+    gh.matmul(dst, n + 5, pb, k, dev(sb), pa, k + 3, dev(sa), m, n, k, stream())
+    got = host(dst)
+    assert_same(np.ascontiguousarray(got[:, :n]), want)
+    assert np.all(got[:, n:] == 7.0)
+    if n % 4 == 0:
+        t2, p2 = at(A, k)
+        out = torch.empty((4, m, n // 4), dtype=torch.float32, device="cuda")
+        gh.matmul_heads(out, pb, dev(sb), p2, dev(sa), m, 4, n // 4, k, stream())
+        heads = host(out).transpose(1, 0, 2).reshape(m, n)
+        assert_same(np.ascontiguousarray(heads), want)
+
+
 # The prefill's fused launches over adjacent weight matrices (gemma_hip_matmul_cols):
 # gemma-3-4b q/k/v and gate/up at 2048 tokens, gemma-3-1b at 512, SigLIP
 # q/k/v, and a ragged split whose inner boundaries suit no tile width.
