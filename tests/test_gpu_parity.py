@@ -222,6 +222,28 @@ def test_gemv_unaligned_rows(gh, oracle):
     assert np.array_equal(bits(host(y)), bits(oracle.gemv_int8(W, ws, qo, so)[0]))
 
 
+@pytest.mark.parametrize("k,off", [(1, 0), (15, 1), (16, 3), (17, 0), (129, 5), (4099, 1)])
+def test_gemv_any_rows(gh, oracle, k, off):
+    """Whole 16-byte pieces and the last bytes of rows at any address, the last
+    row ending its buffer, two jobs."""
+    rng = np.random.default_rng(k)
+    x = outlier_acts(rng, (k,))
+    qo, so = oracle.quantize_act(x)
+    specs, outs, want, keep = [], [], [], []
+    for n in (3, 70):
+        W = rng.integers(-127, 128, (n, k), dtype=np.int8)
+        ws = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
+        buf = dev(np.concatenate([np.full(off, 77, np.int8), W.reshape(-1)]))
+        y = torch.full((n + 1,), 7.0, dtype=torch.float32, device="cuda")
+        keep.append((buf, dev(ws)))
+        specs.append((buf.data_ptr() + off, keep[-1][1], y, n))
+        outs.append(y)
+        want.append(oracle.gemv_int8(W, ws, qo, so)[0])
+    gh.quantize_matmul(specs, dev(x), k, None, None, stream())
+    for y, w in zip(outs, want):
+        assert np.array_equal(bits(host(y)[:-1]), bits(w)) and host(y)[-1] == 7.0
+
+
 # --------------------------------------------------------------- GEMM
 @pytest.mark.parametrize("tag", ["tails", "strided", "m1", "blocks"])
 def test_gemm_golden(gh, golden, tag):
