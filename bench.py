@@ -28,9 +28,9 @@ The JSON line also carries, measured in the same run:
   per_gemv_f32  the fp32 fallback ('U' files, gemv_fpx): the sweep's launches
                 with fp32 weights, GB/s per launch
   gemm_f32      the fp32 GEMM (gemm_fpx) at the gemma-3-4b prefill shapes,
-                TFLOP/s of fp32 work; by default split-bf16 on the bf16
-                matrix cores (six bf16 products per multiply-add: bound
-                2500 / 6 = 416.7 TF/s), with GEMMA_HIP_GEMM_F32=mfma the
+                TFLOP/s of fp32 work; by default in split precision on
+                the f16 matrix cores (three f16 products per multiply-add:
+                bound 2500 / 3 = 833.3 TF/s), with GEMMA_HIP_GEMM_F32=mfma the
                 fp32-MFMA kernel (bound 157.3 TF/s)
   decode_1b     tokens/s of the full W8A8 matmul path of one gemma-3-1b
                 decode token (26 layers x {qkv, o, gate/up, down} + LM head)
@@ -326,12 +326,12 @@ def bench_gemm(torch, gh, gen, timer, reps):
 def bench_gemm_f32(torch, gh, gen, timer, reps):
     """The fp32 GEMM (gemm_fpx, gemma.c:3304-3399; 'U' model files) at the
     gemma-3-4b prefill shapes, TFLOP/s of fp32 work against the bound of the
-    kernel that runs: the split-bf16 one (the library's default) spends six
-    bf16 MFMA products per fp32 multiply-add, so its bound is a sixth of the
-    bf16 peak; the fp32-MFMA one (GEMMA_HIP_GEMM_F32=mfma) is bound by the
+    kernel that runs: the split one (the library's default) spends three
+    f16 MFMA products per fp32 multiply-add, so its bound is a third of the
+    f16 peak, which is the bf16 one; the fp32-MFMA one (GEMMA_HIP_GEMM_F32=mfma) is bound by the
     fp32 matrix peak."""
     split = os.environ.get("GEMMA_HIP_GEMM_F32") != "mfma"
-    peak = BF16_PEAK_TFLOPS / 6 if split else FP32_PEAK_TFLOPS
+    peak = BF16_PEAK_TFLOPS / 3 if split else FP32_PEAK_TFLOPS
     out = {}
     stream = torch.cuda.current_stream().cuda_stream
     for name, m, n, k in GEMM_SHAPES[:5]:
@@ -478,9 +478,9 @@ def bench_decoder(torch, gh, name: str, prompt: int, steps: int) -> dict:
     if quant:
         prefill.update(int8_tops=round(pf_ops / t_pf / 1e12, 1),
                        int8_frac=round(pf_ops / t_pf / 1e12 / INT8_PEAK_TOPS, 4))
-    else:  # the fp32 GEMMs (split-bf16 by default: bound a sixth of the bf16 peak)
+    else:  # the fp32 GEMMs (split precision by default: bound a third of the f16 peak)
         split = os.environ.get("GEMMA_HIP_GEMM_F32") != "mfma"
-        peak = BF16_PEAK_TFLOPS / 6 if split else FP32_PEAK_TFLOPS
+        peak = BF16_PEAK_TFLOPS / 3 if split else FP32_PEAK_TFLOPS
         prefill.update(fp32_tflops=round(pf_ops / t_pf / 1e12, 1),
                        fp32_frac=round(pf_ops / t_pf / 1e12 / peak, 4))
     gb = gemv_bytes if quant else gemv_f32_bytes

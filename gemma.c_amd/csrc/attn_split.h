@@ -38,9 +38,6 @@
 namespace gh {
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-
 // Fragments of a 32-key tile.  A wave computes S^T = K Q^T (rows: 32 keys,
 // columns: 32 queries) and O^T = V^T P^T (rows: 32 dims).  Operand layout of
 // the 32x32x16 MFMA: lane l holds row (or column) l % 32 and the eight k
@@ -67,10 +64,6 @@ struct AttnTile {
   static_assert(HD % 16 == 0 || kTail, "head dim");
 };
 
-__device__ __forceinline__ h2 cvt_pk_f16(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  return __builtin_convertvector(f2{a, b}, h2);
-}
 // The pieces of eight values.
 __device__ __forceinline__ void split8(const float (&x)[8], h8 *hi, h8 *lo) {
 #pragma unroll
@@ -82,12 +75,6 @@ __device__ __forceinline__ void split8(const float (&x)[8], h8 *hi, h8 *lo) {
     (*lo)[e] = b[0];
     (*lo)[e + 1] = b[1];
   }
-}
-// Magnitude for a scale: infinities and NaN don't set it (they stay what
-// they are in their own products and leave the others' precision alone).
-__device__ __forceinline__ float finite_abs(float x) {
-  const float a = fabsf(x);
-  return a <= FLT_MAX ? a : 0.0f;
 }
 // E such that amax 2^-E lies in [2^14, 2^15), f16's upper range; 0 for 0.
 __device__ __forceinline__ int scale_exp(float amax) {

@@ -1,15 +1,17 @@
-// gemm_f32.hip -- fp32 fallback GEMM for unquantized model files
-// (gemma.c:3304-3399 gemm_fpx), on fp32 MFMA (v_mfma_f32_32x32x2_f32).
+// gemm_f32.hip -- fp32 GEMM for unquantized model files (gemma.c:3304-3399
+// gemm_fpx): in split precision on the f16 matrix cores (gemm_h2_kernel), or
+// on fp32 MFMA (v_mfma_f32_32x32x2_f32, gemm_f32_kernel).
 //
 //   dst[i][j] = sum_l src[i][l]*mat[j][l]
 //
-// 256 threads, 2x2 waves, 128x128 or 64x64 block tiles, a K step of 16
+// The fp32-MFMA kernel: 256 threads, 2x2 waves, 128x128 or 64x64 block tiles, a K step of 16
 // floats (64 bytes per row) double-buffered in LDS.  A lane
 // owns 8 consecutive k of each step (lane / 32 picks the half) for A and B
 // alike, so each of the 8 MFMA sub-steps pairs matching k.  The reference's
 // fp32 sum has no fixed order (vectorised, KC-chunked, gemma.c:3287-3299), so
 // parity for this path is a tolerance on |y - y_exact| / sum|a*b|.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 
@@ -122,24 +124,32 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(
   }
 }
 
-// The same GEMM on the bf16 matrix cores in split precision: every fp32
-// operand x is split into three bf16 pieces x = x0 + x1 + x2 (split3x2: each
-// rounded to nearest from the remainder, together x's 24 significant bits)
-// and each product summed from the six piece products whose orders add up
-// to at most 2 (a2 b0, a1 b1, a0 b2, a1 b0, a0 b1, a0 b0, the small ones
-// first), on v_mfma_f32_32x32x16_bf16 with fp32 accumulation: the dropped
-// terms are below 3 * 2^-24 |a b| and bf16 x bf16 products are exact, so
-// each product carries an fp32 rounding's error, and the sums are fp32 as in
-// the fp32-MFMA kernel.  The six bf16 MFMAs cost ~0.4 of that kernel's fp32
-// MFMA work.  Geometry as gemm_f32_kernel (2x2 waves of WM x WN 32x32 tiles,
-// the same output layout: lane l, element r -> row 8 (r/4) + 4 (l/32) + r%4,
-// column l%32; A and B fragments give lane l row l%32 and k 8 (l/32) .. + 7).
-// Per 32-float K step the workgroup splits its A and B rows once into three
-// bf16 planes each in LDS, while the next step's fp32 rows load into
-// registers; one buffer (60 KB at 128x128: two workgroups per CU), two
-// barriers per step.  Measured on the 4b prefill shapes and dropped: two
-// buffers with one barrier per step (16- or 32-float steps) ran 3-10%
-// slower at the same tiles.
+// The same GEMM on the f16 matrix cores in split precision (gh_arith.h): two
+// scaled f16 pieces per operand, three products (v_mfma_f32_16x16x32_f16) with
+// fp32 accumulation.  Three bf16 pieces with six products took twice the matrix
+// work at about the same rate and rounded each sum twice as often.  Both in us
+// and against the 64-bit sums (rms): 512x13824x1152 119 -> 71, 5.2e-7 ->
+// 3.8e-7; 2048x20480x2560 1167 -> 695, 7.9e-7 -> 5.6e-7; 4096x4304x1152 284 ->
+// 155.  That is 0.9 PFLOP/s of f16 products.  Bound by the vector work of the
+// split (61 us of the 71 are left without it), the LDS traffic and the matrix
+// cores together, none of them alone.
+//
+// Scales.  Each row of A and of B has its own power of two, set from its first
+// K step so that the step's largest value lies in [2^10, 2^11): four octaves
+// below what flags it, and with both pieces whole down to 2^-13 of it.  A later
+// step with a scaled value of 2^15 or more flags it; the workgroup then moves
+// those rows' scales, splits the step again and rescales its sums (exactly).
+// Rows of zeros start at the least scale.  A value's error is at most 2^-22 of
+// it or 2^-35 of its row's largest before it, whichever is more.
+//
+// 256 threads, 2x2 waves of 2 WM x 2 WN 16x16 tiles.  Per 32-float K step the
+// workgroup splits its A and B rows into two f16 planes each in LDS, doubly
+// buffered: a wave's products of one step run between the vector instructions
+// that split the next (one barrier a step; 77 -> 72 us against splitting, a
+// barrier, and the products), and each row's registers are loaded again with
+// the step after as soon as they are split.  The product is taken transposed
+// (D = B A^T: lane l, element r holds row l % 16 of A and columns
+// 4 (l / 16) + r), so a lane's four outputs are neighbours in memory.
 //
 // B comes as segments (F32Segs: q, k, v or gate, up side by side in the
 // output); each thread resolves the rows it loads to their segment once.
@@ -155,23 +165,36 @@ struct F32Split {
   int *cnt;  // [tiles], zero between launches
 };
 
+constexpr int kScaleSet = 10, kScaleTop = 15;   // octaves of a row's scaled values
+constexpr int kScaleMin = -126, kScaleMax = 117;  // whose scales are normal floats
+
+// The largest of eight consecutive lanes' values.
+__device__ __forceinline__ float max_of_8(float v) {
+  v = fmaxf(v, dpp_f32<kDppXor1>(v));
+  v = fmaxf(v, dpp_f32<kDppXor2>(v));
+  return fmaxf(v, dpp_f32<kDppHalfMirror>(v));
+}
+
 template <int WM, int WN, bool SK>
-__global__ __launch_bounds__(kThreads, 2) void gemm_bf3_kernel(
+__global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) void gemm_h2_kernel(
     float *__restrict__ dst, int dstr, F32Segs b, int mstr, const float *__restrict__ src,
     int sstr, int m, int k, F32Epilogue ep, F32Split sk) {
   constexpr int kBM = 64 * WM, kBN = 64 * WN;
-  constexpr int BK = 32;              // floats of K per step
-  constexpr int RW = BK + 8;          // plane row (bf16): 8 consecutive rows in distinct banks
-  constexpr int CPR = BK / 4;         // float4 chunks per row and step
-  constexpr int RPP = kThreads / CPR; // rows per load pass
-  constexpr int HA = kBM / RPP, HB = kBN / RPP;
-  static_assert(kBM % RPP == 0 && kBN % RPP == 0, "tile");
-  __shared__ __attribute__((aligned(16))) uint16_t pa[3][kBM * RW];
-  __shared__ __attribute__((aligned(16))) uint16_t pb[3][kBN * RW];
+  constexpr int MI = 2 * WM, NJ = 2 * WN;  // 16x16 tiles of a wave
+  constexpr int BK = 32;                   // floats of K per step
+  constexpr int CPR = BK / 4;              // float4 chunks per row and step
+  constexpr int RPP = kThreads / CPR;      // rows per load pass
+  constexpr int HA = kBM / RPP, HB = kBN / RPP, H = HA + HB;
+  static_assert(kBM % RPP == 0 && kBN % RPP == 0 && CPR == 8, "tile");
+  // two steps' planes of A's rows then B's; a row's 16-byte chunk c stands at
+  // c ^ (row / 4) % 4, which spreads 16 rows' equal chunks over all banks
+  __shared__ __attribute__((aligned(16))) _Float16 plane[2][2][(kBM + kBN) * BK];
+  __shared__ int exps[kBM + kBN], moved[kBM + kBN];
+  __shared__ int flag[2];  // the step that left its range, by its parity
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1;
   const int wn = wave & 1;
   const int n = b.end[b.nseg - 1];
@@ -179,88 +202,75 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_bf3_kernel(
   const int n0 = blockIdx.x * kBN;
   const int ld_row = tid / CPR, ld_c = tid % CPR;  // chunk ld_c of rows ld_row + RPP h
 
-  // the B rows this thread loads (null past the last column)
-  const float *brow[HB];
+  // the rows this thread loads, A's then B's (past the last: the last again,
+  // whose outputs are not stored)
+  const float *row[H];
+#pragma unroll
+  for (int h = 0; h < HA; ++h)
+    row[h] = src + (size_t)min(m0 + ld_row + RPP * h, m - 1) * sstr;
 #pragma unroll
   for (int h = 0; h < HB; ++h) {
-    const int gn = n0 + ld_row + RPP * h;
+    const int gn = min(n0 + ld_row + RPP * h, n - 1);
     const int t = (b.nseg > 1 && gn >= b.end[0]) + (b.nseg > 2 && gn >= b.end[1]);
     const int first = t == 0 ? 0 : t == 1 ? b.end[0] : b.end[1];
     const float *w = t == 0 ? b.w[0] : t == 1 ? b.w[1] : b.w[2];
-    brow[h] = gn < n ? w + (size_t)(gn - first) * mstr : nullptr;
+    row[HA + h] = w + (size_t)(gn - first) * mstr;
   }
 
-  v4f ra[HA], rb[HB];
-  auto load = [&](int kt) {
-    const int kb = kt * BK + 4 * ld_c;
+  v4f x[H];
+  auto load = [&](int kt) {  // past the end of the rows: their last floats again
+    const int kb = min(kt * BK + 4 * ld_c, k - 4);
 #pragma unroll
-    for (int h = 0; h < HA; ++h) {
-      const int gm = m0 + ld_row + RPP * h;
-      ra[h] = (gm < m && kb < k)
-                  ? *reinterpret_cast<const v4f *>(src + (size_t)gm * sstr + kb)
-                  : v4f{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < H; ++h) {
+      x[h] = *reinterpret_cast<const v4f *>(row[h] + kb);
+      __builtin_amdgcn_sched_barrier(0);  // in order: the steps wait for them one by one
     }
-#pragma unroll
-    for (int h = 0; h < HB; ++h)
-      rb[h] = (brow[h] != nullptr && kb < k) ? *reinterpret_cast<const v4f *>(brow[h] + kb)
-                                             : v4f{0.f, 0.f, 0.f, 0.f};
   };
-  auto split_store = [&]() {
+  float f[H];  // 2^-E of those rows; 0 for what load() repeated
+  auto step_max = [&](int h) {
+    return max_of_8(fmaxf(fmaxf(finite_abs(x[h][0]), finite_abs(x[h][1])),
+                          fmaxf(finite_abs(x[h][2]), finite_abs(x[h][3]))));
+  };
+  auto set = [&](int h, float top) {
+    const int e = min(max((__float_as_int(top) >> 23) - 127 - kScaleSet, kScaleMin), kScaleMax);
+    f[h] = __int_as_float((127 - e) << 23);
+    if (ld_c == 0) exps[ld_row + RPP * h] = e;
+  };
+  // splits row h of the step into the planes at `buf`; the largest magnitude
+  const int st_at = ld_row * BK + ((ld_c / 2) ^ (ld_row / 4 % 4)) * 8 + ld_c % 2 * 4;
+  static_assert(RPP % 16 == 0, "rows RPP apart swizzle alike");
+  auto split_store = [&](int buf, int h) {
+    const v4f y = x[h] * f[h];
+    const h2 a = cvt_pk_f16(y[0], y[1]), c = cvt_pk_f16(y[2], y[3]);
+    auto rest = [&](int e, _Float16 p) { return __builtin_fmaf(x[h][e], f[h], -(float)p); };
+    const h2 a1 = cvt_pk_f16(rest(0, a[0]), rest(1, a[1]));
+    const h2 c1 = cvt_pk_f16(rest(2, c[0]), rest(3, c[1]));
+    const int at = st_at + RPP * h * BK;
+    *reinterpret_cast<u2 *>(&plane[buf][0][at]) =
+        u2{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, c)};
+    *reinterpret_cast<u2 *>(&plane[buf][1][at]) =
+        u2{__builtin_bit_cast(uint32_t, a1), __builtin_bit_cast(uint32_t, c1)};
+    return fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
+  };
+  // the rows' last step: nothing past their end
+  auto trim = [&](int kt) {
+    if ((kt + 1) * BK > k && kt * BK + 4 * ld_c >= k) {
 #pragma unroll
-    for (int h = 0; h < HA; ++h) {
-      const Bf3x2 lo = split3x2(ra[h][0], ra[h][1]), hi = split3x2(ra[h][2], ra[h][3]);
-      const int at = (ld_row + RPP * h) * RW + 4 * ld_c;
-      *reinterpret_cast<u2 *>(&pa[0][at]) = u2{lo.q0, hi.q0};
-      *reinterpret_cast<u2 *>(&pa[1][at]) = u2{lo.q1, hi.q1};
-      *reinterpret_cast<u2 *>(&pa[2][at]) = u2{lo.q2, hi.q2};
-    }
-#pragma unroll
-    for (int h = 0; h < HB; ++h) {
-      const Bf3x2 lo = split3x2(rb[h][0], rb[h][1]), hi = split3x2(rb[h][2], rb[h][3]);
-      const int at = (ld_row + RPP * h) * RW + 4 * ld_c;
-      *reinterpret_cast<u2 *>(&pb[0][at]) = u2{lo.q0, hi.q0};
-      *reinterpret_cast<u2 *>(&pb[1][at]) = u2{lo.q1, hi.q1};
-      *reinterpret_cast<u2 *>(&pb[2][at]) = u2{lo.q2, hi.q2};
+      for (int h = 0; h < H; ++h) f[h] = 0.0f;
     }
   };
 
-  v16f acc[WM][WN];
+  v4f acc[MI][NJ];
 #pragma unroll
-  for (int i = 0; i < WM; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < WN; ++j) acc[i][j] = v16f{};
-
-  const int fr = lane & 31, half = lane >> 5;
-  auto mfmas = [&]() {
-#pragma unroll
-    for (int s = 0; s < BK / 16; ++s) {
-      bf8 a[WM][3], bb[WN][3];
-#pragma unroll
-      for (int i = 0; i < WM; ++i) {
-        const int at = (wm * 32 * WM + i * 32 + fr) * RW + 16 * s + 8 * half;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) a[i][p] = *reinterpret_cast<const bf8 *>(&pa[p][at]);
-      }
-#pragma unroll
-      for (int j = 0; j < WN; ++j) {
-        const int at = (wn * 32 * WN + j * 32 + fr) * RW + 16 * s + 8 * half;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) bb[j][p] = *reinterpret_cast<const bf8 *>(&pb[p][at]);
-      }
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) {
-          v16f c = acc[i][j];
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][2], bb[j][0], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][1], bb[j][1], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], bb[j][2], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][1], bb[j][0], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], bb[j][1], c, 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][0], bb[j][0], c, 0, 0, 0);
-        }
-    }
-  };
+    for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  const int fr = lane & 15, grp = lane >> 4;
+  const int arow = wm * 16 * MI, bcol = wn * 16 * NJ;  // the wave's first row and column
+  const int rd_at = fr * BK + (grp ^ (fr / 4)) * 8;
+  // acc[i][j][r] is output row m0 + out_row(i), column n0 + out_col(j, r)
+  auto out_row = [&](int i) { return arow + 16 * i + fr; };
+  auto out_col = [&](int j, int r) { return bcol + 16 * j + 4 * grp + r; };
 
   const int nk = (k + BK - 1) / BK;
   int kt0 = 0, kt1 = nk;
@@ -268,30 +278,98 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_bf3_kernel(
     kt0 = (int)((long)blockIdx.z * nk / sk.splits);
     kt1 = (int)((long)(blockIdx.z + 1) * nk / sk.splits);
   }
+  if (tid < 2) flag[tid] = -1;
   load(kt0);
+#pragma unroll
+  for (int h = 0; h < H; ++h) set(h, step_max(h));
+  trim(kt0);
+#pragma unroll
+  for (int h = 0; h < H; ++h) split_store(kt0 & 1, h);
+  load(min(kt0 + 1, kt1 - 1));
   for (int kt = kt0; kt < kt1; ++kt) {
-    split_store();
-    lds_barrier();  // the step's planes are complete
-    if (kt + 1 < kt1) load(kt + 1);  // the next step's rows load during the MFMAs
-    mfmas();
-    lds_barrier();  // every wave is done with the planes
+    const int buf = kt & 1;
+    lds_barrier();  // the step's planes and flag are complete, the other planes are free
+    if (__builtin_amdgcn_readfirstlane(flag[buf]) == kt) {
+      // rows that left their range: new scales, the step split again, the sums
+      // of those rows and columns rescaled
+      load(kt);
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        const float top = step_max(h);
+        const int old = exps[ld_row + RPP * h];
+        if (top * f[h] >= (float)(1 << kScaleTop)) set(h, top);
+        if (ld_c == 0) moved[ld_row + RPP * h] = old - exps[ld_row + RPP * h];
+        split_store(buf, h);
+      }
+      load(min(kt + 1, kt1 - 1));
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[i][j][r] = ldexpf(acc[i][j][r], moved[out_row(i)] + moved[kBM + out_col(j, r)]);
+    }
+    h8 a[2][MI], w[2][NJ];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        a[1 - p][i] =
+            *reinterpret_cast<const h8 *>(&plane[buf][1 - p][(arow + 16 * i) * BK + rd_at]);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        w[p][j] =
+            *reinterpret_cast<const h8 *>(&plane[buf][p][(kBM + bcol + 16 * j) * BK + rd_at]);
+    }
+    // the products, with the next step's split between them and the loads of
+    // the one after
+    trim(kt + 1);
+    const int kb = min(min(kt + 2, kt1 - 1) * BK + 4 * ld_c, k - 4);
+    float top = 0.0f;
+    constexpr int kPer = 3 * MI * NJ / H;  // products per row of the split
+    static_assert(kPer * H == 3 * MI * NJ, "products");
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      top = fmaxf(top, split_store(1 - buf, h));
+      x[h] = *reinterpret_cast<const v4f *>(row[h] + kb);
+#pragma unroll
+      for (int u = h * kPer; u < (h + 1) * kPer; ++u) {
+        const int q = u / (MI * NJ), j = u / MI % NJ, i = u % MI;  // a1 b0, a0 b1, a0 b0
+        acc[i][j] =
+            __builtin_amdgcn_mfma_f32_16x16x32_f16(w[q == 1][j], a[q == 0][i], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                     // a product,
+        __builtin_amdgcn_sched_group_barrier(0x2, (20 + kPer - 1) / kPer, 0);  // then vector work
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (__any(!(top < (float)(1 << kScaleTop))) && lane == 0) flag[1 - buf] = kt + 1;
   }
+  // to the operands' units
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        acc[i][j][r] = ldexpf(acc[i][j][r], exps[out_row(i)] + exps[kBM + out_col(j, r)]);
 
   if constexpr (SK) {
     // Partials go out and come back in with device-coherent (agent-scope)
     // accesses, which write through and read past this XCD's L2.
-    constexpr int kTileInts = kThreads * WM * WN * 16;
+    constexpr int kTileInts = kThreads * MI * NJ * 4;
     const int tile = blockIdx.y * gridDim.x + blockIdx.x;
     const int z = blockIdx.z;
     int *part = sk.ws + (size_t)tile * sk.splits * kTileInts;
     int *mine = part + (size_t)z * kTileInts;
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          __hip_atomic_store(mine + ((i * WN + j) * 16 + r) * kThreads + tid,
+        for (int r = 0; r < 4; ++r)
+          __hip_atomic_store(mine + ((i * NJ + j) * 4 + r) * kThreads + tid,
                              __float_as_int(acc[i][j][r]), __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
     __shared__ int last;
@@ -300,43 +378,70 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_bf3_kernel(
     if (tid == 0) last = atomicAdd(sk.cnt + tile, 1) == sk.splits - 1;
     __syncthreads();
     if (!last) return;
+    // a split at a time, its loads in flight together (one value's splits in
+    // turn waited for each load: 4 us per split)
+    v4f sum[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < WN; ++j)
+      for (int j = 0; j < NJ; ++j) sum[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int o = 0; o < sk.splits; ++o) {
+      const int *theirs = part + (size_t)o * kTileInts + tid;
+      v4f y[MI][NJ];
+      if (o != z) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int at = ((i * WN + j) * 16 + r) * kThreads + tid;
-          float t = 0.f;
-          for (int o = 0; o < sk.splits; ++o)
-            t += o == z ? acc[i][j][r]
-                        : __int_as_float(__hip_atomic_load(part + (size_t)o * kTileInts + at,
-                                                           __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_AGENT));
-          acc[i][j][r] = t;
-        }
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              y[i][j][r] = __int_as_float(__hip_atomic_load(
+                  theirs + ((i * NJ + j) * 4 + r) * kThreads, __ATOMIC_RELAXED,
+                  __HIP_MEMORY_SCOPE_AGENT));
+      } else {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) y[i][j] = acc[i][j];
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) sum[i][j] += y[i][j];
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = sum[i][j];
     if (tid == 0) sk.cnt[tile] = 0;
   }
 
 #pragma unroll
-  for (int j = 0; j < WN; ++j) {
-    const int col = n0 + wn * 32 * WN + j * 32 + (lane & 31);
-    if (col >= n) continue;
+  for (int i = 0; i < MI; ++i) {
+    const int r0 = m0 + out_row(i);
+    if (r0 >= m) continue;
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int j = 0; j < NJ; ++j) {
+      const int c0 = n0 + out_col(j, 0);
+      float *out = dst + (size_t)r0 * dstr + c0;
+      if (c0 + 4 <= n) {
+        v4f y;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row =
-            m0 + wm * 32 * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < m) dst[(size_t)row * dstr + col] = ep.apply(acc[i][j][r], row, col, dstr);
+        for (int r = 0; r < 4; ++r) y[r] = ep.apply(acc[i][j][r], r0, c0 + r, dstr);
+        __builtin_memcpy(out, &y, 16);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c0 + r < n) out[r] = ep.apply(acc[i][j][r], r0, c0 + r, dstr);
       }
+    }
   }
 }
 
 // One launch of the split kernel: tiles of (64 WM) x (64 WN), `splits`
 // workgroups per tile along z (1: no split-K).
 template <int WM, int WN>
-hipError_t launch_bf3(float *dst, int dstr, const F32Segs &b, int mstr, const float *src,
+hipError_t launch_h2(float *dst, int dstr, const F32Segs &b, int mstr, const float *src,
                       int sstr, int m, int k, const F32Epilogue &ep, int splits,
                       hipStream_t stream) {
   const int n = b.end[b.nseg - 1];
@@ -347,10 +452,10 @@ hipError_t launch_bf3(float *dst, int dstr, const F32Segs &b, int mstr, const fl
     const hipError_t e = split_workspace(
         stream, (size_t)tiles * splits * kThreads * WM * WN * 16, tiles, &sk.ws, &sk.cnt);
     if (e != hipSuccess) return e;
-    gemm_bf3_kernel<WM, WN, true><<<grid, kThreads, 0, stream>>>(dst, dstr, b, mstr, src, sstr,
+    gemm_h2_kernel<WM, WN, true><<<grid, kThreads, 0, stream>>>(dst, dstr, b, mstr, src, sstr,
                                                                 m, k, ep, sk);
   } else {
-    gemm_bf3_kernel<WM, WN, false><<<grid, kThreads, 0, stream>>>(dst, dstr, b, mstr, src, sstr,
+    gemm_h2_kernel<WM, WN, false><<<grid, kThreads, 0, stream>>>(dst, dstr, b, mstr, src, sstr,
                                                                  m, k, ep, sk);
   }
   return hipGetLastError();
@@ -418,7 +523,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f64_kernel(
   }
 }
 
-// The fp32 GEMM's kernel: the split-bf16 one by default, the fp32-MFMA one
+// The fp32 GEMM's kernel: the split one by default, the fp32-MFMA one
 // with GEMMA_HIP_GEMM_F32=mfma (read at every launch, so that one process
 // can time or check both).
 bool gemm_f32_split() {
@@ -454,68 +559,81 @@ long tile_count(int m, int n, Tile t) {
   return (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
 }
 
-// Tile and split-K ways of the split kernel (two 128x128, three 128x64 or
-// four 64x64 workgroups per CU), from a sweep of the gemma-3 prefill and
-// SigLIP shapes (M = 512, 2048, 4096; T = the count of 128x128 tiles):
-//   T >= 1.5 per CU:           128x128, no split
-//   T >= 1 per CU:             128x128 in 3 splits when K >= 3072 floats
-//                              (4b down 743 -> 604 us, SigLIP fc2 315 -> 285);
-//                              else 128x128 in 2 when those fill two per CU
-//                              to within 10% (4b q 166 -> 140), else 128x64
-//                              in 2 (4b o 147)
-//   128x64 tiles >= 1 per CU:  128x64 in 2 (4b k/v 89 -> 83)
-//   fewer:                     64x64, splits for ~1.5 workgroups per CU
-//                              (1b down at M=512: 3 splits, 86 us; 6: 92)
-// Each split keeps at least 8 K steps (256 floats); at most 16 splits.
-// GEMMA_HIP_GEMM_F32_TILE forces the tile (the split then follows the last
-// rule for that tile's count), GEMMA_HIP_GEMM_F32_SPLIT=s the splits
-// (clamped to 1..min(16, K steps)); both are read at every launch.
-struct Bf3Plan {
+// Tile and split-K ways of the split kernel: the least of a time modelled from
+// a sweep of the gemma-3 prompt and SigLIP shapes (each tile in 1, 2, 3, 4, 6
+// and 8 splits; the model's choice is within 8% of the sweep's best).  A tile
+// takes `lat` us a K step while its workgroups are alone on their CUs and
+// `thr` us of a CU's time when `slots` share one; `ends` steps' time goes to its
+// first loads and its stores.  Splitting K costs the partials' way through
+// memory and the last workgroup's sum over them.  As measured, us, without and
+// with splits: 512x2560x10240 (80 128x128 tiles) 160 -> 102 in 6, 2048x2048x2560
+// (256) 83 -> 80 in 2, 64x1024x2048 (16 64x64 tiles) 34 -> 13 in 8, but
+// 4096x4304x1152 (1088) 155 -> 165 in 2.  Each split keeps at least 6 K steps
+// (192 floats); at most 16 splits, and partials of at most 5 128x128 tiles per
+// CU (80 MiB).  Products of under 1.5 128x128 tiles per CU with 512 floats or
+// more of K take two splits at least, whose sums are half as long: 4096x1152x588
+// 38 -> 40 us, 2.8e-7 -> 2.0e-7 off the 64-bit sums (rms); 4096x1152x1152 62 ->
+// 58, 3.8e-7 -> 2.7e-7.
+// GEMMA_HIP_GEMM_F32_TILE forces the tile, GEMMA_HIP_GEMM_F32_SPLIT=s the
+// splits (clamped to 1..min(16, K steps)); both are read at every launch.
+struct H2Plan {
   Tile tile;
   int splits;
 };
-Bf3Plan bf3_plan(int m, int n, int k, const DeviceInfo &dev) {
+H2Plan h2_plan(int m, int n, int k, bool may_split, const DeviceInfo &dev) {
+  struct Cost {
+    Tile tile;
+    int bm, bn, slots;
+    double lat, thr, ends;
+  };
+  static constexpr Cost kCosts[] = {{kTile64, 64, 64, 4, 0.50, 0.33, 2},
+                                    {kTile128x64, 128, 64, 3, 0.72, 0.56, 3},
+                                    {kTile128, 128, 128, 2, 1.0, 0.87, 4}};
+  constexpr double kSplitUs = 1.0, kPerSplitUs = 0.6, kPartialBytesPerUs = 9e6;
   const int nk = (k + 31) / 32;
-  Bf3Plan p{kTile64, 1};
-  const long t128 = tile_count(m, n, kTile128);
-  if (forced_tile(&p.tile)) {
-    const long t = tile_count(m, n, p.tile);
-    p.splits = t >= dev.cus ? 1 : (int)((3L * dev.cus + 2 * t - 1) / (2 * t));
-  } else if (2 * t128 >= 3L * dev.cus) {
-    p = {kTile128, 1};
-  } else if (t128 >= dev.cus) {
-    if (nk >= 96)
-      p = {kTile128, 3};
-    else if (10 * t128 <= 11L * dev.cus)
-      p = {kTile128, 2};
-    else
-      p = {kTile128x64, 2};
-  } else if (tile_count(m, n, kTile128x64) >= dev.cus) {
-    p = {kTile128x64, 2};
-  } else {
-    const long t = tile_count(m, n, kTile64);
-    p = {kTile64, (int)((3L * dev.cus + 2 * t - 1) / (2 * t))};
-  }
-  p.splits = std::min(p.splits, std::max(1, nk / 8));
+  Tile only{};
+  const bool one_tile = forced_tile(&only);
   const char *e = getenv("GEMMA_HIP_GEMM_F32_SPLIT");
-  if (e != nullptr) p.splits = atoi(e);
-  p.splits = std::max(1, std::min({p.splits, nk, 16}));
-  return p;
+  const int forced =
+      !may_split ? 1 : e == nullptr ? 0 : std::max(1, std::min({atoi(e), nk, 16}));
+  const int fewest = nk >= 16 && 2 * tile_count(m, n, kTile128) < 3L * dev.cus ? 2 : 1;
+  H2Plan best{kTile64, fewest};
+  double least = 1e300;
+  for (const Cost &c : kCosts) {
+    if (one_tile && c.tile != only) continue;
+    if (one_tile) best.tile = c.tile;
+    const long tiles = tile_count(m, n, c.tile);
+    for (int s = forced ? forced : fewest; s <= (forced ? forced : 16); ++s) {
+      const double partials = (double)tiles * s * c.bm * c.bn * 4;
+      if (!forced && s > 1 && (nk < 6 * s || partials > 5.0 * dev.cus * 128 * 128 * 4)) break;
+      const double wgs = (double)tiles * s / dev.cus, whole = std::ceil(wgs);
+      const double steps = (nk + s - 1) / s + c.ends;
+      // between the mean and the fullest CU's share: workgroups sharing a CU
+      // run faster once the others have ended
+      double us = steps * std::max(c.lat * std::ceil(wgs / c.slots), c.thr * (wgs + whole) / 2);
+      if (s > 1) us += kSplitUs + kPerSplitUs * s + partials / kPartialBytesPerUs;
+      if (us < least) {
+        least = us;
+        best = {c.tile, s};
+      }
+    }
+  }
+  return best;
 }
 
-hipError_t launch_bf3_auto(float *dst, int dstr, const F32Segs &b, int mstr, const float *src,
-                           int sstr, int m, int k, const F32Epilogue &ep, const DeviceInfo &dev,
-                           hipStream_t stream) {
-  Bf3Plan p = bf3_plan(m, b.end[b.nseg - 1], k, dev);
+hipError_t launch_h2_auto(float *dst, int dstr, const F32Segs &b, int mstr, const float *src,
+                          int sstr, int m, int k, const F32Epilogue &ep, const DeviceInfo &dev,
+                          hipStream_t stream) {
+  // the split-K workspace may have to be allocated: not under capture
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (p.splits > 1 &&
-      (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
-    p.splits = 1;  // the split-K workspace may have to be allocated: not under capture
+  const bool may_split =
+      hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+  const H2Plan p = h2_plan(m, b.end[b.nseg - 1], k, may_split, dev);
   if (p.tile == kTile128)
-    return launch_bf3<2, 2>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
+    return launch_h2<2, 2>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
   if (p.tile == kTile128x64)
-    return launch_bf3<2, 1>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
-  return launch_bf3<1, 1>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
+    return launch_h2<2, 1>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
+  return launch_h2<1, 1>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);
 }
 
 // float4 loads of both operands: K and the row strides multiples of 4
@@ -539,7 +657,7 @@ hipError_t launch_gemm_f32(float *dst, int dstr, const float *mat, int mstr,
   if (f32_vec4(k, mstr, sstr, mat, src)) {
     if (gemm_f32_split()) {
       const F32Segs b{{mat, nullptr, nullptr}, {n, n, n}, 1};
-      return launch_bf3_auto(dst, dstr, b, mstr, src, sstr, m, k, ep, dev, stream);
+      return launch_h2_auto(dst, dstr, b, mstr, src, sstr, m, k, ep, dev, stream);
     }
     const Tile tile = f32_tile(m, n, dev);
     if (tile == kTile128) {
@@ -570,7 +688,7 @@ hipError_t launch_gemm_f32_segs(float *dst, int dstr, const F32Segs &b, int mstr
   bool vec4 = true;
   for (int t = 0; t < b.nseg; ++t) vec4 = vec4 && f32_vec4(k, mstr, sstr, b.w[t], src);
   if (!f64 && vec4 && gemm_f32_split())
-    return launch_bf3_auto(dst, dstr, b, mstr, src, sstr, m, k, ep, dev, stream);
+    return launch_h2_auto(dst, dstr, b, mstr, src, sstr, m, k, ep, dev, stream);
   // one launch per segment, the epilogue's column-indexed inputs shifted
   // to the segment's first column
   for (int t = 0; t < b.nseg; ++t) {

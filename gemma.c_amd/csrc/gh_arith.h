@@ -307,4 +307,22 @@ __device__ __forceinline__ Bf3x2 split3x2(float a, float b) {
 }
 __device__ __forceinline__ bf8 as_bf8(u4 v) { return __builtin_bit_cast(bf8, v); }
 
+// Split precision on the f16 matrix cores: x, scaled by a power of two into
+// f16's upper range, as two f16 pieces (each rounded to nearest, the second
+// from the exact remainder: 22 significant bits).  A product a b summed from
+// a1 b0, a0 b1 and a0 b0 leaves out at most about 2^-21 |a b| (2^-23 rms); f16
+// x f16 products are exact in fp32.
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ h2 cvt_pk_f16(float a, float b) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  return __builtin_convertvector(f2{a, b}, h2);
+}
+// Magnitude for a scale: infinities and NaN don't set it (they stay what
+// they are in their own products and leave the others' precision alone).
+__device__ __forceinline__ float finite_abs(float x) {
+  const float a = fabsf(x);
+  return a <= 3.40282347e38f ? a : 0.0f;
+}
+
 }  // namespace gh

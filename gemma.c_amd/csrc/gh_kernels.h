@@ -164,7 +164,7 @@ hipError_t launch_gemm_f32(float *dst, int dstr, const float *mat, int mstr,
 
 // B as up to kMaxGemmSegs separate fp32 [rows][mstr] matrices whose outputs
 // are adjacent column ranges of one dst (q, k, v; or gate, up): segment t
-// holds output columns [end[t-1], end[t]) (end[-1] = 0).  The split-bf16
+// holds output columns [end[t-1], end[t]) (end[-1] = 0).  The split
 // kernel runs all segments in one launch (split-K when its tiles leave CUs
 // idle); the fp32-MFMA and fp64 kernels run one launch per segment.
 struct F32Segs {

@@ -343,7 +343,7 @@ typedef struct {
  * 5384, 5431) on the device: emb is the fp32 [nvocab][dim] table (also the
  * tied LM head), the projections run as fp32 GEMVs (gemv_fpx) in the step
  * (the norms fused into the q/k/v and gate/up GEMVs, GELU into gate/up, as
- * in the W8A8 step) and as fp32 GEMMs (gemm_fpx: on the bf16 matrix cores in
+ * in the W8A8 step) and as fp32 GEMMs (gemm_fpx: on the f16 matrix cores in
  * split precision, fp32 accuracy) in the prompt pass, with no activation
  * quantize.  Every other decoder entry point takes the result as it takes a
  * W8A8 decoder. */
@@ -487,9 +487,8 @@ int gemma_hip_vision_forward(gemma_hip_vision *vis, const float *img, float *out
  *   GEMMA_HIP_ATTN_F32 (the default) -- fp32 throughout as the reference
  *     computes it (its summation order differs), so results agree with the
  *     exact form to fp32 rounding, amplified where a later int8 quantization
- *     flips.  The patch GEMM runs on the bf16 matrix cores in split precision
- *     and the attention on the f16 ones: each fp32 operand is scaled by a
- *     power of two and split into two f16 pieces (22 significant bits), every
+ *     flips.  The patch GEMM and the attention run on the f16 matrix cores
+ *     in split precision: each fp32 operand is scaled by a power of two and split into two f16 pieces (22 significant bits), every
  *     product is summed from three piece products in fp32, and the result is
  *     closer to the exact one than with three bf16 pieces and six products
  *     (fewer fp32 roundings).  gemma_hip_vision_attention on a stream under

@@ -485,7 +485,7 @@ def check_f32(got, mat, src, oracle):
     assert np.all(err <= TOL_F32 * mag), f"worst relative error {worst:.3e}"
 
 
-# The fp32 GEMM has two kernels: split-bf16 on the bf16 matrix cores (the
+# The fp32 GEMM has two kernels: split precision on the f16 matrix cores (the
 # default) and fp32 MFMA (GEMMA_HIP_GEMM_F32=mfma); both are held to TOL_F32.
 F32_KERNELS = ["split", "mfma"]
 
@@ -588,6 +588,45 @@ def test_f32_split_k(gh, oracle, monkeypatch, splits, m, n, k):
     d.fill_(0.0)
     gh.matmul_f32(d, n, dev(B), k, dev(A), k, m, n, k, stream())
     assert np.array_equal(bits(host(d)), bits(first))
+
+
+# The split kernel's row scales: set from a row's first 32 values and raised
+# when a later step leaves their range (rows that grow along K, first values
+# zero, spikes in the ragged last step and in one split of K), over magnitudes
+# whose products reach both ends of fp32.  Besides TOL_F32, each value of a row may be off by
+# 2^-35 of the row's largest (the second f16 piece ends there).
+@pytest.mark.parametrize("tile,splits", [("128", 1), ("128x64", 2), ("64", 1), ("64", 3)])
+@pytest.mark.parametrize("m,n,k", [(130, 70, 100), (65, 129, 132), (3, 5, 32)])
+def test_f32_row_scales(gh, oracle, monkeypatch, tile, splits, m, n, k):
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32_TILE", tile)
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32_SPLIT", str(splits))
+    note(f"f32 row scales tile {tile} splits {splits} m={m} n={n} k={k}")
+    rng = np.random.default_rng(m + n + k)
+    A = rng.standard_normal((m, k))
+    B = rng.standard_normal((n, k))
+    for X, low, high in ((A, -90, 25), (B, -30, 25)):
+        kind = rng.integers(0, 6, len(X))
+        X[kind == 1] *= 2.0 ** np.linspace(0, 30, k)       # grows along K
+        X[kind == 2] *= 2.0 ** np.linspace(30, 0, k)       # shrinks
+        X[kind == 3, :min(k - 1, 40)] = 0                  # starts with zeros
+        X[kind == 4, -1] *= 2.0 ** 20                      # ends with a spike
+        X[kind == 5] = 0
+        X *= 2.0 ** rng.integers(low, high, (len(X), 1))
+    A, B = A.astype(np.float32), B.astype(np.float32)
+    d = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    gh.matmul_f32(d, n, dev(B), k, dev(A), k, m, n, k, stream())
+    exact, mag = oracle.gemm_f64(B, A)
+    a, b = np.abs(A).astype(np.float64), np.abs(B).astype(np.float64)
+    floor = 2.0 ** -35 * (np.outer(a.max(1), b.sum(1)) + np.outer(a.sum(1), b.max(1)))
+    assert np.all(np.abs(host(d) - exact) <= TOL_F32 * mag + floor)
+    zero = ~A.any(1)
+    assert not host(d)[zero].any()
+    # a value that isn't finite stays in its own row
+    A[1, k // 2] = np.inf
+    gh.matmul_f32(d, n, dev(B), k, dev(A), k, m, n, k, stream())
+    assert not np.isfinite(host(d)[1][B.any(1)]).any()
+    rest = np.arange(m) != 1
+    assert np.all(np.abs(host(d) - exact)[rest] <= (TOL_F32 * mag + floor)[rest])
 
 
 def test_f32_gemm_in_a_graph(gh, oracle, monkeypatch):
