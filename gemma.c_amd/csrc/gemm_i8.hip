@@ -1171,11 +1171,10 @@ __global__ __launch_bounds__(kThreads) void gemm_zero_kernel(int *p, int n) {
   if (i < n) p[i] = 0;
 }
 
-// A split-K launch: square tiles of 64 * wm (wm = 1: 64x64 tiles, four
-// 64-byte K stages; wm = 2: 128x128, two 128-byte stages) in `splits` pieces
-// (1 = no split).
+// A split-K launch: square tiles of 64 * wm (wm = 1: 64x64 tiles; wm = 2:
+// 128x128) and `stages` 128-byte K stages in `splits` pieces (1 = no split).
 struct SplitPlan {
-  int wm = 2, splits = 1;
+  int wm = 2, stages = 2, splits = 1;
 };
 
 int split_tiles(int m, int n, int wm) {
@@ -1228,28 +1227,37 @@ hipError_t launch_dma_split(bool heads, hipStream_t stream, float *dst, int dstr
 hipError_t launch_split(const SplitPlan &p, bool heads, hipStream_t stream, float *dst,
                         int dstr, int hdim, const GemmSegs &bs, int mstr, const int8_t *src,
                         int sstr, const float *ssc, int m, int k, const GemmWs *fixed) {
-  return p.wm == 1 ? launch_dma_split<1, 4, 64>(heads, stream, dst, dstr, hdim, bs, mstr, src,
-                                                sstr, ssc, m, k, p.splits, fixed)
-                   : launch_dma_split<2, 2, 128>(heads, stream, dst, dstr, hdim, bs, mstr, src,
-                                                 sstr, ssc, m, k, p.splits, fixed);
+  if (p.wm == 2)
+    return launch_dma_split<2, 2, 128>(heads, stream, dst, dstr, hdim, bs, mstr, src, sstr, ssc,
+                                       m, k, p.splits, fixed);
+  return p.stages == 4 ? launch_dma_split<1, 4, 128>(heads, stream, dst, dstr, hdim, bs, mstr,
+                                                     src, sstr, ssc, m, k, p.splits, fixed)
+                       : launch_dma_split<1, 3, 128>(heads, stream, dst, dstr, hdim, bs, mstr,
+                                                     src, sstr, ssc, m, k, p.splits, fixed);
 }
 
-// The split-K plan (splits = 1: none).  Measured on MI355X, the partial
-// tiles' round trip through memory costs about as much as 15 K stages, so a
-// split pays only when the grid leaves CUs idle and K is long.  With fewer
-// 64x64 tiles than CUs and K >= 2048, 64x64 tiles in about 1.5 workgroups per
-// CU (at most 6 pieces of at least 8 stages): gemma-3-1b down at 512 tokens
-// 23.3 -> 16.7 us (3 pieces; 128x128 tiles in 6 pieces: 23.3), at 256 tokens
-// 20.5 -> 13.0, gemma-3-4b down at 256 tokens 26.9 -> 22.2.  Otherwise, with
-// at most one 128x128 tile per two CUs and K >= 4096, 128x128 tiles in about
-// two workgroups per CU (at most 8 pieces): gemma-3-1b down at 1024 tokens
-// 28.6 -> 25.8 us, gemma-3-4b down at 512 tokens 40.7 -> 32.5.  Every
-// gemma-3-4b and SigLIP shape at full length (>= 256 tiles of 128x128) lost
-// 15-60% with forced splits.  GEMMA_HIP_GEMM_SPLIT forces 128x128 pieces.
+// The split-K plan (splits = 1: none).  The partial tiles' round trip through
+// memory costs about as much as 15 K stages, so a split pays only when the
+// grid leaves CUs idle and K is long.  Measured on MI355X (us):
+//  - fewer 64x64 tiles than CUs and K >= 2048: 64x64 tiles in about 1.5
+//    workgroups per CU, at most 6 pieces of at least 5 stages.  Four stages of
+//    128 bytes: a 64x64 tile's two products per 64-byte stage and wave are too
+//    few to cover the barrier (471x1152x6912 16.3 -> 14.5 in 3 pieces against
+//    four 64-byte stages, 256x2560x10240 21.9 -> 18.4, 300x640x2048 9.5 -> 8.3
+//    in 3 instead of 4; 23.3 unsplit at the first);
+//  - up to 1.5 64x64 tiles per CU and K >= 4096: 64x64 tiles in 2 pieces, all
+//    resident with three 128-byte stages (48 KiB, three per CU): 1024x1152x6912
+//    25.3 -> 21.7 against 128x128 tiles in 7 pieces, 1000x1152x4096 21.2 -> 15;
+//  - else, fewer 128x128 tiles than CUs and K >= 4096: 128x128 tiles in at most
+//    two workgroups per CU (at most 8 pieces): 1900x1152x6912 (135 tiles) 42.5
+//    unsplit -> 31.4 in 3, 2400x1152x6912 (171) 45.2 -> 39.1 in 2.  With a tile
+//    per CU or more, forced splits lost 15-60% (gemma-3-4b and SigLIP shapes).
+// At most 2 CUs' worth of 128x128 tiles, so a plan fits the static scratch.
+// GEMMA_HIP_GEMM_SPLIT forces 128x128 pieces.
 SplitPlan choose_split(int m, int n, int k, const DeviceInfo &dev, hipStream_t stream,
                        bool fixed_ws) {
   SplitPlan p;
-  const int nk128 = (k + 127) / 128, nk64 = (k + 63) / 64;
+  const int nk128 = (k + 127) / 128;
   const int forced = env_split();
   if (forced > 0) {
     p.splits = forced > nk128 ? nk128 : forced;
@@ -1258,11 +1266,12 @@ SplitPlan choose_split(int m, int n, int k, const DeviceInfo &dev, hipStream_t s
   const long tiles64 = split_tiles(m, n, 1), tiles128 = split_tiles(m, n, 2);
   if (tiles64 <= 0) return p;
   SplitPlan want;
-  if (tiles64 < dev.cus && nk64 >= 32) {
-    want.wm = 1;
+  if (tiles64 < dev.cus && nk128 >= 16) {
     const long fill = (3L * dev.cus + 2 * tiles64 - 1) / (2 * tiles64);  // ~1.5 per CU
-    want.splits = (int)std::min<long>({6, nk64 / 8, fill});
-  } else if (tiles128 * 2 <= dev.cus && nk128 >= 32) {
+    want = {1, 4, (int)std::min<long>({6, nk128 / 5, fill})};
+  } else if (2 * tiles64 <= 3L * dev.cus && nk128 >= 32) {
+    want = {1, 3, 2};
+  } else if (tiles128 < dev.cus && nk128 >= 32) {
     want.splits = (int)std::min<long>({8, 2L * dev.cus / tiles128, nk128 / 8});
   }
   if (want.splits < 2) return p;

@@ -463,6 +463,27 @@ def test_gemm_split_plans(gh, oracle, m, n, k):
         assert np.array_equal(bits(host(dst)), bits(ref)), f"launch {rep}"
 
 
+# The plans' other rules and edges: 64x64 tiles on 128-byte stages in 3 pieces
+# (K = 2064: 17 stages, the last of 16 bytes) and in 2 (288 and 328 tiles, three
+# stages, ragged in every dimension) and 128x128 tiles in 3 and 2 pieces (135
+# and 171 tiles).
+@pytest.mark.parametrize("m,n,k", [(300, 640, 2064), (1000, 1152, 4112), (480, 2570, 8208),
+                                   (1900, 1150, 4112), (2400, 1150, 4112)])
+def test_gemm_split_plan_rules(gh, oracle, m, n, k):
+    note(f"split plan m={m} n={n} k={k}")
+    rng = np.random.default_rng(m + n + k)
+    A = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    B = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    sa = rng.uniform(1e-3, 1e-2, m).astype(np.float32)
+    sb = rng.uniform(1e-3, 1e-2, n).astype(np.float32)
+    pick = np.unique(rng.integers(0, m, 64))
+    ref, _ = oracle.gemm_int8(B, sb, A[pick], sa[pick])
+    for rep in range(2):
+        dst = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+        gh.matmul(dst, n, dev(B), k, dev(sb), dev(A), k, dev(sa), m, n, k, stream())
+        assert np.array_equal(bits(host(dst)[pick]), bits(ref)), f"launch {rep}"
+
+
 def test_gemm_split_plan_heads(gh, oracle):
     m, heads, hdim, k = 300, 2, 256, 4096
     rng = np.random.default_rng(9)
