@@ -65,7 +65,7 @@ __global__ __launch_bounds__(NT) void dec_norm_gemv_kernel(DecNorm na, GemvJobs 
   hold_args(na);
   hold_args(jobs);
   if (GELU) exp_tab_load(etab);  // visible after the prologue's barriers
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   constexpr int kNpt = (CPL * L * 16 + NT * 4 - 1) / (NT * 4);
   static_assert(!GELU || L <= 32, "gate and up rows must share a wave");
   constexpr int kRowsPerWave = 64 / L;
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(NT) void dec_norm_gemv_kernel(DecNorm na, GemvJobs 
     if (GELU) {
       const float up = __shfl_xor(val, L, 64);
       if (sub == 0 && (rloc & 1) == 0 && row < total)
-        as_global(pick4(jobs.dst, 0))[r] = (float)(gelu((double)val, etab, ec) * (double)up);
+        as_global(pick4(jobs.dst, 0))[r] = (float)(gelu(val, etab, gc) * (double)up);
     } else if (sub == 0 && row < total) {
       as_global(pick4(jobs.dst, j))[r] = val;
     }
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kNT) void dec_norm_stream_kernel(DecNorm na, GemvJo
   // the exp table is loaded first and stored to LDS after the other loads
   // are issued (visible after the prologue's barriers)
   const double etv = GELU ? kExp2Tab[threadIdx.x & 127] : 0.0;
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   constexpr int R = 64 / L;
   static_assert(!GELU || R >= 2, "gate and up rows must share a wave");
   const int lane = threadIdx.x & 63;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(kNT) void dec_norm_stream_kernel(DecNorm na, GemvJo
     if (GELU) {
       const float up = __shfl_xor(val, L, 64);  // the up row's lanes
       if (sub == 0 && (rloc & 1) == 0 && a.ok)
-        as_global(pick4(jobs.dst, 0))[a.out] = (float)(gelu((double)val, etab, ec) * (double)up);
+        as_global(pick4(jobs.dst, 0))[a.out] = (float)(gelu(val, etab, gc) * (double)up);
     } else if (sub == 0 && a.ok) {
       as_global(pick4(jobs.dst, a.job))[a.out] = val;
     }
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(kNT) void dec_norm_f32_kernel(DecNorm na, GemvJobs 
   hold_args(jobs);
   asm volatile("" ::"s"(ngroups), "s"(k), "s"(passes));
   const double etv = GELU ? kExp2Tab[threadIdx.x & 127] : 0.0;
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   constexpr int R = 64 / L;
   static_assert(!GELU || R >= 2, "gate and up rows must share a wave");
   const int lane = threadIdx.x & 63;
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(kNT) void dec_norm_f32_kernel(DecNorm na, GemvJobs 
         const float up = __shfl_xor(acc, L, 64);  // the up row's lanes
         if (sub == 0 && (rloc & 1) == 0 && a.ok)
           as_global(pick4(jobs.dst, 0))[a.out] =
-              (float)(gelu((double)acc, etab, ec) * (double)up);
+              (float)(gelu(acc, etab, gc) * (double)up);
       } else if (sub == 0 && a.ok) {
         as_global(pick4(jobs.dst, a.job))[a.out] = acc;
       }

@@ -912,7 +912,7 @@ __global__ __launch_bounds__(kNT) void pf_attn_merge_kernel(PfAttn a, int hdim) 
 __global__ __launch_bounds__(kNT) void gelu_mul_rows_kernel(float *g, int mlp) {
   __shared__ double etab[128];
   exp_tab_load(etab);
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   const int c = blockIdx.x * kNT + threadIdx.x;
   float *gate = g + (size_t)blockIdx.y * 2 * mlp;
   const bool ok = c < mlp / 4;
@@ -925,7 +925,7 @@ __global__ __launch_bounds__(kNT) void gelu_mul_rows_kernel(float *g, int mlp) {
   if (!ok) return;
   v4f out;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) out[e] = (float)(gelu((double)gv[e], etab, ec) * (double)uv[e]);
+  for (int e = 0; e < 4; ++e) out[e] = (float)(gelu(gv[e], etab, gc) * (double)uv[e]);
   reinterpret_cast<v4f *>(gate)[c] = out;
 }
 
@@ -938,7 +938,7 @@ __global__ __launch_bounds__(NT) void pf_gelu_quant_kernel(const float *g, int m
   __shared__ float redf[NT / 64];
   __shared__ double etab[128];
   exp_tab_load(etab);
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   const int tid = threadIdx.x;
   const int n4 = mlp >> 2;
   const float *gate = g + (size_t)blockIdx.x * 2 * mlp;
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(NT) void pf_gelu_quant_kernel(const float *g, int m
   for (int j = 0; j < NPT; ++j)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      out[j][e] = (float)(gelu((double)gv[j][e], etab, ec) * (double)uv[j][e]);
+      out[j][e] = (float)(gelu(gv[j][e], etab, gc) * (double)uv[j][e]);
       amax = fmaxf(amax, abs_daz(out[j][e]));
     }
   amax = block_max<NT>(amax, redf);

@@ -481,7 +481,7 @@ __global__ __launch_bounds__(NT) void vis_gelu_quant_kernel(const float *hbuf, c
   __shared__ float redf[NT / 64];
   __shared__ double etab[128];
   exp_tab_load(etab);
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   const int tid = threadIdx.x, n4 = mlp >> 2;
   const float *row = hbuf + (size_t)blockIdx.x * mlp;
   v4f hv[NPT], bv[NPT];
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(NT) void vis_gelu_quant_kernel(const float *hbuf, c
   for (int j = 0; j < NPT; ++j)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      out[j][e] = (float)gelu((double)(hv[j][e] + bv[j][e]), etab, ec);
+      out[j][e] = (float)gelu(hv[j][e] + bv[j][e], etab, gc);
       amax = fmaxf(amax, abs_daz(out[j][e]));
     }
   amax = block_max<NT>(amax, redf);
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(kNT) void vis_pool_kernel(VisPool a) {
 __global__ __launch_bounds__(kNT) void vis_bias_gelu_kernel(float *h, const float *bias, int mlp) {
   __shared__ double etab[128];
   exp_tab_load(etab);
-  const ExpConsts ec = exp_consts();
+  const GeluConsts gc = gelu_consts();
   const int c = blockIdx.x * kNT + threadIdx.x;
   float *row = h + (size_t)blockIdx.y * mlp;
   const bool ok = c < mlp / 4;
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(kNT) void vis_bias_gelu_kernel(float *h, const floa
   if (!ok) return;
   v4f out;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) out[e] = (float)gelu((double)(hv[e] + bv[e]), etab, ec);
+  for (int e = 0; e < 4; ++e) out[e] = (float)gelu(hv[e] + bv[e], etab, gc);
   reinterpret_cast<v4f *>(row)[c] = out;
 }
 
