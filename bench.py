@@ -43,7 +43,7 @@ The JSON line also carries, measured in the same run:
                 embedding, norms, q/k/v, RoPE, KV cache, attention, o, GELU,
                 down, LM head, argmax); "gemma-3-1b:U" is config 3 as an
                 unquantized ('U') model (gemma_hip_decoder_create_f32: fp32
-                GEMVs, ~4 GB of weights per token; split-bf16 fp32 GEMMs in
+                GEMVs, ~4 GB of weights per token; split fp32 GEMMs in
                 the prompt pass)
   vision        config 4 end to end: one 896x896 image through the SigLIP
                 tower on the GPU (gemma_hip_vision_forward), ms per image;
@@ -349,7 +349,7 @@ def bench_gemm_f32(torch, gh, gen, timer, reps):
         out[name] = dict(m=m, n=n, k=k, us=round(ms * 1e3, 2), tflops=round(tf, 1),
                          frac=round(tf / peak, 4))
         del a, b, d
-    return {"kernel": "split-bf16" if split else "fp32-mfma", "peak_tflops": round(peak, 1),
+    return {"kernel": "split-f16" if split else "fp32-mfma", "peak_tflops": round(peak, 1),
             "shapes": out}
 
 
@@ -512,7 +512,7 @@ def bench_vision(torch, gh) -> dict:
     fp32 matrix cores (the default) and on the fp64 matrix cores (the
     verification mode, equal to the fp64 oracle; gemma_hip_vision_set_attention);
     then the same tower from fp32 weights (an unquantized 'U' file:
-    gemma_hip_vision_create_f32, fp32 GEMMs on the split-bf16 kernel)."""
+    gemma_hip_vision_create_f32, fp32 GEMMs on the split kernel)."""
     import statistics
     import time
 

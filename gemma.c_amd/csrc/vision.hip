@@ -129,7 +129,7 @@ __global__ __launch_bounds__(NT) void vis_ln_rows_kernel(VisLn a) {
 // the end.  Every sum is fp64; each output is rounded to fp32 once.
 constexpr int kVaKeys = 32;          // keys per tile
 constexpr int kVaWaves = 8;          // waves (16 queries each) per workgroup
-constexpr int kVbWaves = 16;         // ... of the split-bf16 kernel (head dims <= 72)
+constexpr int kVbWaves = 16;         // ... of the three-bf16 kernel (head dims <= 72)
 constexpr double kVaSlack = 64.0;    // e^64 * 3.4e38 * n keys stays far below DBL_MAX
 
 template <int HD, int NW>
