@@ -1155,7 +1155,9 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
     return hipErrorInvalidValue;
   bool splitk = false;  // the split-f16 kernel
   PaGeo geo{};
-  if (f32 && a.planes != nullptr) {
+  // (the split kernel takes each tile's largest score from its largest raw
+  // product: a negative scale would make that the smallest)
+  if (f32 && a.planes != nullptr && a.asc >= 0.0f) {
     const PfKind kind = pf_attn_kind();
     if (kind != kPfF32) {
       geo = pa_geo(a, kPbQ);

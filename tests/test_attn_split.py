@@ -160,7 +160,7 @@ def test_vision_attention_under_capture(gh):
         _close(_vision(gh, qkv, bias, heads, dim), want)
 
 
-def _prefill_want(q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense):
+def _prefill_want(q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense, asc=None):
     ctx = pos0 + n
     pos = pos0 + np.arange(n)
     j = np.arange(ctx)[None, :]
@@ -170,21 +170,21 @@ def _prefill_want(q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense):
     out = []
     for h in range(nh):
         s = q[:, h * hd:(h + 1) * hd].astype(F64) @ kc[h // (nh // nkv), :ctx].astype(F64).T
-        s = s / np.sqrt(F64(hd))
+        s = s / np.sqrt(F64(hd)) if asc is None else s * F64(np.float32(asc))
         if cap:
             s = np.tanh(s / cap) * cap
         out.append(_softmax_av(np.where(live, s, -np.inf), vc[h // (nh // nkv), :ctx].astype(F64)))
     return np.concatenate(out, axis=1)
 
 
-def _prefill(gh, q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense):
+def _prefill(gh, q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense, asc=None):
     import torch
 
     dq, dk, dv = (torch.from_numpy(a).cuda() for a in (q, kc, vc))
     out = torch.full((n + 1, nh * hd), float("nan"), device="cuda")
     gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, pos0, nh, nkv, hd, kc.shape[1], slide,
-                         np.float32(1.0) / np.sqrt(np.float32(hd)), cap, dense, 1,
-                         stream=torch.cuda.current_stream().cuda_stream)
+                         np.float32(1.0) / np.sqrt(np.float32(hd)) if asc is None else asc, cap,
+                         dense, 1, stream=torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     got = out.cpu().numpy()
     assert np.isnan(got[n]).all()
@@ -232,6 +232,20 @@ def test_prefill_tiles_of_any_magnitude(gh, monkeypatch, hd):
     got, want = _prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args)
     for i in range(n):
         _close(got[i], want[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["", "bf3", "f32"])
+@pytest.mark.parametrize("n,hd,asc,cap", [(750, 256, -0.0625, 0.0), (90, 256, -0.25, 20.0),
+                                          (90, 128, -0.5, 0.0), (90, 256, 0.0, 0.0)])
+def test_prefill_scale_sign(gh, monkeypatch, kind, n, hd, asc, cap):
+    """Scores are q.k * asc for any asc, whichever kernel runs: negative, and
+    zero (every visible key weighs the same)."""
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", kind)
+    q, kc, vc = _prefill_inputs(n, 7, 4, 1, hd, seed=n)
+    q *= np.float32(0.5)  # |q.k| asc stays below 16, as TOL assumes
+    args = (n, 7, 4, 1, hd, 0, cap, False, asc)
+    _close(_prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args))
 
 
 @pytest.mark.gpu
