@@ -12,10 +12,14 @@
 // products.  Measured against 64-bit sums: see the tests' bars.
 //
 // Scales are exact powers of two: one per query, one per 32-key tile of K
-// and one per tile of V (attn_pack_kernel), so a tile of outliers costs no
-// other tile its precision.  K's goes into the softmax's scale, V's into the
-// weights (the value sums are kept in units of a running exponent, as the
-// weights are relative to a running maximum).
+// and one per tile of V (attn_pack_kernel).  K's goes into the softmax's scale,
+// V's into the weights: the value sums are kept in units of the largest V tile
+// of the workgroup's keys.
+//
+// Two f16 pieces hold a value's 22 bits only near its tile's largest, so a
+// workgroup first looks at what its tiles hold (TileRange: finite, V's tiles
+// within 2^8 of each other, kept by attn_pack_kernel) and otherwise computes
+// its queries by AttnBf3: three bf16 pieces and six products, at any magnitude.
 //
 // K and V are split once per key and layer by attn_pack_kernel into tiles of
 // 32 keys whose pieces lie in the order in which a wave reads its operands:
@@ -29,6 +33,7 @@
 
 #include <float.h>
 #include <limits.h>
+#include <math.h>
 
 #include <type_traits>
 
@@ -76,6 +81,11 @@ __device__ __forceinline__ void split8(const float (&x)[8], h8 *hi, h8 *lo) {
     (*lo)[e + 1] = b[1];
   }
 }
+// Magnitude; infinite for what isn't finite.
+__device__ __forceinline__ float abs_or_inf(float x) {
+  const float a = fabsf(x);
+  return a <= FLT_MAX ? a : INFINITY;
+}
 // E such that amax 2^-E lies in [2^14, 2^15), f16's upper range; 0 for 0.
 __device__ __forceinline__ int scale_exp(float amax) {
   return amax > 0.0f ? ilogbf(amax) - 14 : 0;
@@ -86,6 +96,14 @@ __device__ __forceinline__ int scale_exp4(float amax) {
   return amax > 0.0f ? (scale_exp(amax) + 3 + 1024) / 4 * 4 - 1024 : 0;
 }
 
+// What a packed tile holds, for the choice between the two forms.
+struct TileRange {
+  int ek, ev;   // exponents of K and V; ek INT_MAX: K is not finite
+  float vtop;   // V's largest magnitude; infinite: V is not finite
+  float vlow;   // f16 pieces keep this tile's V beside others of up to this magnitude
+};
+constexpr float kVReach = 0x1p8f;  // how far V's magnitudes may lie apart
+
 // Two workgroups per (32-key tile, kv head), K and V: rows 32 t .. 32 t + 31
 // (rows from `keys` on are zero) with their biases, scaled and split into the
 // tile's fragments.  Memory-bound: reads and writes 4 bytes a value once.
@@ -95,7 +113,7 @@ struct AttnPack {
   const float *bk, *bv;          // biases [heads][HD], or null
   int tile0, ntiles, keys;
   char *planes;                  // [head][ntiles] tiles, tile0 first
-  int2 *exps;                    // [head][ntiles] exponents of K and V
+  TileRange *range;              // [head][ntiles]
 };
 
 // Threads of a packing workgroup: one item of eight values each, up to 512.
@@ -152,15 +170,25 @@ __global__ __launch_bounds__(kPackThreads<HD>) void attn_pack_kernel(AttnPack a)
 #pragma unroll
   for (int j = 0; j < PT; ++j)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, finite_abs(x[j][e]));
+    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, abs_or_inf(x[j][e]));
   amax = wave_max_dpp(amax);
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
-  const int ex = isv ? scale_exp4(amax) : scale_exp(amax);
+  const bool finite = amax <= FLT_MAX;  // if not, the pieces are of no use
+  const int ex = !finite ? 0 : isv ? scale_exp4(amax) : scale_exp(amax);
   const size_t at = (size_t)h * a.ntiles + blockIdx.x;
-  if (tid == 0) reinterpret_cast<int *>(a.exps + at)[isv ? 1 : 0] = ex;
+  if (tid == 0) {
+    TileRange *r = a.range + at;
+    if (isv) {
+      r->ev = ex;
+      r->vtop = amax;
+      r->vlow = amax * kVReach;
+    } else {
+      r->ek = finite ? ex : INT_MAX;
+    }
+  }
   char *kf = a.planes + at * G::kBytes, *vf = kf + G::KFR * 1024;
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
@@ -213,16 +241,28 @@ __device__ __forceinline__ void attn_dma(const char *base, uint32_t off, const v
 #pragma clang diagnostic pop
 }
 
+// ... and each lane's 16 bytes from an address of its own.
+__device__ __forceinline__ void attn_dma_rows(const float *src, const void *lds) {
+  const uint32_t m = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)lds;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m), "v"(src)
+               : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 // What a lane's query sees: keys ws .. p_top; every query of its wave sees keys
 // f_lo .. f_hi.
 struct AttnSee {
   int ws, p_top, f_lo, f_hi;
 };
 
+constexpr float kLog2e = 1.44269502162933349609375f;  // fl(log2 e)
+constexpr float kLog2eLo = 1.92596298909109e-8f;      // log2 e - fl(log2 e)
 constexpr float kAttnFloor = -0x1p55f;  // the reference before a query has seen a key
 constexpr int kAttnTop = 15;          // weights stay below 2^15
+constexpr float kAttnVTop = 0x1p100f;  // the value sums stay finite below
 constexpr int kAttnSet = 7;           // a moved reference puts the largest at 2^6 .. 2^7
-constexpr int kAttnReach = 64;        // octaves between tiles of V that one query's sums can hold
 
 // The attention of one wave's 32 queries over tiles ta .. tb (packed tiles of
 // its kv head; the workgroup's waves share them through LDS).  On return
@@ -345,52 +385,30 @@ struct AttnWave {
 #pragma unroll
     for (int b = 0; b < G::NB; ++b) o[b] *= f;
   }
-  // Moves the running maximum and exponent for a tile whose largest score of
-  // the lane is top2 (base 2) and whose V has exponent ev.  Rarely does
-  // anything: the maximum has kAttnTop - kAttnSet octaves of slack, V's
-  // exponent goes up at once and down with slack (settled() says whether it
-  // would).  Returns how far the tile's
-  // units lie below the sums' (<= 0), for the weights to carry.  A tile more
-  // than kAttnReach octaves below the sums is out of their reach: it only adds
-  // its weights to l, here (with the returned -1000 they vanish elsewhere).
-  __device__ __forceinline__ int refer(const v16f &x, float c1, float c2, float top2, int ev,
-                                       bool first) {
-    if (__any(top2 > m2 + (float)kAttnTop)) {
-      const float rmax = fmaxf(top2, __shfl_xor(top2, 32, 64));
-      const float m_new = fmaxf(m2, ceilf(rmax) - (float)kAttnSet);
-      const float alpha = __builtin_amdgcn_exp2f(m2 - m_new);  // a power of two, or 0
-      m2 = m_new;
-      l *= alpha;
-      if (!first) scale_o(alpha);
-    }
-    int df = ev - e_o;
-    if (df > 0 || df < -8) {  // wave-uniform
-      if (df >= -kAttnReach) {
-        if (!first) scale_o(ldexpf(1.0f, max(-df, -300)));
-        e_o = ev;
-        df = 0;
-      } else {
-        float s = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s += __builtin_amdgcn_exp2f(fmaf(x[r], c1, fmaf(x[r], c2, -m2)));
-        l += s;
-        df = -1000;
-      }
-    }
-    return df;
+  // Moves the running maximum for a tile whose largest score of the lane is
+  // top2 (base 2).  Rarely does anything: the maximum has kAttnTop - kAttnSet
+  // octaves of slack (settled() says whether it would).
+  __device__ __forceinline__ void refer(float top2, bool first) {
+    if (settled(top2)) return;
+    const float rmax = fmaxf(top2, __shfl_xor(top2, 32, 64));
+    const float m_new = fmaxf(m2, ceilf(rmax) - (float)kAttnSet);
+    const float alpha = __builtin_amdgcn_exp2f(m2 - m_new);  // a power of two, or 0
+    m2 = m_new;
+    l *= alpha;
+    if (!first) scale_o(alpha);
   }
 
-  __device__ __forceinline__ bool settled(float top2, int df) const {
-    return !__any(top2 > m2 + (float)kAttnTop) && df <= 0 && df >= -8;
+  __device__ __forceinline__ bool settled(float top2) const {
+    return !__any(top2 > m2 + (float)kAttnTop);
   }
 
-  // lds: 2 K tiles, then 2 V tiles.  c_hi + c_lo: the scores' scale (asc)
-  // times log2 e, without the tiles' exponents; cap: the soft cap of the
-  // scaled scores (0: none).
-  __device__ __forceinline__ void run(const char *tiles, const int2 *exps, int ta, int tb,
+  // lds: 2 K tiles, then 2 V tiles; red: a v4f per wave.  c_hi + c_lo: the
+  // scores' scale (asc) times log2 e, without the tiles' exponents; cap: the
+  // soft cap of the scaled scores (0: none).  False, for the whole workgroup
+  // and with nothing computed, where the tiles hold what two f16 pieces don't.
+  __device__ __forceinline__ bool run(const char *tiles, const TileRange *range, int ta, int tb,
                                       const AttnSee &see, float asc, float c_hi, float c_lo,
-                                      float cap, char *lds, int wave, int lane) {
+                                      float cap, char *lds, v4f *red, int wave, int lane) {
     const int half = lane >> 5;
     char *kbuf = lds, *vbuf = lds + 2 * G::KFR * 1024;
     const uint32_t loff = lane * 16;
@@ -419,20 +437,41 @@ struct AttnWave {
     for (int b = 0; b < G::NB; ++b) o[b] = v16f{};
     m2 = kAttnFloor;
     l = 0.0f;
-    e_o = -(1 << 20);  // below every exponent: the first tile sets it
 
-    int2 ex = exps[ta + zero];
+    auto exps = [&](int t) { return *reinterpret_cast<const int2 *>(&range[t].ek); };
+    int2 ex = exps(ta + zero);
     fetch_k(ta);
     fetch_v(ta);
+    float vtop = 0.0f, vlow = FLT_MAX;
+    bool finite = true;
+    for (int t = ta + 64 * wave + lane; t <= tb; t += 64 * NW) {
+      const TileRange r = range[t];
+      vtop = fmaxf(vtop, r.vtop);
+      vlow = fminf(vlow, r.vlow);
+      finite = finite && r.ek != INT_MAX;
+    }
+    red[wave] = v4f{wave_max_dpp(vtop), -wave_max_dpp(-vlow), __all(finite) ? 0.0f : 1.0f, 0.0f};
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's DMAs landed
     lds_barrier();                       // every wave's did
+    vtop = red[0][0], vlow = red[0][1];
+    float bad = red[0][2];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+      vtop = fmaxf(vtop, red[w][0]);
+      vlow = fminf(vlow, red[w][1]);
+      bad += red[w][2];
+    }
+    const bool fit = bad == 0.0f && vtop <= kAttnVTop && vlow >= vtop;
+    if (!__builtin_amdgcn_readfirstlane((int)fit)) return false;
+    e_o = __builtin_amdgcn_readfirstlane(scale_exp4(vtop));  // the largest tile's exponent
     if (ta < tb) fetch_k(ta + 1);
     v16f sc = {};
     {
       const char *k0 = kbuf + (ta & 1) * (G::KFR * 1024) + loff;
       const h8 none[2][2] = {};
       h8 f[kQ][2];
-      each_chunk(std::integral_constant<int, (kQ < 4 ? kQ : 4)>{}, [&](auto I) { read<I>(k0, nullptr, f[I]); });
+      each_chunk(std::integral_constant<int, (kQ < 4 ? kQ : 4)>{},
+                 [&](auto I) { read<I>(k0, nullptr, f[I]); });
       __builtin_amdgcn_sched_barrier(0);
       each_chunk(std::integral_constant<int, kQ>{}, [&](auto I) {
         if constexpr (I + 4 < kQ) read<I + 4>(k0, nullptr, f[I + 4]);
@@ -458,7 +497,7 @@ struct AttnWave {
       const int ek = __builtin_amdgcn_readfirstlane(ex.x);
       ev = __builtin_amdgcn_readfirstlane(ex.y);
       if (t < tb) {
-        ex = exps[t + 1 + zero];
+        ex = exps(t + 1 + zero);
         fetch_v(t + 1);
         if (t + 1 < tb) fetch_k(t + 2);
       }
@@ -470,8 +509,8 @@ struct AttnWave {
         const float as = ldexpf(asc, ek);
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[r] = tanhf(sc[r] * as / cap) * cap;
-        c1 = 1.44269502162933349609375f;  // fl(log2 e)
-        c2 = 1.92596298909109e-8f;        // log2 e - fl(log2 e)
+        c1 = kLog2e;
+        c2 = kLog2eLo;
       }
       if (32 * t < see.f_lo || 32 * t + 31 > see.f_hi) {  // wave-uniform: some key masked
         // a score whose weight is 0: -2^118 once scaled, or -2^57 and below
@@ -490,8 +529,9 @@ struct AttnWave {
     int t = ta;
     begin(t);
     for (;;) {
-      int df = refer(sc, c1, c2, top2, ev, t == ta);
+      refer(top2, t == ta);
       do {
+        const int df = ev - e_o;  // the tile's units below the sums', for the weights to carry
         const float m = m2 - (float)df;
         const char *kn = kbuf + ((t + 1) & 1) * (G::KFR * 1024) + loff;
         const char *vt = vbuf + (t & 1) * (G::VFR * 1024) + loff;
@@ -516,17 +556,17 @@ struct AttnWave {
             for (int j = 8 * I / n; j < 8 * (I + 1) / n; ++j) weights(j, sc, c1, c2, m, sum, p);
           if constexpr (I == n)
             l += (((sum[0] + sum[1]) + (sum[2] + sum[3])) +
-                  ((sum[4] + sum[5]) + (sum[6] + sum[7]))) * ldexpf(1.0f, df < -8 ? 0 : -df);
+                  ((sum[4] + sum[5]) + (sum[6] + sum[7]))) * ldexpf(1.0f, -df);
           __builtin_amdgcn_sched_barrier(0);
         });
         sc = sn;
         if (++t > tb) break;
         begin(t);
-        df = ev - e_o;
-      } while (settled(top2, df));
+      } while (settled(top2));
       if (t > tb) break;
     }
     l += __shfl_xor(l, 32, 64);
+    return true;
   }
 
   // The value sums of dims 32 b + 8 j + 4 (lane / 32) .. + 3, in units of 2^e_o
@@ -548,6 +588,296 @@ struct AttnWave {
         if (32 * b + 8 * j < HD) f(32 * b + 8 * j + 4 * half, dims(b, j));
   }
 };
+
+// The same attention at any magnitude, on the bf16 matrix cores: every fp32
+// operand x of the two products (q, k, the weights p and v) as three bf16
+// pieces x = x0 + x1 + x2 (split3x2: 24 significant bits, fp32's exponents),
+// each product a b from the six piece products whose orders add up to at most
+// 2, the small ones first, on v_mfma_f32_16x16x32_bf16 (lane l: A[l%16][8(l/16)
+// .. +7], B[8(l/16) .. +7][l%16], D[4(l/16) + r][l%16]) with fp32 accumulation:
+// the dropped ones are below 3 * 2^-24 |a b|, and bf16 x bf16 products are
+// exact there.  NW waves x 16 queries of one head, 32-key tiles of
+// K and V as they stand in memory: a tile's K rows come by LDS DMA into a
+// staging buffer while the tile before is in use, and its V rows likewise (VS)
+// or at its start; there they get their biases and are split,
+// once per workgroup, into planes: K [key][dim] (head dims padded to whole
+// 32-dim chunks) and V^T [dim][k], where k = 8 g + 4 b + r is the value
+// product's index of key 16 b + 4 g + r, the key whose score lane (query, g)
+// holds in element r of block b, so a lane's eight weights are its operand of
+// that product as they stand.  Lane (query col, g) ends with dims 16 nb + 4 g
+// .. + 3 in o[nb].  A wave skips the tiles that none of its queries sees.
+struct AttnRows {
+  const float *k, *v;    // row r at r * stride
+  size_t stride;
+  const float *bk, *bv;  // biases, or null
+};
+// What a lane's query sees, what each of its wave's 16 sees and what any does.
+struct AttnGroup {
+  int ws, p_top, f_lo, f_hi, w_lo, w_hi;
+};
+
+// VS: V's rows come through the staging buffer too, during the tile before; not
+// where the LDS for it would cost the f16 form of the same kernel a workgroup.
+// BIAS: K, V and the queries have biases.
+template <int HD, int NW, bool BIAS, bool VS>
+struct AttnBf3 {
+  static constexpr int TK = 32;              // keys per tile
+  static constexpr int NT = NW * 64;
+  static constexpr int CH = (HD + 31) / 32;  // 32-dim chunks of the score product
+  static constexpr int DP = CH * 32;         // padded head dim of the K planes
+  // A last chunk of 8 dims (head dim 72) takes two MFMAs instead of six: its
+  // k index carries four piece products over the 8 dims, k = 8 g + e for
+  // dim 32 CF + e of piece pair g (first MFMA: k2 q0, k1 q1, k0 q2, k1 q0;
+  // second: k0 q1, k0 q0 and two zero pairs)
+  static constexpr bool kTail8 = HD % 32 == 8;
+  static constexpr int CF = kTail8 ? CH - 1 : CH;  // chunks summed piece by piece
+  static constexpr int NB = (HD + 15) / 16;  // 16-dim output blocks
+  static constexpr int RK = DP + 8;          // K plane row (bf16): 16 rows in distinct banks
+  static constexpr int RV = TK + 8;          // V^T plane row (bf16)
+  static constexpr int C4 = HD / 4;          // float4 per key row
+  static constexpr int SG = TK * C4;         // float4 of a K tile
+  static constexpr int VB = 8 * C4;          // V blocks of a tile
+  static constexpr int kUnroll = VS ? 4 : 1;
+  // planes 16 bytes apart in the banks: the first tail MFMA reads three of
+  // them at one offset
+  static constexpr int kKPlane = TK * RK + 8, kVPlane = NB * 16 * RV;
+  static constexpr size_t kBytes =
+      (size_t)(kKPlane + kVPlane) * 6 + (size_t)((VS ? 2 : 1) * SG + 2 * C4) * 16;
+  static_assert(HD % 8 == 0 && SG % 64 == 0 && kKPlane % 8 == 0, "head dim");
+
+  v4f o[NB];
+  float m, l;  // base-2 reference maximum (a whole number) and weights' sum
+
+  // qrow, see: the lane's query.  vexp: V enters as v 2^-vexp (for
+  // values whose pieces bf16 would not hold), and so do the sums.
+  __device__ __forceinline__ void run(const AttnRows &rows, int k_lo, int k_end,
+                                      const float *qrow, const float *qbias,
+                                      const AttnGroup &see, float asc, float cap, int vexp,
+                                      char *lds, int wave, int lane) {
+    __bf16 *kt = reinterpret_cast<__bf16 *>(lds);
+    __bf16 *vt = kt + 3 * kKPlane;
+    v4f *stg = reinterpret_cast<v4f *>(vt + 3 * kVPlane);
+    v4f *kvb = stg + (VS ? 2 : 1) * SG;  // K's bias, then V's
+    const int tid = 64 * wave + lane, col = lane & 15, grp = lane >> 4;
+
+    // the queries' pieces: lane (col, g) holds dims 32 c + 8 g .. + 7
+    bf8 qa[3][CH];
+    bf8 qt1 = {}, qt2 = {};
+    int tsel = 0;  // the K plane lane (col, g) reads in the first tail MFMA
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      u4 w0, w1, w2;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const int d = 32 * c + 8 * grp + e;  // HD is even: d and d + 1 are both in or out
+        float x0 = 0.0f, x1 = 0.0f;
+        if (HD % 32 == 0 || d < HD) {
+          x0 = BIAS ? qrow[d] + qbias[d] : qrow[d];
+          x1 = BIAS ? qrow[d + 1] + qbias[d + 1] : qrow[d + 1];
+        }
+        const Bf3x2 sp = split3x2(x0, x1);
+        w0[e / 2] = sp.q0;
+        w1[e / 2] = sp.q1;
+        w2[e / 2] = sp.q2;
+      }
+      qa[0][c] = as_bf8(w0);
+      qa[1][c] = as_bf8(w1);
+      qa[2][c] = as_bf8(w2);
+    }
+    // the tail chunk's operands: lane (col, 0) holds dims 32 CF .. + 7 of
+    // every piece in qa[p][CF]; lane (col, g) takes the piece of pair g
+    if constexpr (kTail8) {
+      u4 t[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const u4 v = __builtin_bit_cast(u4, qa[p][CF]);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) t[p][d] = (uint32_t)__shfl((int)v[d], col, 64);
+      }
+      qt1 = as_bf8(grp == 1 ? t[1] : grp == 2 ? t[2] : t[0]);          // q0 q1 q2 q0
+      qt2 = as_bf8(grp == 0 ? t[1] : grp == 1 ? t[0] : u4{0, 0, 0, 0});  // q1 q0 0 0
+      tsel = grp == 0 ? 2 : grp == 2 ? 0 : 1;                               // k2 k1 k0 k1
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) o[nb] = v4f{0.f, 0.f, 0.f, 0.f};
+    m = kFloor;
+    l = 0.0f;
+    const float c1 = kLog2e, c2 = kLog2eLo;
+
+    // zero padding: K dims HD .. DP-1 and V^T rows HD .. 16 NB - 1, never staged
+    const __bf16 bz = (__bf16)0.0f;
+    constexpr int KP = DP - HD > 0 ? DP - HD : 1, VP = 16 * NB - HD > 0 ? 16 * NB - HD : 1;
+    for (int i = tid; i < 3 * TK * (DP - HD); i += NT) {
+      const int p = i / (TK * KP), j = i % (TK * KP);
+      kt[p * kKPlane + (j / KP) * RK + HD + j % KP] = bz;
+    }
+    for (int i = tid; i < 3 * (16 * NB - HD) * RV; i += NT) {
+      const int p = i / (VP * RV), j = i % (VP * RV);
+      vt[p * kVPlane + HD * RV + j] = bz;
+    }
+    if constexpr (BIAS)
+      for (int i = tid; i < 2 * C4; i += NT)
+        kvb[i] = reinterpret_cast<const v4f *>(i < C4 ? rows.bk : rows.bv)[i % C4];
+
+    auto fetch = [&](int t0) {  // rows past the last repeat it: their weights are 0
+      for (int i = wave; i < (VS ? 2 : 1) * SG / 64; i += NW) {  // wave-uniform
+        const int ch = (64 * i + lane) % SG, t = ch / C4;
+        attn_dma_rows((i < SG / 64 ? rows.k : rows.v) +
+                          (size_t)min(t0 + t, k_end) * rows.stride + 4 * (ch - t * C4),
+                      stg + 64 * i);
+      }
+    };
+    fetch(k_lo);
+    for (int t0 = k_lo; t0 <= k_end; t0 += TK) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's DMAs landed
+      lds_barrier();  // every wave's did, and every wave is done with the planes
+#pragma unroll kUnroll
+      for (int j = 0; j < (SG + NT - 1) / NT; ++j) {
+        const int i = tid + j * NT;
+        if (i >= SG) break;
+        const int t = i / C4, c4 = i - t * C4;
+        v4f kv = stg[i];
+        if constexpr (BIAS) kv += kvb[c4];
+        const Bf3x2 lo = split3x2(kv[0], kv[1]), hi = split3x2(kv[2], kv[3]);
+        __bf16 *at = kt + t * RK + 4 * c4;
+        *reinterpret_cast<u2 *>(at) = u2{lo.q0, hi.q0};
+        *reinterpret_cast<u2 *>(at + kKPlane) = u2{lo.q1, hi.q1};
+        *reinterpret_cast<u2 *>(at + 2 * kKPlane) = u2{lo.q2, hi.q2};
+      }
+      // 4 keys x 4 dims, first by the threads that have the least of K
+      for (int b = NT - 1 - tid; b < VB; b += NT) {
+        const int tq = b % 8, c4 = b / 8;
+        const int k0i = 8 * (tq % 4) + 4 * (tq / 4);  // the value product's k of key 4 tq
+        v4f x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if constexpr (VS)
+            x[u] = stg[SG + (4 * tq + u) * C4 + c4];
+          else
+            x[u] = *reinterpret_cast<const v4f *>(
+                rows.v + (size_t)min(t0 + 4 * tq + u, k_end) * rows.stride + 4 * c4);
+        }
+        if constexpr (BIAS)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u] += kvb[C4 + c4];
+        if (vexp != 0)  // workgroup-uniform
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[u][e] = ldexpf(x[u][e], -vexp);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const Bf3x2 lo = split3x2(x[0][e], x[1][e]), hi = split3x2(x[2][e], x[3][e]);
+          __bf16 *at = vt + (4 * c4 + e) * RV + k0i;
+          *reinterpret_cast<u2 *>(at) = u2{lo.q0, hi.q0};
+          *reinterpret_cast<u2 *>(at + kVPlane) = u2{lo.q1, hi.q1};
+          *reinterpret_cast<u2 *>(at + 2 * kVPlane) = u2{lo.q2, hi.q2};
+        }
+      }
+      lds_barrier();  // the planes are complete; the staging buffer is free
+      if (t0 + TK <= k_end) fetch(t0 + TK);
+
+      if (t0 > see.w_hi || t0 + TK - 1 < see.w_lo) continue;  // wave-uniform
+      // sc[b][r] = q(col) . k(t0 + 16 b + 4 grp + r)
+      v4f sc[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        sc[b] = v4f{0.f, 0.f, 0.f, 0.f};
+        if constexpr (kTail8) {
+          const __bf16 *at = kt + (16 * b + col) * RK + 32 * CF;
+          const bf8 a1 = *reinterpret_cast<const bf8 *>(at + tsel * kKPlane);
+          const bf8 a2 = *reinterpret_cast<const bf8 *>(at);
+          sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qt1, sc[b], 0, 0, 0);
+          sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, qt2, sc[b], 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < CF; ++c)
+          sc[b] = six(kt + (16 * b + col) * RK + 32 * c + 8 * grp, kKPlane, qa[0][c],
+                      qa[1][c], qa[2][c], sc[b]);
+      }
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        sc[b] *= asc;
+        if (cap != 0.0f)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[b][r] = tanhf(sc[b][r] / cap) * cap;
+      }
+      if (t0 < see.f_lo || t0 + TK - 1 > see.f_hi) {  // wave-uniform: some key masked
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = t0 + 16 * b + 4 * grp + r;
+            sc[b][r] = key <= see.p_top && key >= see.ws ? sc[b][r] : -FLT_MAX;
+          }
+      }
+      float top = -FLT_MAX;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) top = fmaxf(top, sc[b][r]);
+      const float top2 = top * c1;
+      if (__any(top2 > m + kSlack)) {
+        float rmax = fmaxf(top2, __shfl_xor(top2, 16, 64));
+        rmax = fmaxf(rmax, __shfl_xor(rmax, 32, 64));
+        const float m_new = fmaxf(m, ceilf(rmax));
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        l *= alpha;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) o[nb] *= alpha;
+      }
+      u4 w0, w1, w2;  // weight k = 4 b + r of the lane's eight is dword 2 b + r / 2
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          float p[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const float x = sc[b][r + u];
+            p[u] = x > -FLT_MAX ? __builtin_amdgcn_exp2f(fmaf(x, c1, fmaf(x, c2, -m))) : 0.0f;
+            l += p[u];
+          }
+          const Bf3x2 sp = split3x2(p[0], p[1]);
+          w0[2 * b + r / 2] = sp.q0;
+          w1[2 * b + r / 2] = sp.q1;
+          w2[2 * b + r / 2] = sp.q2;
+        }
+      const bf8 p0 = as_bf8(w0), p1 = as_bf8(w1), p2 = as_bf8(w2);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        o[nb] = six(vt + (16 * nb + col) * RV + 8 * grp, kVPlane, p0, p1, p2, o[nb]);
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+  }
+
+ private:
+  static constexpr float kSlack = 16.0f;  // weights stay below 2^16
+  static constexpr float kFloor = -0x1p100f;  // below any score
+  // acc + a b from the planes of a (at, at + plane, at + 2 plane) and b's pieces
+  static __device__ __forceinline__ v4f six(const __bf16 *at, int plane, bf8 b0, bf8 b1, bf8 b2,
+                                            v4f acc) {
+    const bf8 a0 = *reinterpret_cast<const bf8 *>(at);
+    const bf8 a1 = *reinterpret_cast<const bf8 *>(at + plane);
+    const bf8 a2 = *reinterpret_cast<const bf8 *>(at + 2 * plane);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b0, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b2, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc, 0, 0, 0);
+  }
+};
+
+// The power of two that AttnBf3 takes out of V, from what run() left in `red`:
+// 0 but for values so small that their third pieces would be subnormal.
+__device__ __forceinline__ int any_vexp(const v4f *red, int waves) {
+  float vtop = 0.0f;
+  for (int w = 0; w < waves; ++w) vtop = fmaxf(vtop, red[w][0]);
+  return __builtin_amdgcn_readfirstlane(vtop < 0x1p-60f ? -64 : 0);
+}
 
 __device__ __forceinline__ v4f ldexp4(v4f x, int e) {
 #pragma unroll

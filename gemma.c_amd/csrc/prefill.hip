@@ -619,11 +619,36 @@ __global__ __launch_bounds__(kNT, 2) void pf_attn_f32_kernel(PfAttn a) {
 constexpr int kPbWaves = 4;
 constexpr int kPbQ = kPbWaves * 32;  // query vectors per workgroup
 
+// Where a lane's query goes: the output row, or its chunk's partial.
+struct PfSplitOut {
+  float *row, *ml;  // ml: null with one chunk
+  __device__ __forceinline__ PfSplitOut(const PfAttn &a, const PaLane &L, int hd) {
+    float *part = reinterpret_cast<float *>(a.part);
+    const size_t at = (size_t)L.chunk_id * a.n + L.row;
+    const bool one = L.nchunks == 1;
+    row = (one ? a.xo + (size_t)L.row * a.q_sz : part + at * a.q_sz) + L.head * hd;
+    ml = one ? nullptr
+             : part + (size_t)kPfMaxSplit * a.n * a.q_sz + (at * a.n_heads + L.head) * 2;
+  }
+  // x times 2^e: value sums or outputs of dims d .. + 3
+  __device__ __forceinline__ void store(int d, v4f x, int e) const {
+    *reinterpret_cast<v4f *>(row + d) = ldexp4(x, e);
+  }
+  __device__ __forceinline__ void store_ml(float m, float l) const {
+    if (ml == nullptr) return;
+    ml[0] = m;
+    ml[1] = l;
+  }
+};
+
 template <int HD, bool CAP>
 __global__ __launch_bounds__(kPbWaves * 64, HD == 256 ? 1 : 2) void pf_attn_split_kernel(
-    PfAttn a, const int2 *exps, int tile0, int ntiles) {
+    PfAttn a, const TileRange *range, int tile0, int ntiles) {
   typedef AttnTile<HD> G;
-  __shared__ __attribute__((aligned(16))) char lds[2 * G::kBytes];
+  typedef AttnBf3<HD, kPbWaves, false, false> Any;
+  __shared__ __attribute__((aligned(16))) char
+      lds[2 * G::kBytes > Any::kBytes ? 2 * G::kBytes : Any::kBytes];
+  __shared__ v4f red[kPbWaves];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
@@ -637,25 +662,42 @@ __global__ __launch_bounds__(kPbWaves * 64, HD == 256 ? 1 : 2) void pf_attn_spli
   }
   see.f_lo = __builtin_amdgcn_readfirstlane(see.f_lo);
   see.f_hi = __builtin_amdgcn_readfirstlane(see.f_hi);
-  AttnWave<HD, kPbWaves, CAP> w;
-  const int eq = w.load_q(a.qkv + (size_t)L.row * a.stride + L.head * HD, nullptr, half);
-  float c_hi, c_lo;
-  log2_scale(a.asc, eq, &c_hi, &c_lo);
-  const size_t first = (size_t)L.hk * ntiles;
-  w.run(a.planes + first * G::kBytes - (size_t)tile0 * G::kBytes, exps + first - tile0,
-        L.k_lo / kPaKeys, L.k_end / kPaKeys, see, ldexpf(a.asc, eq), c_hi, c_lo, a.sc_att, lds,
-        wave, lane);
-  if (!L.valid) return;
-  float *pf = reinterpret_cast<float *>(a.part);
-  const size_t at = (size_t)L.chunk_id * a.n + L.row;
   const bool one = L.nchunks == 1;
-  float *prow = (one ? a.xo + (size_t)L.row * a.q_sz : pf + at * a.q_sz) + L.head * HD;
-  const float f = one ? 1.0f / w.l : 1.0f;
-  w.each(half, [&](int d, v4f x) { *reinterpret_cast<v4f *>(prow + d) = ldexp4(x * f, w.e_o); });
-  if (!one && half == 0) {
-    float *ml = pf + (size_t)kPfMaxSplit * a.n * a.q_sz + (at * a.n_heads + L.head) * 2;
-    ml[0] = w.m2;
-    ml[1] = w.l;
+  {
+    AttnWave<HD, kPbWaves, CAP> w;
+    const int eq = w.load_q(a.qkv + (size_t)L.row * a.stride + L.head * HD, nullptr, half);
+    float c_hi, c_lo;
+    log2_scale(a.asc, eq, &c_hi, &c_lo);
+    const size_t first = (size_t)L.hk * ntiles;
+    if (w.run(a.planes + first * G::kBytes - (size_t)tile0 * G::kBytes, range + first - tile0,
+              L.k_lo / kPaKeys, L.k_end / kPaKeys, see, ldexpf(a.asc, eq), c_hi, c_lo, a.sc_att,
+              lds, red, wave, lane)) {
+      if (!L.valid) return;
+      const PfSplitOut out(a, L, HD);
+      const float f = one ? 1.0f / w.l : 1.0f;
+      w.each(half, [&](int d, v4f x) { out.store(d, x * f, w.e_o); });
+      if (half == 0) out.store_ml(w.m2, w.l);
+      return;
+    }
+  }
+  // the keys and values as they stand: the wave's first 16 queries, then the others
+  const AttnRows rows{a.kc + (size_t)L.hk * a.clen * HD, a.vc + (size_t)L.hk * a.clen * HD,
+                      (size_t)HD, nullptr, nullptr};
+  const int vexp = any_vexp(red, kPbWaves);
+#pragma unroll 1
+  for (int g = 0; g < 2; ++g) {
+    const PaLane M = pa_lane<16>(a, 2 * wave + g, lane & 15);
+    Any w;
+    w.run(rows, M.k_lo, M.k_end, a.qkv + (size_t)M.row * a.stride + M.head * HD, nullptr,
+          AttnGroup{M.ws, M.p_top, INT_MAX, 0, M.w_lo, M.w_hi}, a.asc,
+          CAP ? a.sc_att : 0.0f, vexp, lds, wave, lane);
+    if (!M.valid) continue;
+    const PfSplitOut out(a, M, HD);
+    const int grp = lane >> 4;
+#pragma unroll
+    for (int nb = 0; nb < Any::NB; ++nb)
+      out.store(16 * nb + 4 * grp, one ? w.o[nb] / w.l : w.o[nb], vexp);
+    if (grp == 0) out.store_ml(w.m, w.l);
   }
 }
 
@@ -1198,14 +1240,15 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
     const int ntiles = (keys + kPaKeys - 1) / kPaKeys - tile0;
     auto go = [&](auto hd) {
       constexpr int HD = decltype(hd)::value;
-      int2 *exps = reinterpret_cast<int2 *>(a.planes + (size_t)a.nkv * ntiles * AttnTile<HD>::kBytes);
+      TileRange *range =
+          reinterpret_cast<TileRange *>(a.planes + (size_t)a.nkv * ntiles * AttnTile<HD>::kBytes);
       const AttnPack pk{a.kc, a.vc, (size_t)HD, (size_t)a.clen * HD, nullptr, nullptr,
-                        tile0, ntiles, keys, a.planes, exps};
+                        tile0, ntiles, keys, a.planes, range};
       attn_pack_kernel<HD><<<dim3(ntiles, a.nkv, 2), kPackThreads<HD>, 0, stream>>>(pk);
       if (a.sc_att != 0.0f)
-        pf_attn_split_kernel<HD, true><<<grid, kPbWaves * 64, 0, stream>>>(b, exps, tile0, ntiles);
+        pf_attn_split_kernel<HD, true><<<grid, kPbWaves * 64, 0, stream>>>(b, range, tile0, ntiles);
       else
-        pf_attn_split_kernel<HD, false><<<grid, kPbWaves * 64, 0, stream>>>(b, exps, tile0, ntiles);
+        pf_attn_split_kernel<HD, false><<<grid, kPbWaves * 64, 0, stream>>>(b, range, tile0, ntiles);
     };
     switch (hdim) {
       case 128: go(std::integral_constant<int, 128>{}); break;

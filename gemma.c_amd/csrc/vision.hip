@@ -630,280 +630,39 @@ hipError_t launch_vis_ln_rows(const VisLn &a, int n, hipStream_t stream) {
   return go(std::integral_constant<int, 256>{});
 }
 
-// The fp32 mode's attention without a workspace (calls under stream capture,
-// which can't allocate one), on the bf16 matrix cores: every fp32 operand x
-// of the two products (q, k, the probabilities p and v) is split into three
-// bf16 pieces x = x0 + x1 + x2 (each rounded to nearest from the remainder,
-// so together they hold x's 24 significant bits), and each product a.b is
-// summed from the six piece products whose orders add up to at most 2
-// (a0 b0, a0 b1, a1 b0, a0 b2, a1 b1, a2 b0): the dropped ones are below
-// 3 * 2^-24 |a b|, fp32 rounding.  bf16 x bf16 products are exact in the
-// fp32 accumulators.  v_mfma_f32_16x16x32_bf16 (lane l: A[l%16][8(l/16) ..
-// +7], B[8(l/16) .. +7][l%16], D[4(l/16) + r][l%16], checked on the GPU)
-// runs 14x the fp32 MFMA's rate here, so the six cost ~0.4 of one fp32 MFMA
-// step.  Geometry as vis_attn_f32_kernel: NW waves x 16 queries of one head,
-// 32-key tiles.  The next tile's fp32 K and V rows go by LDS DMA into a
-// staging buffer while the current tile's planes are in use; at a tile's
-// start the staged rows get their bias and are split into the planes (once
-// per workgroup, not per wave; with no prefetch registers the kernel fits
-// two workgroups per CU at head dim 72).  Scores per 16-key
-// block b: S[key 16b + 4g + r][query col] over 32-dim chunks of the head dim
-// (padded with zeros to CH * 32); K in LDS as three bf16 planes [key][dim].
-// Values: the PV product's k index is 8g + 4b + r, the key 16b + 4g + r,
-// so a lane's own eight probabilities are its B operand as they stand; V^T
-// is staged in LDS as three bf16 planes [dim][k] in that key order.
-// One LDS DMA load: every lane's 16 bytes at g land at lds + 16 * lane (lds
-// wave-uniform); from inline asm so that the compiler does not wait for the
-// pending load before later LDS reads (the kernel waits itself).  m0 has no
-// other user in the kernel that calls this.
-__device__ __forceinline__ void vis_dma16(const float *g, void *lds) {
-  const uint32_t m = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)lds;
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m), "v"(g)
-               : "memory", "m0");
-#pragma clang diagnostic pop
+// 16 queries of one head from q0 on by AttnBf3: K, V and the queries with their
+// biases, every key for every query.
+template <int HD, int NW, bool VS>
+__device__ __forceinline__ void vis_attn_any(const VisAttn &a, int h, int q0, int vexp, char *lds,
+                                             int wave, int lane) {
+  const int qr = q0 + (lane & 15), grp = lane >> 4;
+  const float *qrow = a.qkv + (size_t)min(qr, a.n - 1) * a.stride + h * HD;
+  const float *k = a.qkv + a.dim + h * HD, *bk = a.bias + a.dim + h * HD;
+  const AttnRows rows{k, k + a.dim, (size_t)a.stride, bk, bk + a.dim};
+  typedef AttnBf3<HD, NW, true, VS> Any;
+  Any w;
+  w.run(rows, 0, a.n - 1, qrow, a.bias + h * HD,
+        AttnGroup{0, a.n - 1, 0, a.n - 1, 0, a.n - 1}, a.scale, 0.0f, vexp, lds, wave, lane);
+  if (qr >= a.n) return;
+  float *orow = a.out + (size_t)qr * a.dim + h * HD + 4 * grp;
+#pragma unroll
+  for (int nb = 0; nb < Any::NB; ++nb)
+    if (16 * nb + 4 * grp < HD)
+      *reinterpret_cast<v4f *>(orow + 16 * nb) = ldexp4(w.o[nb] / w.l, vexp);
 }
 
+// The fp32 mode's attention without a workspace, by AttnBf3 alone: calls under
+// stream capture, which can't allocate one.
 template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64, 16 / NW) void vis_attn_bf3_kernel(VisAttn a) {
-  constexpr int TK = 32;              // keys per tile
-  constexpr int CH = (HD + 31) / 32;  // 32-dim chunks of the score product
-  constexpr int DP = CH * 32;         // padded head dim of the K planes
-  // A last chunk of 8 dims (head dim 72) takes two MFMAs instead of six: its
-  // k index carries four piece products over the 8 dims, k = 8 g + e for
-  // dim 32 CF + e of piece pair g (first MFMA: k2 q0, k1 q1, k0 q2, k1 q0;
-  // second: k0 q1, k0 q0 and two zero pairs)
-  constexpr bool kTail8 = HD % 32 == 8;
-  constexpr int CF = kTail8 ? CH - 1 : CH;  // chunks summed piece by piece
-  constexpr int NB = (HD + 15) / 16;  // 16-dim output blocks
-  constexpr int RK = DP + 8;          // K plane row (bf16): 16 rows in distinct banks
-  constexpr int RV = TK + 8;          // V^T plane row (bf16)
-  constexpr int NT = NW * 64, QB = NW * 16;
-  constexpr int C4 = HD / 4;
-  constexpr int PF = (TK * C4 + NT - 1) / NT;  // K float4 per thread
-  static_assert(HD % 8 == 0 && HD <= 128, "head dim");
-  // planes 16 bytes apart in the banks: the first tail MFMA reads three of
-  // them at one offset
-  __shared__ __attribute__((aligned(16))) __bf16 kt[3][TK * RK + 8];
-  __shared__ __attribute__((aligned(16))) __bf16 vt[3][NB * 16 * RV];
-  __shared__ v4f kvb[2][C4];
-  // the next tile's fp32 K and V rows land here by LDS DMA, key-major [key][C4]
-  constexpr int SG = TK * C4;
-  __shared__ v4f stg[2][SG];
-  static_assert(SG % 64 == 0, "whole DMA instructions per tile");
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nqb = (a.n + QB - 1) / QB, nblk = nqb * a.n_heads;
+  __shared__ __attribute__((aligned(16))) char lds[AttnBf3<HD, NW, true, true>::kBytes];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nqb = (a.n + NW * 16 - 1) / (NW * 16), nblk = nqb * a.n_heads;
   int blk = blockIdx.x;
   if (nblk % 8 == 0) blk = (blk % 8) * (nblk / 8) + blk / 8;
   const int h = blk / nqb;
-  const int q0 = (blk - h * nqb) * QB + wave * 16;
-  const int col = lane & 15, grp = lane >> 4;
-
-  // the query's pieces: lane (col, g) holds dims 32 c + 8 g .. + 7
-  bf8 qa[3][CH];
-  {
-    const int qr = min(q0 + col, a.n - 1);
-    const float *qrow = a.qkv + (size_t)qr * a.stride + h * HD;
-    const float *bq = a.bias + h * HD;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      u4 w0, w1, w2;
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const int d = 32 * c + 8 * grp + e;  // HD is even: d and d + 1 are both in or out
-        const float x0 = d < HD ? qrow[d] + bq[d] : 0.0f;
-        const float x1 = d < HD ? qrow[d + 1] + bq[d + 1] : 0.0f;
-        const Bf3x2 sp = split3x2(x0, x1);
-        w0[e / 2] = sp.q0;
-        w1[e / 2] = sp.q1;
-        w2[e / 2] = sp.q2;
-      }
-      qa[0][c] = as_bf8(w0);
-      qa[1][c] = as_bf8(w1);
-      qa[2][c] = as_bf8(w2);
-    }
-  }
-  // the tail chunk's operands: lane (col, 0) holds dims 32 CF .. + 7 of
-  // every piece in qa[p][CF]; lane (col, g) takes the piece of pair g
-  bf8 qt1 = {}, qt2 = {};
-  int tsel = 0;  // the K plane lane (col, g) reads in the first tail MFMA
-  if constexpr (kTail8) {
-    u4 t[3];
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const u4 v = __builtin_bit_cast(u4, qa[p][CF]);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) t[p][d] = (uint32_t)__shfl((int)v[d], col, 64);
-    }
-    qt1 = as_bf8(grp == 1 ? t[1] : grp == 2 ? t[2] : t[0]);          // q0 q1 q2 q0
-    qt2 = as_bf8(grp == 0 ? t[1] : grp == 1 ? t[0] : u4{0, 0, 0, 0});  // q1 q0 0 0
-    tsel = grp == 0 ? 2 : grp == 2 ? 0 : 1;                            // k2 k1 k0 k1
-  }
-  v4f o[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) o[nb] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m_ref = -FLT_MAX, l_part = 0.0f;
-  const float *bk = a.bias + a.dim + h * HD;
-  const float *bv = a.bias + 2 * a.dim + h * HD;
-  const float *kbase = a.qkv + a.dim + h * HD;
-  const float *vbase = a.qkv + 2 * a.dim + h * HD;
-
-  // zero padding: K dims HD .. DP-1 and V^T rows HD .. 16 NB - 1, never staged
-  const __bf16 bz = (__bf16)0.0f;
-  for (int i = tid; i < 3 * TK * (DP - HD); i += NT) {
-    const int p = i / (TK * (DP - HD)), j = i % (TK * (DP - HD));
-    kt[p][(j / (DP - HD)) * RK + HD + j % (DP - HD)] = bz;
-  }
-  for (int i = tid; i < 3 * (16 * NB - HD) * RV; i += NT) {
-    const int p = i / ((16 * NB - HD) * RV), j = i % ((16 * NB - HD) * RV);
-    vt[p][HD * RV + j] = bz;
-  }
-  for (int i = tid; i < 2 * C4; i += NT)
-    kvb[i / C4][i % C4] = reinterpret_cast<const v4f *>(i < C4 ? bk : bv)[i % C4];
-
-  static_assert(TK / 4 == 8, "V blocks: 8 key quads per tile");
-  constexpr int VB = 8 * C4;              // V blocks (4 keys x 4 dims) per tile
-  constexpr int PV = (VB + NT - 1) / NT;  // V blocks per thread
-  constexpr int NI = 2 * SG / 64;  // DMA instructions per tile (K, then V)
-  auto fetch = [&](int t0) {  // rows clamped into range: every load is unconditional
-    for (int i = wave; i < NI; i += NW) {  // wave-uniform
-      const int kv = i / (SG / 64), ch = (i % (SG / 64)) * 64 + lane;
-      const int t = ch / C4, c4 = ch - t * C4;
-      vis_dma16((kv == 0 ? kbase : vbase) + (size_t)min(t0 + t, a.n - 1) * a.stride + 4 * c4,
-                &stg[kv][(i % (SG / 64)) * 64]);
-    }
-  };
-  fetch(0);
-  for (int t0 = 0; t0 < a.n; t0 += TK) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's DMAs landed
-    lds_barrier();  // every wave is done with the previous tile (and every DMA landed)
-    const v4f zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < PF; ++j) {
-      const int i = tid + j * NT;
-      if (i >= TK * C4) break;
-      const int t = i / C4, c4 = i - t * C4;
-      const v4f kv = t0 + t < a.n ? stg[0][i] + kvb[0][c4] : zero;
-      const Bf3x2 lo = split3x2(kv[0], kv[1]), hi = split3x2(kv[2], kv[3]);
-      *reinterpret_cast<u2 *>(&kt[0][t * RK + 4 * c4]) = u2{lo.q0, hi.q0};
-      *reinterpret_cast<u2 *>(&kt[1][t * RK + 4 * c4]) = u2{lo.q1, hi.q1};
-      *reinterpret_cast<u2 *>(&kt[2][t * RK + 4 * c4]) = u2{lo.q2, hi.q2};
-    }
-#pragma unroll
-    for (int j = 0; j < PV; ++j) {
-      const int b = tid + j * NT;
-      if (b >= VB) break;
-      const int tq = b % 8, c4 = b / 8;
-      const int k0i = 8 * (tq % 4) + 4 * (tq / 4);  // PV index of key 4 tq
-      v4f r[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        r[u] = t0 + 4 * tq + u < a.n ? stg[1][(4 * tq + u) * C4 + c4] + kvb[1][c4] : zero;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const Bf3x2 lo = split3x2(r[0][e], r[1][e]), hi = split3x2(r[2][e], r[3][e]);
-        const int at = (4 * c4 + e) * RV + k0i;
-        *reinterpret_cast<u2 *>(&vt[0][at]) = u2{lo.q0, hi.q0};
-        *reinterpret_cast<u2 *>(&vt[1][at]) = u2{lo.q1, hi.q1};
-        *reinterpret_cast<u2 *>(&vt[2][at]) = u2{lo.q2, hi.q2};
-      }
-    }
-    lds_barrier();
-    if (t0 + TK < a.n) fetch(t0 + TK);
-
-    // scores: sc[b][r] = q(col) . k(t0 + 16 b + 4 grp + r), the small piece
-    // products first
-    v4f sc[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      sc[b] = v4f{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kTail8) {
-        const int at = (16 * b + col) * RK + 32 * CF;
-        const bf8 a1 = *reinterpret_cast<const bf8 *>(&kt[tsel][at]);
-        const bf8 a2 = *reinterpret_cast<const bf8 *>(&kt[0][at]);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qt1, sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, qt2, sc[b], 0, 0, 0);
-      }
-#pragma unroll
-      for (int c = 0; c < CF; ++c) {
-        const int at = (16 * b + col) * RK + 32 * c + 8 * grp;
-        const bf8 k0 = *reinterpret_cast<const bf8 *>(&kt[0][at]);
-        const bf8 k1 = *reinterpret_cast<const bf8 *>(&kt[1][at]);
-        const bf8 k2 = *reinterpret_cast<const bf8 *>(&kt[2][at]);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, qa[0][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qa[1][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[2][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qa[0][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[1][c], sc[b], 0, 0, 0);
-        sc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qa[0][c], sc[b], 0, 0, 0);
-      }
-    }
-    float tmax = -FLT_MAX;
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool ok = t0 + 16 * b + 4 * grp + r < a.n;
-        sc[b][r] = ok ? sc[b][r] * a.scale : -FLT_MAX;
-        tmax = fmaxf(tmax, sc[b][r]);
-      }
-    if (__any(tmax > m_ref + kVaSlackF)) {
-      float rmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-      rmax = fmaxf(rmax, __shfl_xor(rmax, 32, 64));
-      const float m_new = fmaxf(m_ref, rmax);
-      const float alpha = __expf(m_ref - m_new);
-      m_ref = m_new;
-      l_part *= alpha;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) o[nb] *= alpha;
-    }
-    // probabilities, their pieces (k = 4 b + r of this lane's eight)
-    u4 w0, w1, w2;  // weight k = 4 b + r of the lane's eight is dword 2 b + r / 2
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const float pa = sc[b][r] > -FLT_MAX ? __expf(sc[b][r] - m_ref) : 0.0f;
-        const float pb = sc[b][r + 1] > -FLT_MAX ? __expf(sc[b][r + 1] - m_ref) : 0.0f;
-        l_part += pa;
-        l_part += pb;
-        const Bf3x2 sp = split3x2(pa, pb);
-        w0[2 * b + r / 2] = sp.q0;
-        w1[2 * b + r / 2] = sp.q1;
-        w2[2 * b + r / 2] = sp.q2;
-      }
-    const bf8 p0 = as_bf8(w0), p1 = as_bf8(w1), p2 = as_bf8(w2);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int at = (16 * nb + col) * RV + 8 * grp;
-      const bf8 v0 = *reinterpret_cast<const bf8 *>(&vt[0][at]);
-      const bf8 v1 = *reinterpret_cast<const bf8 *>(&vt[1][at]);
-      const bf8 v2 = *reinterpret_cast<const bf8 *>(&vt[2][at]);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v2, p0, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, p1, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p2, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v1, p0, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p1, o[nb], 0, 0, 0);
-      o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v0, p0, o[nb], 0, 0, 0);
-    }
-  }
-  float l = l_part + __shfl_xor(l_part, 16, 64);
-  l = l + __shfl_xor(l, 32, 64);
-  const int qr = q0 + col;
-  if (qr < a.n) {
-    float *orow = a.out + (size_t)qr * a.dim + h * HD;
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = 16 * nb + 4 * grp + r;
-        if (d < HD) orow[d] = o[nb][r] / l;
-      }
-  }
+  vis_attn_any<HD, NW, true>(a, h, (blk - h * nqb) * NW * 16 + wave * 16, 0, lds, wave, lane);
 }
 
 // The fp32 mode's attention on the f16 matrix cores in split precision
@@ -918,10 +677,15 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void vis_attn_bf3_kernel(VisAttn 
 // fp32 roundings per sum).  The tower's image (9 of 27 layers): 6.73 -> 4.7 ms.
 template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, const char *planes,
-                                                                   const int2 *exps, int ntiles) {
+                                                                   const TileRange *range,
+                                                                   int ntiles) {
   typedef AttnTile<HD> G;
+  constexpr bool kVs = HD <= 72;
+  typedef AttnBf3<HD, NW, true, kVs> Any;
   constexpr int QB = NW * 32;
-  __shared__ __attribute__((aligned(16))) char lds[2 * G::kBytes];
+  __shared__ __attribute__((aligned(16))) char
+      lds[2 * G::kBytes > Any::kBytes ? 2 * G::kBytes : Any::kBytes];
+  __shared__ v4f red[NW];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
@@ -930,15 +694,21 @@ __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, c
   int blk = blockIdx.x;
   if (nblk % 8 == 0) blk = (blk % 8) * (nblk / 8) + blk / 8;
   const int h = blk / nqb;
-  const int qr = (blk - h * nqb) * QB + wave * 32 + (lane & 31);
+  const int q0 = (blk - h * nqb) * QB + wave * 32, qr = q0 + (lane & 31);
   AttnWave<HD, NW> w;
   const int eq = w.load_q(a.qkv + (size_t)min(qr, a.n - 1) * a.stride + h * HD, a.bias + h * HD,
                           half);
   float c_hi, c_lo;
   log2_scale(a.scale, eq, &c_hi, &c_lo);
   const AttnSee see{0, a.n - 1, 0, a.n - 1};
-  w.run(planes + (size_t)h * ntiles * G::kBytes, exps + (size_t)h * ntiles, 0, ntiles - 1, see,
-        0.0f, c_hi, c_lo, 0.0f, lds, wave, lane);
+  if (!w.run(planes + (size_t)h * ntiles * G::kBytes, range + (size_t)h * ntiles, 0, ntiles - 1,
+             see, 0.0f, c_hi, c_lo, 0.0f, lds, red, wave, lane)) {
+    const int vexp = any_vexp(red, NW);
+#pragma unroll 1
+    for (int g = 0; g < 32; g += 16)
+      vis_attn_any<HD, NW, kVs>(a, h, q0 + g, vexp, lds, wave, lane);
+    return;
+  }
   if (qr >= a.n) return;
   float *orow = a.out + (size_t)qr * a.dim + h * HD;
   const float f = 1.0f / w.l;
@@ -948,19 +718,20 @@ __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, c
 template <int HD>
 void launch_vis_split(const VisAttn &a, char *planes, const DeviceInfo &dev, hipStream_t stream) {
   const int ntiles = (a.n + 31) / 32;
-  int2 *exps = reinterpret_cast<int2 *>(planes + (size_t)a.n_heads * ntiles * AttnTile<HD>::kBytes);
+  TileRange *range =
+      reinterpret_cast<TileRange *>(planes + (size_t)a.n_heads * ntiles * AttnTile<HD>::kBytes);
   const AttnPack pk{a.qkv + a.dim, a.qkv + 2 * a.dim, (size_t)a.stride, (size_t)HD,
-                    a.bias + a.dim, a.bias + 2 * a.dim, 0, ntiles, a.n, planes, exps};
+                    a.bias + a.dim, a.bias + 2 * a.dim, 0, ntiles, a.n, planes, range};
   attn_pack_kernel<HD><<<dim3(ntiles, a.n_heads, 2), kPackThreads<HD>, 0, stream>>>(pk);
   // 128 queries a workgroup while those have a CU each (784 patches, 16 heads:
   // 39 us against 50 with 256; 2401 patches, 12 heads: 77 against 103), else
   // 256, which share each tile's way to LDS (4096 patches: 243 against 250)
   const int few = (a.n + 127) / 128 * a.n_heads;
   if (few <= dev.cus)
-    vis_attn_split_kernel<HD, 4><<<few, 256, 0, stream>>>(a, planes, exps, ntiles);
+    vis_attn_split_kernel<HD, 4><<<few, 256, 0, stream>>>(a, planes, range, ntiles);
   else
-    vis_attn_split_kernel<HD, 8><<<(a.n + 255) / 256 * a.n_heads, 512, 0, stream>>>(a, planes, exps,
-                                                                                   ntiles);
+    vis_attn_split_kernel<HD, 8><<<(a.n + 255) / 256 * a.n_heads, 512, 0, stream>>>(a, planes,
+                                                                                   range, ntiles);
 }
 
 // The fp32 mode's kernel: a split one by default (f16 pieces with a workspace,
@@ -982,7 +753,7 @@ size_t attn_planes_bytes(int hdim, int heads, int keys) {
     case 128: tile = AttnTile<128>::kBytes; break;
     case 256: tile = AttnTile<256>::kBytes; break;
   }
-  return tiles * (tile + sizeof(int2));
+  return tiles * (tile + sizeof(TileRange));
 }
 
 hipError_t launch_vis_attention(const VisAttn &a, int hdim, bool f32, char *planes,

@@ -114,6 +114,43 @@ def test_vision_small_tiles_keep_their_precision(gh):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hd", [16, 32, 64, 72, 128])
+@pytest.mark.parametrize("exps", [(55, 0, -55), (None, -62, -62), (-62, None, -62), (0, None, 0),
+                                  (30, 60, 90), (100, 50, 0, -50, -100), (-9, 0, 0)],
+                         ids=lambda e: "v2^" + "_".join(map(str, e)))
+def test_vision_value_tiles_far_apart(gh, exps, hd):
+    """Tiles of V that fall or rise time and again, and tiles of zeros (None):
+    every query's output is that of all of them."""
+    rng = np.random.default_rng(hd)
+    n, heads = 32 * len(exps) + 5, 2
+    dim = heads * hd
+    qkv = rng.standard_normal((n, 3 * dim))
+    e = np.array([-np.inf if x is None else x for x in exps])[(np.arange(n) // 32) % len(exps)]
+    qkv[:, 2 * dim:] *= np.exp2(e)[:, None]
+    qkv = qkv.astype(np.float32)
+    bias = np.zeros(3 * dim, np.float32)
+    _close(_vision(gh, qkv, bias, heads, dim), _vision_want(qkv, bias, heads, dim))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [0, 128, 288])
+@pytest.mark.parametrize("exp", [70, 110])
+def test_vision_huge_tile_of_no_weight(gh, exp, first):
+    """A tile of V further above the rest than any running unit could follow,
+    whose weights are zero: the others' values stay whole."""
+    rng = np.random.default_rng(exp + first)
+    n, hd = 320, 72
+    q, k, v = (rng.standard_normal((n, hd)) for _ in range(3))
+    q[:, 0] = 40.0  # the huge tile's keys score -40 * 40 / sqrt(72) below the rest: e^-188
+    k[:, 0] = 0.0
+    k[first:first + 32, 0] = -40.0
+    v[first:first + 32] *= 2.0 ** exp
+    qkv = np.concatenate([q, k, v], axis=1).astype(np.float32)
+    bias = np.zeros(3 * hd, np.float32)
+    _close(_vision(gh, qkv, bias, 1, hd), _vision_want(qkv, bias, 1, hd))
+
+
+@pytest.mark.gpu
 def test_vision_zero_and_peaked(gh):
     """All-zero q, k or v tiles, and scores so far apart that one key takes
     all the weight (the reference maximum moves with nearly every tile)."""
@@ -219,8 +256,7 @@ def test_prefill_tile_edges(gh, monkeypatch, n, pos0, nh, nkv, hd, slide, cap, d
 @pytest.mark.parametrize("hd", [128, 256])
 def test_prefill_tiles_of_any_magnitude(gh, monkeypatch, hd):
     """Tiles of V at magnitudes far apart, a window that hides the largest
-    from some rows (held to their own largest output), masked keys with
-    infinities in their rows' place in the window."""
+    from some rows (held to their own largest output)."""
     monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
     n, pos0, nh, nkv, slide = 150, 200, 4, 2, 90
     q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=3)
@@ -232,6 +268,30 @@ def test_prefill_tiles_of_any_magnitude(gh, monkeypatch, hd):
     got, want = _prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args)
     for i in range(n):
         _close(got[i], want[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["v2^70", "v2^110", "vinf", "vnan", "kinf"])
+@pytest.mark.parametrize("hd", [128, 256])
+def test_prefill_unseen_tiles(gh, monkeypatch, hd, what):
+    """Rows 0 .. 95 of a causal pass, 16 to a wave, against keys 96 .. 127 that
+    none of them sees but that their workgroup walks: huge, infinite or no
+    numbers, they leave those rows what they are; and the same of the first 32
+    keys for rows 64 .. 127 behind a 16-key window."""
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
+    n, nh, nkv = 128, 2, 2
+    for slide, hidden, rows in ((0, slice(96, 128), slice(0, 96)),
+                                (16, slice(0, 32), slice(64, 128))):
+        q, kc, vc = _prefill_inputs(n, 0, nh, nkv, hd, seed=hd)
+        to = kc if what[0] == "k" else vc
+        if what[1:] in ("inf", "nan"):
+            to[:, hidden] = np.float32(what[1:])
+        else:
+            to[:, hidden] *= np.float32(2.0 ** int(what[3:]))
+        got = _prefill(gh, q, kc, vc, n, 0, nh, nkv, hd, slide, 0.0, False)
+        kc[:, hidden] = vc[:, hidden] = 0  # nothing of them reaches those rows
+        want = _prefill_want(q, kc, vc, n, 0, nh, nkv, hd, slide, 0.0, False)
+        _close(got[rows], want[rows])
 
 
 @pytest.mark.gpu
