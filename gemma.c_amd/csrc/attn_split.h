@@ -16,10 +16,19 @@
 // V's into the weights: the value sums are kept in units of the largest V tile
 // of the workgroup's keys.
 //
-// Two f16 pieces hold a value's 22 bits only near its tile's largest, so a
-// workgroup first looks at what its tiles hold (TileRange: finite, V's tiles
-// within 2^8 of each other, kept by attn_pack_kernel) and otherwise computes
-// its queries by AttnBf3: three bf16 pieces and six products, at any magnitude.
+// Two f16 pieces hold a value's 22 bits only down to 2^-17 of its tile's
+// largest, and a weight's down to 2^-8 of its query's largest.  So a workgroup
+// first looks at what its tiles hold (TileRange, kept by attn_pack_kernel) and
+// computes its queries by AttnBf3, three bf16 pieces and six products at any
+// magnitude, unless all of this holds:
+//  - K and V are finite.
+//  - Every key's largest V, and every dim's in every tile (of kThin keys or
+//    more) but for dims of zeros, is within 2^6 of the largest V of all.  A
+//    weight's pieces drop at most 2^-31 of the query's largest weight, in units
+//    of the largest V (about 2^-26 rms over 4096 keys): 2^-20 of the least such
+//    key or dim, of ordinary ones far less.
+//  - HD 2^-9 of a raw score's unit, the most that q's and k's pieces drop from a
+//    score by ending at 2^-25, is below 2^-19 octaves.
 //
 // K and V are split once per key and layer by attn_pack_kernel into tiles of
 // 32 keys whose pieces lie in the order in which a wave reads its operands:
@@ -81,17 +90,41 @@ __device__ __forceinline__ void split8(const float (&x)[8], h8 *hi, h8 *lo) {
     (*lo)[e + 1] = b[1];
   }
 }
-// Magnitude; infinite for what isn't finite.
-__device__ __forceinline__ float abs_or_inf(float x) {
-  const float a = fabsf(x);
-  return a <= FLT_MAX ? a : INFINITY;
+// The bits of |x|, which order as the magnitudes do, what isn't finite above all.
+__device__ __forceinline__ int abs_bits(float x) { return __float_as_int(x) & 0x7fffffff; }
+constexpr int kInfBits = 0x7f800000;
+template <int CTRL>
+__device__ __forceinline__ int dpp_i32(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
 }
-// E such that amax 2^-E lies in [2^14, 2^15), f16's upper range; 0 for 0.
+// Max over the 64 lanes of a wave.
+__device__ __forceinline__ int wave_max_i32(int v) {
+  v = max(v, dpp_i32<kDppXor1>(v));
+  v = max(v, dpp_i32<kDppXor2>(v));
+  v = max(v, dpp_i32<kDppHalfMirror>(v));
+  v = max(v, dpp_i32<kDppMirror>(v));
+  return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+// Lane l's result: the largest t[l % 8] of its eight lanes.  Each step hands
+// half of a lane's values to a lane that keeps that half.
+__device__ __forceinline__ int max_across_8(const int (&t)[8], int lane) {
+  int a[4], b[2];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    a[e] = max(lane & 4 ? t[4 + e] : t[e], dpp_i32<kDppHalfMirror>(lane & 4 ? t[e] : t[4 + e]));
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    b[e] = max(lane & 2 ? a[2 + e] : a[e], dpp_i32<kDppXor2>(lane & 2 ? a[e] : a[2 + e]));
+  return max(lane & 1 ? b[1] : b[0], dpp_i32<kDppXor1>(lane & 1 ? b[0] : b[1]));
+}
+// E such that amax 2^-E lies in [2^14, 2^15), f16's upper range; for 0 one that
+// is below any other's.
 __device__ __forceinline__ int scale_exp(float amax) {
-  return amax > 0.0f ? ilogbf(amax) - 14 : 0;
+  return amax > 0.0f ? ilogbf(amax) - 14 : -200;
 }
-// ... rounded up to a multiple of 4: the V tiles of ordinary layers then
-// share one exponent and the running one rarely moves.
+// ... rounded up to a multiple of 4, which most V tiles of ordinary layers
+// share; 0 for 0.
 __device__ __forceinline__ int scale_exp4(float amax) {
   return amax > 0.0f ? (scale_exp(amax) + 3 + 1024) / 4 * 4 - 1024 : 0;
 }
@@ -102,7 +135,10 @@ struct TileRange {
   float vtop;   // V's largest magnitude; infinite: V is not finite
   float vlow;   // f16 pieces keep this tile's V beside others of up to this magnitude
 };
-constexpr float kVReach = 0x1p8f;  // how far V's magnitudes may lie apart
+constexpr float kVReach = 0x1p6f;  // how far V's keys and dims may lie apart
+// Tiles of fewer keys don't speak for their dims: by chance alone one of a few
+// values lies far below the rest (ordinary rows of one key: one dim in 70).
+constexpr int kThin = 8;
 
 // Two workgroups per (32-key tile, kv head), K and V: rows 32 t .. 32 t + 31
 // (rows from `keys` on are zero) with their biases, scaled and split into the
@@ -129,9 +165,15 @@ __global__ __launch_bounds__(kPackThreads<HD>) void attn_pack_kernel(AttnPack a)
   constexpr int NT = kPackThreads<HD>;
   constexpr int N = 4 * HD;                // items of the tile: 32 HD / 8
   constexpr int PT = (N + NT - 1) / NT;    // per thread
-  __shared__ float red[NT / 64];
+  __shared__ int red[NT / 64];             // K's largest magnitude, as bits
+  __shared__ int keytop[32], dimtop[HD];  // V's, of each key and dim
   const int tid = threadIdx.x, h = blockIdx.y;
   const bool isv = blockIdx.z != 0;
+  if (isv) {
+    if (tid < 32) keytop[tid] = 0;
+    for (int i = tid; i < HD; i += NT) dimtop[i] = 0;
+    __syncthreads();
+  }
   const int t0 = (a.tile0 + blockIdx.x) * 32;
   const float *src = (isv ? a.v : a.k) + h * a.hstride;
   const float *bias = isv ? a.bv : a.bk;
@@ -166,29 +208,36 @@ __global__ __launch_bounds__(kPackThreads<HD>) void attn_pack_kernel(AttnPack a)
       }
     }
   }
-  float amax = 0.0f;
+  int top = 0;
+  if (!isv) {
 #pragma unroll
-  for (int j = 0; j < PT; ++j)
+    for (int j = 0; j < PT; ++j)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, abs_or_inf(x[j][e]));
-  amax = wave_max_dpp(amax);
-  if ((tid & 63) == 0) red[tid >> 6] = amax;
-  __syncthreads();
+      for (int e = 0; e < 8; ++e) top = max(top, abs_bits(x[j][e]));
+    top = wave_max_i32(top);
+    if ((tid & 63) == 0) red[tid >> 6] = top;
+    __syncthreads();
 #pragma unroll
-  for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
-  const bool finite = amax <= FLT_MAX;  // if not, the pieces are of no use
-  const int ex = !finite ? 0 : isv ? scale_exp4(amax) : scale_exp(amax);
-  const size_t at = (size_t)h * a.ntiles + blockIdx.x;
-  if (tid == 0) {
-    TileRange *r = a.range + at;
-    if (isv) {
-      r->ev = ex;
-      r->vtop = amax;
-      r->vlow = amax * kVReach;
-    } else {
-      r->ek = finite ? ex : INT_MAX;
+    for (int w = 0; w < NT / 64; ++w) top = max(top, red[w]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+      const int i = min(tid + j * NT, N - 1), d = i % HD, q = i / HD, s = q >> 1, half = q & 1;
+      int t[8], most = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) most = max(most, t[e] = abs_bits(x[j][e]));
+      // eight lanes hold eight dims of the same keys (HD % 8 == 0)
+      const int e = tid % 8;
+      atomicMax(&keytop[8 * (2 * s + e / 4) + 4 * half + e % 4], max_across_8(t, tid));
+      atomicMax(&dimtop[d], most);
     }
+    __syncthreads();
+    top = wave_max_i32(keytop[tid % 32]);
   }
+  const bool finite = top < kInfBits;  // if not, the pieces are of no use
+  const float amax = finite ? __int_as_float(top) : 0.0f;
+  const int ex = isv ? scale_exp4(amax) : scale_exp(amax);
+  const size_t at = (size_t)h * a.ntiles + blockIdx.x;
   char *kf = a.planes + at * G::kBytes, *vf = kf + G::KFR * 1024;
 #pragma unroll
   for (int j = 0; j < PT; ++j) {
@@ -225,6 +274,24 @@ __global__ __launch_bounds__(kPackThreads<HD>) void attn_pack_kernel(AttnPack a)
       const int f = i / 32, half = (i / 16) % 2, r = 16 + i % 16;
       *reinterpret_cast<h8 *>(vf + f * 1024 + (32 * half + r) * 16) = zero;
     }
+  if (tid >= 64) return;
+  TileRange *r = a.range + at;
+  if (!isv) {
+    if (tid == 0) r->ek = finite ? ex : INT_MAX;
+    return;
+  }
+  const int keys = min(32, a.keys - t0);
+  int low = INT_MAX;
+  if (tid < keys) low = keytop[tid];
+  if (keys >= kThin)
+    for (int d = tid; d < HD; d += 64)
+      if (dimtop[d] != 0) low = min(low, dimtop[d]);
+  low = -wave_max_i32(-low);
+  if (tid == 0) {
+    r->ev = ex;
+    r->vtop = finite ? amax : INFINITY;
+    r->vlow = __int_as_float(low) * kVReach;
+  }
 }
 
 // One LDS DMA load: lane l's 16 bytes at base + 16 l land at lds + 16 l (base
@@ -404,11 +471,12 @@ struct AttnWave {
 
   // lds: 2 K tiles, then 2 V tiles; red: a v4f per wave.  c_hi + c_lo: the
   // scores' scale (asc) times log2 e, without the tiles' exponents; cap: the
-  // soft cap of the scaled scores (0: none).  False, for the whole workgroup
-  // and with nothing computed, where the tiles hold what two f16 pieces don't.
+  // soft cap of the scaled scores (0: none); keys: how many there are.  False,
+  // for the whole workgroup and with nothing computed, where the tiles hold
+  // what two f16 pieces don't.
   __device__ __forceinline__ bool run(const char *tiles, const TileRange *range, int ta, int tb,
-                                      const AttnSee &see, float asc, float c_hi, float c_lo,
-                                      float cap, char *lds, v4f *red, int wave, int lane) {
+                                      int keys, const AttnSee &see, float asc, float c_hi,
+                                      float c_lo, float cap, char *lds, v4f *red, int wave, int lane) {
     const int half = lane >> 5;
     char *kbuf = lds, *vbuf = lds + 2 * G::KFR * 1024;
     const uint32_t loff = lane * 16;
@@ -442,26 +510,26 @@ struct AttnWave {
     int2 ex = exps(ta + zero);
     fetch_k(ta);
     fetch_v(ta);
-    float vtop = 0.0f, vlow = FLT_MAX;
-    bool finite = true;
+    float vtop = 0.0f, vlow = FLT_MAX, ek = -1e9f;
     for (int t = ta + 64 * wave + lane; t <= tb; t += 64 * NW) {
       const TileRange r = range[t];
       vtop = fmaxf(vtop, r.vtop);
       vlow = fminf(vlow, r.vlow);
-      finite = finite && r.ek != INT_MAX;
+      ek = fmaxf(ek, (float)r.ek);
     }
-    red[wave] = v4f{wave_max_dpp(vtop), -wave_max_dpp(-vlow), __all(finite) ? 0.0f : 1.0f, 0.0f};
+    red[wave] = v4f{wave_max_dpp(vtop), -wave_max_dpp(-vlow), wave_max_dpp(ek), wave_max_dpp(c_hi)};
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's DMAs landed
     lds_barrier();                       // every wave's did
-    vtop = red[0][0], vlow = red[0][1];
-    float bad = red[0][2];
+    v4f all = red[0];
 #pragma unroll
     for (int w = 1; w < NW; ++w) {
-      vtop = fmaxf(vtop, red[w][0]);
-      vlow = fminf(vlow, red[w][1]);
-      bad += red[w][2];
+      const v4f r = red[w];
+      all = v4f{fmaxf(all[0], r[0]), fminf(all[1], r[1]), fmaxf(all[2], r[2]), fmaxf(all[3], r[3])};
     }
-    const bool fit = bad == 0.0f && vtop <= kAttnVTop && vlow >= vtop;
+    vtop = all[0];
+    const bool fit = vtop <= kAttnVTop && all[1] >= vtop && all[2] < 1e6f &&
+                     ldexpf(all[3], (int)all[2]) <= 0x1p-10f / HD &&
+                     (tb > ta || keys - 32 * ta >= kThin);
     if (!__builtin_amdgcn_readfirstlane((int)fit)) return false;
     e_o = __builtin_amdgcn_readfirstlane(scale_exp4(vtop));  // the largest tile's exponent
     if (ta < tb) fetch_k(ta + 1);

@@ -670,8 +670,8 @@ __global__ __launch_bounds__(kPbWaves * 64, HD == 256 ? 1 : 2) void pf_attn_spli
     log2_scale(a.asc, eq, &c_hi, &c_lo);
     const size_t first = (size_t)L.hk * ntiles;
     if (w.run(a.planes + first * G::kBytes - (size_t)tile0 * G::kBytes, range + first - tile0,
-              L.k_lo / kPaKeys, L.k_end / kPaKeys, see, ldexpf(a.asc, eq), c_hi, c_lo, a.sc_att,
-              lds, red, wave, lane)) {
+              L.k_lo / kPaKeys, L.k_end / kPaKeys, a.pos0 + a.n, see, ldexpf(a.asc, eq), c_hi,
+              c_lo, a.sc_att, lds, red, wave, lane)) {
       if (!L.valid) return;
       const PfSplitOut out(a, L, HD);
       const float f = one ? 1.0f / w.l : 1.0f;

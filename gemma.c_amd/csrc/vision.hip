@@ -702,7 +702,7 @@ __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, c
   log2_scale(a.scale, eq, &c_hi, &c_lo);
   const AttnSee see{0, a.n - 1, 0, a.n - 1};
   if (!w.run(planes + (size_t)h * ntiles * G::kBytes, range + (size_t)h * ntiles, 0, ntiles - 1,
-             see, 0.0f, c_hi, c_lo, 0.0f, lds, red, wave, lane)) {
+             a.n, see, 0.0f, c_hi, c_lo, 0.0f, lds, red, wave, lane)) {
     const int vexp = any_vexp(red, NW);
 #pragma unroll 1
     for (int g = 0; g < 32; g += 16)

@@ -132,6 +132,94 @@ def test_vision_value_tiles_far_apart(gh, exps, hd):
     _close(_vision(gh, qkv, bias, heads, dim), _vision_want(qkv, bias, heads, dim))
 
 
+def _close_each(got, want, axis, tol=TOL):
+    """Every row (axis 1) or column (axis 0) held to its own largest value: TOL is
+    that of the weights, which all of a row's or a column's outputs share."""
+    rel = float((np.abs(got - want).max(axis=axis) / np.abs(want).max(axis=axis)).max())
+    print(f"largest |d|/max of one = {rel:.3g}", flush=True)
+    assert rel <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,exp", [(96, -6), (96, -10), (300, -18), (96, -24), (33, -24),
+                                   (5, -24), (96, -60)])
+@pytest.mark.parametrize("hd", [64, 72])
+def test_vision_small_dims(gh, n, exp, hd):
+    """Dims of V far below the rest of their tiles keep their own precision."""
+    rng = np.random.default_rng(n - exp)
+    qkv = rng.standard_normal((n, 3 * hd))
+    small = [2 * hd + 5, 3 * hd - 1]
+    qkv[:, small] *= 2.0 ** exp
+    qkv = qkv.astype(np.float32)
+    bias = np.zeros(3 * hd, np.float32)
+    _close_each(_vision(gh, qkv, bias, 1, hd), _vision_want(qkv, bias, 1, hd), 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exp", [-4, -12, -20, -40, None])
+@pytest.mark.parametrize("hd", [16, 72, 128])
+def test_vision_small_keys(gh, exp, hd):
+    """Queries whose weight is all but wholly on keys with values far below the
+    others', which are in their tile, or zero: the others' share of them, about
+    e^-14, is as precise as the rest."""
+    rng = np.random.default_rng(hd)
+    n = 200
+    q, k, v = (rng.standard_normal((n, hd)) for _ in range(3))
+    q *= 0.3
+    k *= 0.3
+    q[:, 0] = 2.0
+    k[:, 0] = 0.0
+    k[[3, 77, 78, 150], 0] = 7.0 * np.sqrt(hd)
+    v[[3, 77, 78, 150]] *= 0.0 if exp is None else 2.0 ** exp
+    qkv = np.concatenate([q, k, v], axis=1).astype(np.float32)
+    bias = np.zeros(3 * hd, np.float32)
+    _close_each(_vision(gh, qkv, bias, 1, hd), _vision_want(qkv, bias, 1, hd), 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exp", [4, 12, 20, 40])
+def test_vision_query_outliers(gh, exp):
+    """A dim of the queries far above the others, met by zeros in the keys, and
+    one of the keys met by zeros in the queries: scores come from the others."""
+    rng = np.random.default_rng(exp)
+    n, hd = 160, 72
+    qkv = rng.standard_normal((n, 3 * hd))
+    qkv[:, 7] *= 2.0 ** exp
+    qkv[:, hd + 7] = 0
+    qkv[:, 9] = 0
+    qkv[:, hd + 9] *= 2.0 ** exp
+    qkv = qkv.astype(np.float32)
+    bias = np.zeros(3 * hd, np.float32)
+    _close_each(_vision(gh, qkv, bias, 1, hd), _vision_want(qkv, bias, 1, hd), 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["dims", "keys", "outlier"])
+@pytest.mark.parametrize("hd,n,pos0,slide", [(256, 150, 90, 0), (128, 260, 0, 100)])
+def test_prefill_small_values(gh, monkeypatch, what, hd, n, pos0, slide):
+    """The same of the prompt pass, whole and in chunks of its keys."""
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
+    nh, nkv = 4, 2
+    q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=hd)
+    ctx = pos0 + n
+    q *= np.float32(0.5)
+    if what == "dims":
+        vc[:, :ctx, [5, hd - 1]] *= np.float32(2.0 ** -24)
+    elif what == "keys":
+        kc[:, :ctx, 0] = 0
+        q[:, 0:nh * hd:hd] = 2
+        kc[:, 3:ctx:40, 0] = 7.0 * np.sqrt(hd)
+        vc[:, 3:ctx:40] *= np.float32(2.0 ** -16)
+    else:
+        q[:, 1:nh * hd:hd] *= np.float32(2.0 ** 20)
+        kc[:, :ctx, 1] = 0
+    args = (n, pos0, nh, nkv, hd, slide, 0.0, False)
+    got, want = _prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args)
+    for h in range(nh):
+        c = slice(h * hd, (h + 1) * hd)
+        _close_each(got[:, c], want[:, c], 0 if what == "dims" else 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("first", [0, 128, 288])
 @pytest.mark.parametrize("exp", [70, 110])
