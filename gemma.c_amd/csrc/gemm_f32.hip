@@ -128,19 +128,30 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(
 // scaled f16 pieces per operand, three products (v_mfma_f32_16x16x32_f16) with
 // fp32 accumulation.  Three bf16 pieces with six products took twice the matrix
 // work at about the same rate and rounded each sum twice as often.  Both in us
-// and against the 64-bit sums (rms): 512x13824x1152 119 -> 71, 5.2e-7 ->
-// 3.8e-7; 2048x20480x2560 1167 -> 695, 7.9e-7 -> 5.6e-7; 4096x4304x1152 284 ->
-// 155.  That is 0.9 PFLOP/s of f16 products.  Bound by the vector work of the
-// split (61 us of the 71 are left without it), the LDS traffic and the matrix
-// cores together, none of them alone.
+// and against the 64-bit sums (rms): 512x13824x1152 105 -> 76, 5.3e-7 ->
+// 3.8e-7; 2048x20480x2560 1128 -> 758, 7.9e-7 -> 5.6e-7; 4096x4304x1152 276 ->
+// 166.  That is 0.85 PFLOP/s of f16 products.  Bound by the vector work of the
+// split (six sevenths of the time are left without it), the LDS traffic and the
+// matrix cores together, none of them alone.
 //
 // Scales.  Each row of A and of B has its own power of two, set from its first
 // K step so that the step's largest value lies in [2^10, 2^11): four octaves
 // below what flags it, and with both pieces whole down to 2^-13 of it.  A later
 // step with a scaled value of 2^15 or more flags it; the workgroup then moves
 // those rows' scales, splits the step again and rescales its sums (exactly).
-// Rows of zeros start at the least scale.  A value's error is at most 2^-22 of
-// it or 2^-35 of its row's largest before it, whichever is more.
+// Rows of zeros start at the least scale.
+// Range.  The second piece ends at 2^-25, a full one for values from 2^-2 on.
+// Each lane keeps the largest of its part of a row (four of every 32 floats)
+// over eight to fifteen steps; a workgroup in which one of those is below 2^-2,
+// and not zero, does its steps over with three bf16 pieces and six products,
+// which hold any magnitudes.  So a value's error is at most 2^-23 of it or of the
+// largest of those 32 to 60, whichever is more.  (An outlier 2^24 above its row
+// and met by zeros left 2e-4 of the result.)  Over so many, rows in which values
+// near zero are common pass: gelu(gate) up with three of five below 2^-12 of
+// the largest; and over steps, not lanes, because the kernel is bound by the
+// vector work: the first product above takes 76 us so, 73 without any check and
+// 86 with the maxima of each step over four lanes.  Where every tile is done
+// over, it takes 165.
 //
 // 256 threads, 2x2 waves of 2 WM x 2 WN 16x16 tiles.  Per 32-float K step the
 // workgroup splits its A and B rows into two f16 planes each in LDS, doubly
@@ -191,6 +202,7 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
   __shared__ __attribute__((aligned(16))) _Float16 plane[2][2][(kBM + kBN) * BK];
   __shared__ int exps[kBM + kBN], moved[kBM + kBN];
   __shared__ int flag[2];  // the step that left its range, by its parity
+  __shared__ int wide;     // some row holds more than two pieces do
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -236,6 +248,19 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
     f[h] = __int_as_float((127 - e) << 23);
     if (ld_c == 0) exps[ld_row + RPP * h] = e;
   };
+  // the largest magnitude of the lane's part of row h since the last check, and
+  // the bits (less 1: zeros don't count) of the least of those
+  float g[H];
+  uint32_t low = ~0u;
+  auto check = [&]() {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      low = min(low, (uint32_t)__float_as_int(g[h]) - 1u);
+      g[h] = 0.0f;
+    }
+  };
+  constexpr uint32_t kLeast = 0x3e800000u;  // 2^-2
+  constexpr int kSteps = 8;                 // between checks, and at least before the last
   // splits row h of the step into the planes at `buf`; the largest magnitude
   const int st_at = ld_row * BK + ((ld_c / 2) ^ (ld_row / 4 % 4)) * 8 + ld_c % 2 * 4;
   static_assert(RPP % 16 == 0, "rows RPP apart swizzle alike");
@@ -279,16 +304,18 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
     kt1 = (int)((long)(blockIdx.z + 1) * nk / sk.splits);
   }
   if (tid < 2) flag[tid] = -1;
+  if (tid == 2) wide = 0;
   load(kt0);
+  lds_barrier();  // flag and wide are set
 #pragma unroll
   for (int h = 0; h < H; ++h) set(h, step_max(h));
   trim(kt0);
 #pragma unroll
-  for (int h = 0; h < H; ++h) split_store(kt0 & 1, h);
+  for (int h = 0; h < H; ++h) g[h] = split_store(kt0 & 1, h);
   load(min(kt0 + 1, kt1 - 1));
   for (int kt = kt0; kt < kt1; ++kt) {
     const int buf = kt & 1;
-    lds_barrier();  // the step's planes and flag are complete, the other planes are free
+    lds_barrier();  // the step's planes and flags are complete, the other planes are free
     if (__builtin_amdgcn_readfirstlane(flag[buf]) == kt) {
       // rows that left their range: new scales, the step split again, the sums
       // of those rows and columns rescaled
@@ -298,8 +325,10 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
         const float top = step_max(h);
         const int old = exps[ld_row + RPP * h];
         if (top * f[h] >= (float)(1 << kScaleTop)) set(h, top);
-        if (ld_c == 0) moved[ld_row + RPP * h] = old - exps[ld_row + RPP * h];
-        split_store(buf, h);
+        // as the row's first lane, which never lies past its end, set it
+        const int by = __shfl(old - exps[ld_row + RPP * h], lane & ~7, 64);
+        if (ld_c == 0) moved[ld_row + RPP * h] = by;
+        g[h] = fmaxf(ldexpf(g[h], by), split_store(buf, h));
       }
       load(min(kt + 1, kt1 - 1));
       lds_barrier();
@@ -332,7 +361,9 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
     static_assert(kPer * H == 3 * MI * NJ, "products");
 #pragma unroll
     for (int h = 0; h < H; ++h) {
-      top = fmaxf(top, split_store(1 - buf, h));
+      const float top4 = split_store(1 - buf, h);
+      top = fmaxf(top, top4);
+      g[h] = fmaxf(g[h], top4);
       x[h] = *reinterpret_cast<const v4f *>(row[h] + kb);
 #pragma unroll
       for (int u = h * kPer; u < (h + 1) * kPer; ++u) {
@@ -345,6 +376,58 @@ __global__ __launch_bounds__(kThreads, WM * WN == 4 ? 2 : WM * WN == 2 ? 3 : 4) 
       __builtin_amdgcn_sched_barrier(0);
     }
     if (__any(!(top < (float)(1 << kScaleTop))) && lane == 0) flag[1 - buf] = kt + 1;
+    if ((kt + 2 - kt0) % kSteps == 0 && kt1 - kt - 2 >= kSteps) check();
+  }
+  check();
+  // (a single lane's floats have no others beside them)
+  if (__any(low < kLeast - 1 || k - kt0 * BK <= 4) && lane == 0) wide = 1;
+  lds_barrier();  // every wave is done with the planes
+  if (__builtin_amdgcn_readfirstlane(wide) != 0) {  // the steps over, at the same scales
+#pragma unroll
+    for (int h = 0; h < H; ++h) f[h] = __int_as_float((127 - exps[ld_row + RPP * h]) << 23);
+    __bf16 *p3 = reinterpret_cast<__bf16 *>(&plane[0][0][0]);
+    constexpr int kP3 = (kBM + kBN) * BK;  // 3 planes where 4 were
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    load(kt0);
+#pragma unroll 1
+    for (int kt = kt0; kt < kt1; ++kt) {
+      trim(kt);
+      lds_barrier();  // every wave is done with the step before
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        const v4f y = x[h] * f[h];
+        const Bf3x2 lo = split3x2(y[0], y[1]), hi = split3x2(y[2], y[3]);
+        __bf16 *at = p3 + st_at + RPP * h * BK;
+        *reinterpret_cast<u2 *>(at) = u2{lo.q0, hi.q0};
+        *reinterpret_cast<u2 *>(at + kP3) = u2{lo.q1, hi.q1};
+        *reinterpret_cast<u2 *>(at + 2 * kP3) = u2{lo.q2, hi.q2};
+      }
+      load(min(kt + 1, kt1 - 1));
+      lds_barrier();
+      bf8 a[3][MI], w[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          a[p][i] = *reinterpret_cast<const bf8 *>(p3 + p * kP3 + (arow + 16 * i) * BK + rd_at);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          w[p] = *reinterpret_cast<const bf8 *>(p3 + p * kP3 + (kBM + bcol + 16 * j) * BK + rd_at);
+#pragma unroll
+        for (int o = 2; o >= 0; --o)  // the small piece products first
+#pragma unroll
+          for (int p = o; p >= 0; --p)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+              acc[i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[o - p], a[p][i], acc[i][j], 0, 0, 0);
+      }
+    }
   }
   // to the operands' units
 #pragma unroll

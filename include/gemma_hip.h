@@ -215,8 +215,10 @@ int gemma_hip_quantize_matmul(const gemma_hip_job *jobs, int njobs,
  * m == 1: dst[i][j] = sum_l src[i][l]*mat[j][l] in fp32.  The GEMM (rows
  * that start at 16-byte boundaries, k a multiple of 4) runs in split
  * precision on the f16 matrix cores: a value enters with an error of at most
- * 2^-22 of it or 2^-35 of the largest magnitude of its row, whichever is
- * more.  GEMMA_HIP_GEMM_F32=mfma in the environment, read at every launch,
+ * 2^-23 of it, or of the largest of the 32 or more values of its row that share
+ * its place in 32 over the steps around it; tiles in which one such set lies
+ * below 2^-12 of its row run with 24 bits of each value instead, at half the
+ * rate.  GEMMA_HIP_GEMM_F32=mfma in the environment, read at every launch,
  * selects the fp32 matrix cores. */
 int gemma_hip_matmul_f32(float *dst, int dstr, const float *mat, int mstr,
                          const float *src, int sstr, int m, int n, int k,

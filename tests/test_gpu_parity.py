@@ -650,6 +650,34 @@ def test_f32_row_scales(gh, oracle, monkeypatch, tile, splits, m, n, k):
     assert np.all(np.abs(host(d) - exact)[rest] <= (TOL_F32 * mag + floor)[rest])
 
 
+# Rows whose values lie apart by more than two f16 pieces hold: an outlier
+# (anywhere, of either operand) met by a zero, rows that fall along K and rows
+# with a spike are held to TOL_F32 of sum |a b| like any others, for which each
+# value must keep its own precision and not its row's.
+@pytest.mark.parametrize("tile,splits", [("128", 1), ("128x64", 2), ("64", 1), ("64", 3)])
+@pytest.mark.parametrize("m,n,k", [(130, 70, 100), (65, 129, 132), (200, 96, 1024)])
+@pytest.mark.parametrize("exp", [10, 24, 60])
+def test_f32_wide_rows(gh, oracle, monkeypatch, exp, m, n, k, tile, splits):
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32_TILE", tile)
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32_SPLIT", str(splits))
+    note(f"f32 wide rows 2^{exp} tile {tile} splits {splits} m={m} n={n} k={k}")
+    rng = np.random.default_rng(m + n + k + exp)
+    for at in (0, k // 2, k - 1):
+        A, B = rng.standard_normal((m, k)), rng.standard_normal((n, k))
+        A[::3, at] *= 2.0 ** exp
+        B[:, at] = 0
+        B[::2, (at + 50) % k] *= 2.0 ** exp
+        A[:, (at + 50) % k] = 0
+        A[1::3] *= 2.0 ** np.linspace(0, -exp / 2, k)
+        A, B = A.astype(np.float32), B.astype(np.float32)
+        d = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        gh.matmul_f32(d, n, dev(B), k, dev(A), k, m, n, k, stream())
+        exact, mag = oracle.gemm_f64(B, A)
+        err = np.abs(host(d) - exact) / mag
+        note(f"at {at}: {err.max():.3g}")
+        assert err.max() <= TOL_F32
+
+
 def test_f32_gemm_in_a_graph(gh, oracle, monkeypatch):
     """Captured into a graph, a launch that would split K runs unsplit (the
     split-K workspace may have to be allocated, which capture forbids): every
