@@ -370,11 +370,12 @@ int build_jobs(const char *fn, const gemma_hip_job *jobs, int njobs,
 
 // Attention workspaces of the entry points that take device buffers, one per
 // (device, stream): launches on one stream run in order, so they can share
-// it.  Grown on demand, kept for the next call and freed by shutdown; past
-// kAttnWsKeep bytes in all, the other streams' go, and a call that needs more
-// than that by itself has its own, freed before it returns.  (Allocated and
-// freed by every call, a 2048-row layer's took 7.5 ms beside 0.1 ms of
-// kernels.)
+// it.  Grown on demand (to twice its size at least: a prompt in chunks asks for
+// more with every chunk, and growing waits for the stream), kept for the next
+// call and freed by shutdown; past kAttnWsKeep bytes in all, the other streams'
+// go, and a call that needs more than that by itself has its own, freed before
+// it returns.  (Allocated and freed by every call, a 2048-row layer's took 7.5
+// ms beside 0.1 ms of kernels.)
 constexpr size_t kAttnWsKeep = (size_t)1 << 30;
 struct AttnWs {
   char *p = nullptr;
@@ -411,18 +412,20 @@ class AttnHold {
     }
     AttnWs &w = g_attn_ws[{dev, stream_}];
     if (w.bytes < bytes) {
-      size_t total = bytes;
+      size_t others = 0;
       for (const auto &kv : g_attn_ws)
-        if (&kv.second != &w) total += kv.second.bytes;
-      if (total > kAttnWsKeep) attn_workspaces_free(&w);
+        if (&kv.second != &w) others += kv.second.bytes;
+      size_t want = std::max(bytes, 2 * w.bytes);
+      if (others + want > kAttnWsKeep) want = bytes;
+      if (others + want > kAttnWsKeep) attn_workspaces_free(&w);
       // calls already queued on the stream may still use the old buffer
       if (w.p != nullptr && ((e = hipStreamSynchronize(stream_)) != hipSuccess ||
                              (e = hipFree(w.p)) != hipSuccess))
         return e;
       w.p = nullptr;
       w.bytes = 0;
-      if ((e = hipMalloc((void **)&w.p, bytes)) != hipSuccess) return e;
-      w.bytes = bytes;
+      if ((e = hipMalloc((void **)&w.p, want)) != hipSuccess) return e;
+      w.bytes = want;
     }
     *out = w.p;
     return hipSuccess;

@@ -452,3 +452,27 @@ def test_attention_workspaces_by_stream(gh):
         with pytest.raises(GemmaHipError, match="captured"):
             gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, 0, nh, nkv, hd, kc.shape[1], 0,
                                  asc, 0.0, False, 1, stream=streams[0].cuda_stream)
+
+
+@pytest.mark.gpu
+def test_attention_workspace_grows_seldom(gh):
+    """A prompt in 48 chunks, each behind the ones before: the workspace doubles
+    a few times, where one that grew to each call's size would wait for the
+    stream and allocate with nearly every chunk (2 MiB more each)."""
+    import torch
+
+    nh, nkv, hd, rows, chunks = 4, 4, 256, 256, 48
+    q = torch.randn(rows, nh * hd, device="cuda")
+    kc = torch.randn(nkv, rows * chunks, hd, device="cuda")
+    out = torch.empty_like(q)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    sizes = []
+    for i in range(chunks):
+        gh.prefill_attention(out, q, nh * hd, kc, kc, rows, rows * i, nh, nkv, hd, rows * chunks, 0,
+                             1 / 16, 0.0, False, 1, stream=stream.cuda_stream)
+        sizes.append(torch.cuda.mem_get_info()[0])
+    torch.cuda.synchronize()
+    changes = sum(a != b for a, b in zip(sizes, sizes[1:]))
+    print(f"{changes} allocations", flush=True)
+    assert changes <= 8
