@@ -395,6 +395,18 @@ void attn_workspaces_free(const AttnWs *but) {  // hipFree waits for the device'
   }
 }
 
+// Lets this thread allocate and free while another one's stream is being
+// captured (in the global mode, the default, that fails otherwise): nothing
+// here belongs to that capture.
+class AllocAnyway {
+ public:
+  AllocAnyway() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  ~AllocAnyway() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // One call's hold on its stream's workspace, to its last launch: no other
 // thread frees it before they are queued.
 class AttnHold {
@@ -402,6 +414,7 @@ class AttnHold {
   explicit AttnHold(hipStream_t stream) : hold_(g_attn_mu), stream_(stream) {}
   ~AttnHold() { (void)done(); }
   hipError_t get(size_t bytes, char **out) {
+    const AllocAnyway anyway;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
@@ -432,6 +445,7 @@ class AttnHold {
   }
   hipError_t done() {  // waits only for a workspace of the call's own
     if (own_ == nullptr) return hipSuccess;
+    const AllocAnyway anyway;
     const hipError_t e = hipStreamSynchronize(stream_);
     (void)hipFree(own_);
     own_ = nullptr;
@@ -947,9 +961,13 @@ int gemma_hip_vision_attention(float *out, const float *qkv, const float *bias, 
   const bool f32 = mode == GEMMA_HIP_ATTN_F32;
   char *planes = nullptr;
   AttnHold ws(s);
-  if (f32 && !capturing(s))  // a captured call can't allocate: the kernel without a workspace
-    GH_CHECK("gemma_hip_vision_attention: workspace",
-             ws.get(gh::attn_planes_bytes(hdim, n_heads, n), &planes));
+  // without a workspace (a captured call can't allocate one, and memory may be
+  // short) the kernel that needs none runs
+  if (f32 && !capturing(s) &&
+      ws.get(gh::attn_planes_bytes(hdim, n_heads, n), &planes) != hipSuccess) {
+    (void)hipGetLastError();
+    planes = nullptr;
+  }
   GH_CHECK("gemma_hip_vision_attention: launch",
            gh::launch_vis_attention(at, hdim, f32, planes, g.info, s));
   GH_CHECK("gemma_hip_vision_attention", ws.done());

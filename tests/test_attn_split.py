@@ -476,3 +476,41 @@ def test_attention_workspace_grows_seldom(gh):
     changes = sum(a != b for a, b in zip(sizes, sizes[1:]))
     print(f"{changes} allocations", flush=True)
     assert changes <= 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["vision", "prefill"])
+def test_attention_beside_a_capture(gh, entry):
+    """Eager attention on one stream while another is being captured (in the
+    global mode): it may need its first workspace, gets it, and leaves the
+    capture whole."""
+    import torch
+
+    rng = np.random.default_rng(11)
+    n, heads, hd, nh, nkv = 300, 2, 72, 4, 2
+    dim = heads * hd
+    qkv = rng.standard_normal((n, 3 * dim)).astype(np.float32)
+    bias = np.zeros(3 * dim, np.float32)
+    q, kc, vc = _prefill_inputs(n, 0, nh, nkv, 128, seed=12)
+    dqkv, db, dq, dk, dv = (torch.from_numpy(a).cuda() for a in (qkv, bias, q, kc, vc))
+    x = torch.zeros(1000, device="cuda")
+    out = torch.empty((n, dim if entry == "vision" else nh * 128), device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[0], capture_error_mode="global"):
+        x += 1
+        s = streams[1].cuda_stream
+        if entry == "vision":
+            gh.vision_attention(out, dqkv, db, n, heads, dim, 1, s)
+        else:
+            gh.prefill_attention(out, dq, q.shape[1], dk, dv, n, 0, nh, nkv, 128, kc.shape[1], 0,
+                                 np.float32(1) / np.sqrt(np.float32(128)), 0.0, False, 1, stream=s)
+        x += 2
+    torch.cuda.synchronize()
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (x == 3 * (i + 1)).all()
+    _close(out.cpu().numpy(), _vision_want(qkv, bias, heads, dim) if entry == "vision" else
+           _prefill_want(q, kc, vc, n, 0, nh, nkv, 128, 0, 0.0, False))
