@@ -707,10 +707,12 @@ H2Plan h2_plan(int m, int n, int k, bool may_split, const DeviceInfo &dev) {
 hipError_t launch_h2_auto(float *dst, int dstr, const F32Segs &b, int mstr, const float *src,
                           int sstr, int m, int k, const F32Epilogue &ep, const DeviceInfo &dev,
                           hipStream_t stream) {
-  // the split-K workspace may have to be allocated: not under capture
+  // the split-K workspace is kept by stream, and may have to be allocated: not
+  // for a handle of several streams, not under capture
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool may_split =
-      hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+  const bool may_split = stream_has_own_handle(stream) &&
+                         hipStreamIsCapturing(stream, &cap) == hipSuccess &&
+                         cap == hipStreamCaptureStatusNone;
   const H2Plan p = h2_plan(m, b.end[b.nseg - 1], k, may_split, dev);
   if (p.tile == kTile128)
     return launch_h2<2, 2>(dst, dstr, b, mstr, src, sstr, m, k, ep, p.splits, stream);

@@ -1259,7 +1259,7 @@ SplitPlan choose_split(int m, int n, int k, const DeviceInfo &dev, hipStream_t s
   SplitPlan p;
   const int nk128 = (k + 127) / 128;
   const int forced = env_split();
-  if (forced > 0) {
+  if (forced > 0 && (fixed_ws || stream_has_own_handle(stream))) {
     p.splits = forced > nk128 ? nk128 : forced;
     return p;
   }
@@ -1276,9 +1276,12 @@ SplitPlan choose_split(int m, int n, int k, const DeviceInfo &dev, hipStream_t s
   }
   if (want.splits < 2) return p;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (!fixed_ws &&
-      (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone))
-    return p;  // the workspace may have to be allocated: not under capture
+  // the workspace is kept by stream, and may have to be allocated: not for a
+  // handle of several streams, not under capture
+  if (!fixed_ws && (!stream_has_own_handle(stream) ||
+                    hipStreamIsCapturing(stream, &cap) != hipSuccess ||
+                    cap != hipStreamCaptureStatusNone))
+    return p;
   return want;
 }
 

@@ -373,8 +373,8 @@ int build_jobs(const char *fn, const gemma_hip_job *jobs, int njobs,
 // it.  Grown on demand (to twice its size at least: a prompt in chunks asks for
 // more with every chunk, and growing waits for the stream), kept for the next
 // call and freed by shutdown; past kAttnWsKeep bytes in all, the other streams'
-// go, and a call that needs more than that by itself has its own, freed before
-// it returns.  (Allocated and freed by every call, a 2048-row layer's took 7.5
+// go, and a call that needs more than that by itself, or whose handle names
+// several threads' streams, has its own, freed before it returns.  (Allocated and freed by every call, a 2048-row layer's took 7.5
 // ms beside 0.1 ms of kernels.)
 constexpr size_t kAttnWsKeep = (size_t)1 << 30;
 struct AttnWs {
@@ -418,7 +418,7 @@ class AttnHold {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    if (bytes > kAttnWsKeep) {
+    if (bytes > kAttnWsKeep || !gh::stream_has_own_handle(stream_)) {
       if ((e = hipMalloc((void **)&own_, bytes)) != hipSuccess) return e;
       *out = own_;
       return hipSuccess;
@@ -961,9 +961,10 @@ int gemma_hip_vision_attention(float *out, const float *qkv, const float *bias, 
   const bool f32 = mode == GEMMA_HIP_ATTN_F32;
   char *planes = nullptr;
   AttnHold ws(s);
-  // without a workspace (a captured call can't allocate one, and memory may be
-  // short) the kernel that needs none runs
-  if (f32 && !capturing(s) &&
+  // without a workspace (a captured call can't allocate one, one for a handle of
+  // several streams would be allocated by every call, and memory may be short)
+  // the kernel that needs none runs
+  if (f32 && gh::stream_has_own_handle(s) && !capturing(s) &&
       ws.get(gh::attn_planes_bytes(hdim, n_heads, n), &planes) != hipSuccess) {
     (void)hipGetLastError();
     planes = nullptr;

@@ -119,6 +119,10 @@ hipError_t launch_gemm_i8_segs(float *dst, int dstr, const GemmSegs &b, const in
                                int sstr, const float *ssc, int m, int k, const DeviceInfo &dev,
                                hipStream_t stream);
 
+// Whether a workspace can be kept for a stream's later launches by its handle:
+// hipStreamPerThread is one handle for a different stream in every thread.
+inline bool stream_has_own_handle(hipStream_t stream) { return stream != hipStreamPerThread; }
+
 // gemm_f32.hip: dst = src . mat^T in fp32; bias (nullable) adds bias[col],
 // clamp limits every output to [-FLT_MAX, FLT_MAX] (clamp_fpx).
 hipError_t launch_gemm_f32(float *dst, int dstr, const float *mat, int mstr,

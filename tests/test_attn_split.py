@@ -514,3 +514,74 @@ def test_attention_beside_a_capture(gh, entry):
         assert (x == 3 * (i + 1)).all()
     _close(out.cpu().numpy(), _vision_want(qkv, bias, heads, dim) if entry == "vision" else
            _prefill_want(q, kc, vc, n, 0, nh, nkv, 128, 0, 0.0, False))
+
+
+@pytest.mark.gpu
+def test_per_thread_streams(gh):
+    """hipStreamPerThread, one handle for a stream of each thread's own: calls
+    that need workspaces (both attentions, int8 and fp32 split-K products) from
+    four threads at once give what they give one after another."""
+    import threading
+
+    import torch
+
+    per_thread = 2  # hipStreamPerThread
+    nh, nkv, hd, m, n8, k8 = 4, 2, 128, 300, 640, 2064
+    asc = np.float32(1) / np.sqrt(np.float32(hd))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+
+    def inputs():
+        r = lambda *s: torch.randn(s, generator=gen, device="cuda")  # noqa: E731
+        i8 = lambda *s: torch.randint(-127, 128, s, generator=gen, device="cuda",  # noqa: E731
+                                      dtype=torch.int8)
+        d = dict(q=r(400, nh * hd), kc=r(nkv, 400, hd), vc=r(nkv, 400, hd), qkv=r(400, 3 * 144),
+                 a=r(64, 2048), b=r(512, 2048), a8=i8(m, k8), b8=i8(n8, k8), sa=r(m).abs(),
+                 sb=r(n8).abs())
+        d["out"] = [torch.zeros(s, device="cuda")
+                    for s in ((400, nh * hd), (400, 144), (64, 512), (m, n8))]
+        return d
+
+    bias = torch.zeros(3 * 144, device="cuda")
+
+    def calls(d):
+        o = d["out"]
+        gh.prefill_attention(o[0], d["q"], nh * hd, d["kc"], d["vc"], 400, 0, nh, nkv, hd, 400, 0,
+                             asc, 0.0, False, 1, stream=per_thread)
+        gh.vision_attention(o[1], d["qkv"], bias, 400, 2, 144, 1, per_thread)
+        gh.matmul_f32(o[2], 512, d["b"], 2048, d["a"], 2048, 64, 512, 2048, per_thread)
+        gh.matmul(o[3], n8, d["b8"], k8, d["sb"], d["a8"], k8, d["sa"], m, n8, k8, per_thread)
+
+    jobs = [inputs() for _ in range(4)]
+    torch.cuda.synchronize()
+    want = []
+    for d in jobs:
+        calls(d)
+        torch.cuda.synchronize()
+        want.append([t.clone() for t in d["out"]])
+        for t in d["out"]:
+            t.zero_()
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(d):
+        try:
+            for _ in range(20):
+                calls(d)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(d,)) for d in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for d, w in zip(jobs, want):
+        assert all(torch.equal(a, b) for a, b in zip(d["out"], w))
+    # and what they give is right
+    d = jobs[0]
+    _close(d["out"][0].cpu().numpy(),
+           _prefill_want(d["q"].cpu().numpy(), d["kc"].cpu().numpy(), d["vc"].cpu().numpy(), 400, 0,
+                         nh, nkv, hd, 0, 0.0, False))
+    _close(d["out"][2].cpu().numpy(), (d["a"].double() @ d["b"].double().T).cpu().numpy())
