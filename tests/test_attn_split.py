@@ -285,6 +285,38 @@ def test_vision_attention_under_capture(gh):
         _close(_vision(gh, qkv, bias, heads, dim), want)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [16, 32, 64, 72, 128])
+@pytest.mark.parametrize("n,heads", [(1, 1), (33, 2), (129, 1), (257, 3), (300, 8)])
+def test_vision_workspace_free_kernel(gh, n, heads, hd):
+    """The kernel of captured calls at every head dim and around its 16-query
+    waves, 128- and 256-query workgroups and 32-key tiles, V's tiles at
+    magnitudes far apart."""
+    import torch
+
+    rng = np.random.default_rng(n + hd)
+    dim = heads * hd
+    qkv = rng.standard_normal((n, 3 * dim))
+    qkv[:, 2 * dim:] *= _tile_scales(n, (0, 40, -40))
+    qkv = qkv.astype(np.float32)
+    bias = (0.5 * rng.standard_normal(3 * dim)).astype(np.float32)
+    want = _vision_want(qkv, bias, heads, dim)
+    dq, db = torch.from_numpy(qkv).cuda(), torch.from_numpy(bias).cuda()
+    out = torch.full((n + 1, dim), float("nan"), device="cuda")
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        gh.vision_attention(out, dq, db, n, heads, dim, 1, side.cuda_stream)
+    for _ in range(2):
+        out[:n] = 0
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert np.isnan(got[n]).all()
+        _close(got[:n], want)
+
+
 def _prefill_want(q, kc, vc, n, pos0, nh, nkv, hd, slide, cap, dense, asc=None):
     ctx = pos0 + n
     pos = pos0 + np.arange(n)
