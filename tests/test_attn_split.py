@@ -617,3 +617,50 @@ def test_per_thread_streams(gh):
            _prefill_want(d["q"].cpu().numpy(), d["kc"].cpu().numpy(), d["vc"].cpu().numpy(), 400, 0,
                          nh, nkv, hd, 0, 0.0, False))
     _close(d["out"][2].cpu().numpy(), (d["a"].double() @ d["b"].double().T).cpu().numpy())
+
+
+def _rms(got, want):
+    return float(np.linalg.norm(got - want) / np.linalg.norm(want))
+
+
+# Where the errors of the two forms stand, as a guard against growth that the
+# bars of single values would let through: two f16 pieces round each sum half as
+# often as three bf16 pieces with six products, and stay below them (measured,
+# split against three pieces: 4.3e-7 / 5.4e-7 over 1024 patches, 2.7e-7 / 3.3e-7 in
+# a 300-row prompt).
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,heads,hd", [(300, 2, 72), (1024, 2, 72), (1000, 2, 128), (600, 4, 64)])
+def test_vision_error_level(gh, n, heads, hd):
+    import torch
+
+    rng = np.random.default_rng(n)
+    dim = heads * hd
+    qkv = rng.standard_normal((n, 3 * dim)).astype(np.float32)
+    bias = (0.02 * rng.standard_normal(3 * dim)).astype(np.float32)
+    want = _vision_want(qkv, bias, heads, dim)
+    split = _rms(_vision(gh, qkv, bias, heads, dim), want)
+    dq, db = torch.from_numpy(qkv).cuda(), torch.from_numpy(bias).cuda()
+    out = torch.zeros((n, dim), device="cuda")
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        gh.vision_attention(out, dq, db, n, heads, dim, 1, side.cuda_stream)
+    graph.replay()
+    torch.cuda.synchronize()
+    three = _rms(out.cpu().numpy(), want)
+    print(f"split {split:.3g}, three pieces {three:.3g}", flush=True)
+    assert split <= three
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,pos0,nh,nkv,hd", [(300, 0, 4, 1, 256), (257, 500, 4, 1, 256),
+                                              (500, 0, 4, 2, 128)])
+def test_prefill_error_level(gh, monkeypatch, n, pos0, nh, nkv, hd):
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
+    q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=n)
+    args = (n, pos0, nh, nkv, hd, 0, 0.0, False)
+    split = _rms(_prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args))
+    vc[:, 0:pos0 + n:32] = 0  # a zero key in every tile: three pieces
+    three = _rms(_prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args))
+    print(f"split {split:.3g}, three pieces {three:.3g}", flush=True)
+    assert split <= three

@@ -678,6 +678,35 @@ def test_f32_wide_rows(gh, oracle, monkeypatch, exp, m, n, k, tile, splits):
         assert err.max() <= TOL_F32
 
 
+# Where the errors stand (TOL_F32 would let them grow thirtyfold): two f16 pieces
+# round each sum half as often as three bf16 ones, and less than fp32 MFMA.
+# Measured, unsplit, K = 2560: 5.6e-7, three pieces 7.8e-7, MFMA 9.0e-7.
+@pytest.mark.parametrize("m,n,k", [(128, 128, 640), (200, 300, 1152), (128, 512, 2560)])
+def test_f32_error_level(gh, monkeypatch, m, n, k):
+    note(f"f32 error level m={m} n={n} k={k}")
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32_SPLIT", "1")
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn(m, k, device="cuda", generator=gen)
+    a[:, ::97] *= 8
+    b = torch.randn(n, k, device="cuda", generator=gen) * 0.02
+
+    def error(a, b):
+        d = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        gh.matmul_f32(d, n, b, k, a, k, m, n, k, stream())
+        want = a.double() @ b.double().t()
+        return float((d - want).norm() / want.norm())
+
+    split = error(a, b)
+    wide_a, wide_b = a.clone(), b.clone()
+    wide_a[:, 5] = 2.0 ** 40
+    wide_b[:, 5] = 0
+    three = error(wide_a, wide_b)
+    monkeypatch.setenv("GEMMA_HIP_GEMM_F32", "mfma")
+    mfma = error(a, b)
+    note(f"split {split:.3g}, three pieces {three:.3g}, mfma {mfma:.3g}")
+    assert split <= three and split <= mfma
+
+
 def test_f32_gemm_in_a_graph(gh, oracle, monkeypatch):
     """Captured into a graph, a launch that would split K runs unsplit (the
     split-K workspace may have to be allocated, which capture forbids): every
