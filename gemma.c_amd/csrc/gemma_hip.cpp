@@ -1304,6 +1304,7 @@ struct gemma_hip_decoder {
   int *pf_tok = nullptr;
   double *pf_part = nullptr;  // attention key-split partials
   char *pf_planes = nullptr;  // ... and packed K and V tiles
+  size_t pf_planes_bytes = 0;
 };
 
 namespace {
@@ -1321,9 +1322,19 @@ void decoder_free(gemma_hip_decoder *d) {
 // Row buffers of the batched prefill for n rows (kept, and regrown only for
 // a larger n): x, y [n][dim]; q/k/v [n][q_sz + 2 kv_sz]; attention output
 // [n][q_sz]; gate|up [n][2 mlp]; quantized rows [n][max K] + their scales.
-int prefill_reserve(gemma_hip_decoder *d, int n) {
-  if (n <= d->pf_rows) return 0;
+// The packed tiles hold `keys` keys (in the mode that packs them), twice what
+// they did at least when they grow and at most the whole cache's: 1 GiB for the
+// 131072 positions of gemma-3-4b, which short prompts don't need.
+int prefill_reserve(gemma_hip_decoder *d, int n, int keys) {
   const gemma_hip_text_config &c = d->cfg;
+  auto tiles = [&](int of) { return gh::attn_planes_bytes(c.hdim, c.nkv, of); };
+  size_t planes = d->attn_f32 ? tiles(keys) : 0;
+  if (n <= d->pf_rows && planes <= d->pf_planes_bytes) return 0;
+  if (planes > d->pf_planes_bytes)
+    planes = std::min(tiles(d->clen), std::max(planes, 2 * d->pf_planes_bytes));
+  else
+    planes = d->pf_planes_bytes;
+  n = std::max(n, d->pf_rows);
   const size_t rows = (size_t)n, q_sz = (size_t)c.n_heads * c.hdim,
                kv_sz = (size_t)c.nkv * c.hdim, dim = c.dim, mlp = c.mlp_dim;
   const size_t kmax = std::max(dim, std::max(q_sz, mlp));
@@ -1333,13 +1344,13 @@ int prefill_reserve(gemma_hip_decoder *d, int n) {
                o_g = cv.take(rows * 2 * mlp * 4), o_a8 = cv.take(rows * kmax),
                o_as = cv.take(rows * 4), o_tok = cv.take(rows * 4),
                o_part = cv.take(gh::pf_attn_part_doubles(rows, c.n_heads, c.hdim) * 8),
-               o_h = cv.take(d->quant ? 0 : rows * dim * 4),
-               o_pl = cv.take(gh::attn_planes_bytes(c.hdim, c.nkv, d->clen));
+               o_h = cv.take(d->quant ? 0 : rows * dim * 4), o_pl = cv.take(planes);
   if (d->pf_mem != nullptr) {
     (void)hipStreamSynchronize(g.stream);
     (void)hipFree(d->pf_mem);
     d->pf_mem = nullptr;
     d->pf_rows = 0;
+    d->pf_planes_bytes = 0;
   }
   hipError_t e = hipMalloc((void **)&d->pf_mem, cv.used);
   if (e != hipSuccess) return hip_fail("gemma_hip_decoder_prefill: alloc", e);
@@ -1355,6 +1366,7 @@ int prefill_reserve(gemma_hip_decoder *d, int n) {
   d->pf_part = (double *)(m + o_part);
   d->pf_h = d->quant ? nullptr : (float *)(m + o_h);
   d->pf_planes = m + o_pl;
+  d->pf_planes_bytes = planes;
   d->pf_rows = n;
   return 0;
 }
@@ -1490,10 +1502,10 @@ int prefill_check(const gemma_hip_decoder *dec, const char *name, int n, int pos
     if (gh_e_ != hipSuccess) return fail("%s: %s: %s", kName, what, hipGetErrorString(gh_e_)); \
   } while (0)
 
-// Waits for earlier work on the stream and makes room for n rows.
-int prefill_stage(gemma_hip_decoder *dec, const char *kName, int n) {
+// Waits for earlier work on the stream and makes room for n rows at pos.
+int prefill_stage(gemma_hip_decoder *dec, const char *kName, int n, int pos) {
   PF_CHECK("sync", hipStreamSynchronize(g.stream));
-  return prefill_reserve(dec, n);
+  return prefill_reserve(dec, n, pos + n);
 }
 
 // With the rows staged (tokens in pf_tok when embed, else the rows in pf_x):
@@ -2109,7 +2121,7 @@ int gemma_hip_decoder_prefill(gemma_hip_decoder *dec, const int *tokens, int n, 
     if (tokens[i] < 0 || tokens[i] >= dec->cfg.nvocab)
       return fail("%s: token %d at %d out of range (vocab %d)", kName, tokens[i], i,
                   dec->cfg.nvocab);
-  if (prefill_stage(dec, kName, n)) return 1;
+  if (prefill_stage(dec, kName, n, pos)) return 1;
   PF_CHECK("tokens H2D",
            hipMemcpyAsync(dec->pf_tok, tokens, (size_t)n * 4, hipMemcpyHostToDevice, g.stream));
   perf_enter(kPhasePrefill);
@@ -2121,7 +2133,7 @@ int gemma_hip_decoder_prefill_rows(gemma_hip_decoder *dec, const float *x, int n
   static const char *kName = "gemma_hip_decoder_prefill_rows";
   if (need_init()) return 1;
   if (dec == nullptr || x == nullptr) return fail("%s: null argument", kName);
-  if (prefill_check(dec, kName, n, pos) || prefill_stage(dec, kName, n)) return 1;
+  if (prefill_check(dec, kName, n, pos) || prefill_stage(dec, kName, n, pos)) return 1;
   PF_CHECK("rows copy", hipMemcpyAsync(dec->pf_x, x, (size_t)n * dec->cfg.dim * 4,
                                        hipMemcpyDefault, g.stream));
   // text rows belong to the prefill phase, image soft tokens (the dense
@@ -2590,7 +2602,7 @@ int gemma_hip_gemma_image(gemma_hip_decoder *dec, gemma_hip_vision *vis, const f
   if (c.text_dim != dec->cfg.dim)
     return fail("%s: the tower projects to %d, the decoder is %d wide", kName, c.text_dim,
                 dec->cfg.dim);
-  if (prefill_check(dec, kName, c.img_tok, *pos) || prefill_stage(dec, kName, c.img_tok))
+  if (prefill_check(dec, kName, c.img_tok, *pos) || prefill_stage(dec, kName, c.img_tok, *pos))
     return 1;
   PF_CHECK("image H2D", hipMemcpyAsync(vis->img, img, (size_t)c.img_px * c.img_px * 3 * 4,
                                        hipMemcpyHostToDevice, g.stream));

@@ -466,6 +466,25 @@ def test_prefill_in_chunks_f32_attention(gh, oracle, models):
 
 
 @pytest.mark.gpu
+def test_prefill_memory_follows_the_prompt(gh, models):
+    """A short prompt takes no memory for the whole cache's packed keys: 256 MiB
+    of them for 131072 positions here."""
+    import torch
+
+    prompt = np.arange(16, dtype=np.int32)
+    dec = gh.decoder(models["hd128"], 131072, attention=ATTN_F32)
+    try:
+        before = torch.cuda.mem_get_info()[0]
+        dec.prefill(prompt, 0)
+        dec.prefill(prompt, 16)
+        taken = before - torch.cuda.mem_get_info()[0]
+    finally:
+        dec.close()
+    print(f"{taken / 2 ** 20:.1f} MiB", flush=True)
+    assert taken < 64 << 20
+
+
+@pytest.mark.gpu
 def test_prefill_argument_errors(gh, models):
     from gemma_hip import GemmaHipError
 
