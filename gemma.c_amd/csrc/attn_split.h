@@ -476,7 +476,8 @@ struct AttnWave {
   // what two f16 pieces don't.
   __device__ __forceinline__ bool run(const char *tiles, const TileRange *range, int ta, int tb,
                                       int keys, const AttnSee &see, float asc, float c_hi,
-                                      float c_lo, float cap, char *lds, v4f *red, int wave, int lane) {
+                                      float c_lo, float cap, char *lds, v4f *red, int wave,
+                                      int lane) {
     const int half = lane >> 5;
     char *kbuf = lds, *vbuf = lds + 2 * G::KFR * 1024;
     const uint32_t loff = lane * 16;

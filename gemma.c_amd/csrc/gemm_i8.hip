@@ -97,7 +97,7 @@ __device__ __forceinline__ v4i load16_tail(const int8_t *row, int kb, int k) {
 
 // Rows/columns beyond m/n and K beyond k load as zeros.  With ANY, rows at any
 // address and any k (odd widths; the DMA kernels need 16-byte rows): one thread
-// per output, byte by byte, took 9.5 ms at 1064 x 10240 x 7089, here 0.1.
+// per output, byte by byte, took 112.5 ms at 1064 x 10240 x 7089, here 0.21.
 // Without (checked by the launcher) k % 16 == 0 and every row 16-byte aligned:
 // operands beyond 32-bit offsets.
 // WM x WN: each wave's sub-tile in 32x32 MFMA tiles; waves form a 2x2 grid,

@@ -318,12 +318,12 @@ struct PfAttn {
   int8_t *xq;
   float *xs;
   // fp32 mode: room for the split kernel's packed K and V tiles of keys
-  // 0 .. pos0+n-1 (attn_planes_bytes); null: the fp32-MFMA kernel only
+  // 0 .. pos0+n-1 (attn_planes_bytes)
   char *planes;
   int log2m;  // partials' reference maxima are base-2 logarithms (set by the launcher)
 };
-// Bytes of the packed K and V tiles (attn_split.h) of `keys` keys, the tiles'
-// exponents included.
+// Bytes of the packed K and V tiles (attn_split.h) of `keys` keys, what each
+// tile holds included.
 size_t attn_planes_bytes(int hdim, int heads, int keys);
 constexpr int kPfMaxSplit = 8;
 constexpr int kPfMaxMergeHeads = 64;  // q heads the key-split merge handles

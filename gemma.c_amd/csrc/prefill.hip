@@ -609,13 +609,15 @@ __global__ __launch_bounds__(kNT, 2) void pf_attn_f32_kernel(PfAttn a) {
 // head's q heads at 128 / hn rows), and its tiles are the cache's keys packed by
 // attn_pack_kernel.  At head dim 256 a wave holds its queries' pieces and the
 // value sums in 256 registers, so each SIMD runs one wave and a CU one
-// workgroup (128 KB of LDS); the tile loop overlaps its softmax with the next
+// workgroup (128 KB of LDS for the tiles); the tile loop overlaps its softmax with the next
 // tile's score products by itself.  A tile of 32 keys takes 2.7 us, 2.4 of them
 // with its loads and LDS reads taken out: the 96 products of a wave at the clock
 // that the chip holds under f16 products on all CUs.  gemma-3-4b, 2048 rows,
-// window 1024: packing 11, kernel 63, merge 11 us, where three bf16 pieces with
-// six products, split in the kernel, took 111 + 11; global layers 12 + 71 + 11
-// against 135 + 11.  Error against 64-bit sums 4.0e-7 -> 3.3e-7 relative.
+// window 1024: packing 10.4, kernel 62.4, merge 11 us, where three bf16 pieces
+// with six products, split in the kernel, took 111 + 11; global layers 12 + 71 +
+// 11 against 135 + 11.  Error against 64-bit sums 4.0e-7 -> 3.3e-7 relative.
+// Workgroups whose tiles need three pieces (attn_split.h) take about three
+// times as long: both layers 250 and 300 us with V's tiles 2^24 apart.
 constexpr int kPbWaves = 4;
 constexpr int kPbQ = kPbWaves * 32;  // query vectors per workgroup
 
@@ -1066,8 +1068,9 @@ int pf_chunk(int kmax, int split) {
 
 // The key split for the split-f16 kernel, which runs one workgroup per CU (head
 // dim 256): each candidate split's blocks are dealt, in launch order (pa_lane's
-// block order), to the CU of their XCD that frees first, each costing its chunk's tiles plus
-// a fixed prologue and epilogue of about four tiles, and the merge pass reads and writes the partials once per chunk.
+// block order), to the CU of their XCD that frees first, each costing its
+// chunk's tiles plus a fixed prologue and epilogue of about four tiles, and the
+// merge pass reads and writes the partials once per chunk.
 // Measured, kernel + merge, 8 q heads on 4 kv heads: 2048 rows in a 1024-key
 // window 75 us in two chunks (one 96, three 98), global 80 in three (two 99,
 // four 115), 1024 global rows 47 in four (two 59, seven 61); this model ranks
@@ -1146,9 +1149,9 @@ int pf_key_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int
 }
 
 // The fp32 mode's kernel, read at every launch so that one process can time
-// or check both: GEMMA_HIP_PF_ATTN=f32 the fp32-MFMA one, =bf3 the split-f16
-// one; unset, the split-f16 one from kPbMinFlops of score and value products
-// on.  Below, its packing launch and its longer prologue (about 15 us together)
+// or check both: GEMMA_HIP_PF_ATTN=f32 the fp32-MFMA one, =split (or =bf3, the
+// name of the kernel before it) the split-f16 one; unset, the split-f16 one from
+// kPbMinFlops of score and value products on.  Below, its packing launch and its longer prologue (about 15 us together)
 // outweigh its rate, 2.5 times the other's: whole prompt passes, fp32-MFMA
 // against split, gemma-3-270m (6 layers) at 512 rows (0.8 GFLOP a layer) 611
 // against 660 us, 700 rows 679 / 694; gemma-3-4b (2 layers) at 400 rows (0.66)
@@ -1158,7 +1161,8 @@ enum PfKind { kPfF32, kPfSplit, kPfAuto };
 PfKind pf_attn_kind() {
   const char *e = getenv("GEMMA_HIP_PF_ATTN");
   if (e == nullptr) return kPfAuto;
-  return strcmp(e, "f32") == 0 ? kPfF32 : strcmp(e, "bf3") == 0 ? kPfSplit : kPfAuto;
+  if (strcmp(e, "f32") == 0) return kPfF32;
+  return strcmp(e, "split") == 0 || strcmp(e, "bf3") == 0 ? kPfSplit : kPfAuto;
 }
 
 // Score and value products of the n rows: 4 hdim flops per head and (row, key)
@@ -1193,13 +1197,13 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
                                hipStream_t stream) {
   const int hn = a.nkv > 0 ? a.n_heads / a.nkv : 0;
   if (hn <= 0 || kPbQ % hn != 0 || kPaQ % hn != 0 || kPaQPair % hn != 0 || a.n <= 0 ||
-      a.part == nullptr || a.n_heads > kPfMaxMergeHeads)
+      a.part == nullptr || (f32 && a.planes == nullptr) || a.n_heads > kPfMaxMergeHeads)
     return hipErrorInvalidValue;
   bool splitk = false;  // the split-f16 kernel
   PaGeo geo{};
   // (the split kernel takes each tile's largest score from its largest raw
   // product: a negative scale would make that the smallest)
-  if (f32 && a.planes != nullptr && a.asc >= 0.0f) {
+  if (f32 && a.asc >= 0.0f) {
     const PfKind kind = pf_attn_kind();
     if (kind != kPfF32) {
       geo = pa_geo(a, kPbQ);
@@ -1248,7 +1252,8 @@ hipError_t launch_pf_attention(const PfAttn &a, int hdim, bool f32, const Device
       if (a.sc_att != 0.0f)
         pf_attn_split_kernel<HD, true><<<grid, kPbWaves * 64, 0, stream>>>(b, range, tile0, ntiles);
       else
-        pf_attn_split_kernel<HD, false><<<grid, kPbWaves * 64, 0, stream>>>(b, range, tile0, ntiles);
+        pf_attn_split_kernel<HD, false><<<grid, kPbWaves * 64, 0, stream>>>(b, range, tile0,
+                                                                            ntiles);
     };
     switch (hdim) {
       case 128: go(std::integral_constant<int, 128>{}); break;

@@ -670,11 +670,13 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void vis_attn_bf3_kernel(VisAttn 
 // attn_pack_kernel made of K and V with their biases.  Bound by the matrix
 // cores at the clock that the chip holds under them: SigLIP at 896 px (4096
 // patches, 16 heads of 72) takes 30 products per 32 queries and tile, 258
-// TFLOP of f16 in 215 us (1.2 PFLOP/s; v_mfma_f32_32x32x16_f16 on random
-// registers alone sustains 1.6), packing 18 us.  The three-bf16-piece kernel
-// before it took 426 us at the same matrix rate with twice the products, and
-// its error against 64-bit sums was larger: 9.6e-7 relative, here 7.0e-7 (fewer
-// fp32 roundings per sum).  The tower's image (9 of 27 layers): 6.73 -> 4.7 ms.
+// GFLOP of f16 in 215-235 us (1.1-1.2 PFLOP/s; v_mfma_f32_32x32x16_f16 on random
+// registers alone sustains 1.6), packing 17.8 us.  Three bf16 pieces take 430
+// by themselves (vis_attn_bf3_kernel) at the same matrix rate with twice the
+// products, and their error against 64-bit sums is larger: 9.6e-7 relative, here
+// 7.0e-7 (fewer fp32 roundings per sum).  Where the tiles need them all the
+// same, the layer takes 710 us (V's tiles 2^24 apart).  The tower's image (9 of
+// 27 layers): 6.73 -> 4.7 ms.
 template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64, 2) void vis_attn_split_kernel(VisAttn a, const char *planes,
                                                                    const TileRange *range,
@@ -735,8 +737,8 @@ void launch_vis_split(const VisAttn &a, char *planes, const DeviceInfo &dev, hip
 }
 
 // The fp32 mode's kernel: a split one by default (f16 pieces with a workspace,
-// bf16 pieces without), the fp32-MFMA one with GEMMA_HIP_VIS_ATTN=f32.  Read at every launch (one getenv per layer),
-// so that one process can time or check both.
+// bf16 pieces without), the fp32-MFMA one with GEMMA_HIP_VIS_ATTN=f32.  Read at
+// every launch (one getenv per layer), so that one process can time or check both.
 bool vis_attn_split() {
   const char *e = getenv("GEMMA_HIP_VIS_ATTN");
   return e == nullptr || strcmp(e, "f32") != 0;

@@ -351,9 +351,9 @@ typedef struct {
  * tied LM head), the projections run as fp32 GEMVs (gemv_fpx) in the step
  * (the norms fused into the q/k/v and gate/up GEMVs, GELU into gate/up, as
  * in the W8A8 step) and as fp32 GEMMs (gemm_fpx: on the f16 matrix cores in
- * split precision, fp32 accuracy) in the prompt pass, with no activation
- * quantize.  Every other decoder entry point takes the result as it takes a
- * W8A8 decoder. */
+ * split precision, with gemma_hip_matmul_f32's accuracy) in the prompt pass,
+ * with no activation quantize.  Every other decoder entry point takes the
+ * result as it takes a W8A8 decoder. */
 gemma_hip_decoder *gemma_hip_decoder_create_f32(const gemma_hip_text_config *cfg,
                                                 const gemma_hip_layer_f32 *layers,
                                                 const float *emb, const float *fnorm,
@@ -396,12 +396,15 @@ int gemma_hip_decoder_prefill_rows(gemma_hip_decoder *dec, const float *x, int n
  * the exact sum: the verification mode, equal to an fp64 evaluation of the
  * same formulas).  The fp32 mode runs on the f16 matrix cores in split
  * precision (each fp32 operand scaled by a power of two and split into two f16
- * pieces, each product summed from three piece products, fp32 accumulation:
- * closer to the exact result than fp32 matrix cores, whose sums round more
- * often), or, for passes below about a GFLOP of attention a layer, on the fp32
- * matrix cores; the environment variable GEMMA_HIP_PF_ATTN=bf3 (the split
- * kernel) or =f32, read at every launch, forces either.  The decode step's attention
- * is fp64 either way.  0 or 1 on an unknown mode. */
+ * pieces, 22 to 23 significant bits, each product summed from three piece
+ * products, fp32 accumulation: about 3e-7 of the result from the exact one, as
+ * the fp32 matrix cores are); workgroups whose keys hold more than that keeps (V
+ * over 2^6 apart between keys or dims, outliers in q or K, values that aren't
+ * finite) take three bf16 pieces, 24 bits, and six products.  Passes below
+ * about a GFLOP of attention a layer, and negative score scales, run on the fp32
+ * matrix cores; the environment variable GEMMA_HIP_PF_ATTN=split or =f32, read at
+ * every launch, forces either kernel.  The decode step's attention is fp64
+ * either way.  0 or 1 on an unknown mode. */
 #define GEMMA_HIP_ATTN_F64 0
 #define GEMMA_HIP_ATTN_F32 1
 int gemma_hip_decoder_set_attention(gemma_hip_decoder *dec, int mode);
@@ -495,11 +498,15 @@ int gemma_hip_vision_forward(gemma_hip_vision *vis, const float *img, float *out
  *     computes it (its summation order differs), so results agree with the
  *     exact form to fp32 rounding, amplified where a later int8 quantization
  *     flips.  The patch GEMM and the attention run on the f16 matrix cores
- *     in split precision: each fp32 operand is scaled by a power of two and split into two f16 pieces (22 significant bits), every
- *     product is summed from three piece products in fp32, and the result is
- *     closer to the exact one than with three bf16 pieces and six products
- *     (fewer fp32 roundings).  gemma_hip_vision_attention on a stream under
- *     capture, which can't allocate a workspace, takes the three-piece kernel;
+ *     in split precision: each fp32 operand is scaled by a power of two and
+ *     split into two f16 pieces (22 to 23 significant bits), every product is
+ *     summed from three piece products in fp32, and the result is closer to the
+ *     exact one than with three bf16 pieces and six products (fewer fp32
+ *     roundings).  Values that two pieces don't hold beside the others take
+ *     three bf16 pieces, as for gemma_hip_decoder_set_attention and
+ *     gemma_hip_matmul_f32.  gemma_hip_vision_attention on a stream under
+ *     capture or on hipStreamPerThread, where no workspace can be kept, takes
+ *     the three-piece kernel always;
  *     the environment variable GEMMA_HIP_VIS_ATTN=f32, read at every launch,
  *     selects the plain fp32 matrix-core kernel instead;
  *   GEMMA_HIP_ATTN_F64 -- fp64 (matrix cores for the attention), every

@@ -121,8 +121,8 @@ def test_prefill_attention_kernels_match_oracle(gh, case, monkeypatch):
     want = reference(q, kc, vc, n, pos0, nh, nkv, hd, slide, asc, sc_att, dense)
     dq, dk, dv = (torch.from_numpy(a).cuda() for a in (q, kc, vc))
     scale = float(np.abs(want).max())
-    # ATTN_F32 three times: the default choice (the split-bf16 kernel, or the
-    # fp32-MFMA one for the smallest passes) and each kernel forced per launch
+    # ATTN_F32 three times: the default choice (the split-f16 kernel, or the
+    # fp32-MFMA one for the smaller passes) and each kernel forced per launch
     # by GEMMA_HIP_PF_ATTN
     for mode, kernel, tol in ((ATTN_F64, "f64", ATT_F64_TOL), (ATTN_F32, "default", ATT_F32_TOL),
                               (ATTN_F32, "bf3", ATT_F32_TOL), (ATTN_F32, "f32", ATT_F32_TOL)):

@@ -656,7 +656,7 @@ def test_vision_error_level(gh, n, heads, hd):
 @pytest.mark.parametrize("n,pos0,nh,nkv,hd", [(300, 0, 4, 1, 256), (257, 500, 4, 1, 256),
                                               (500, 0, 4, 2, 128)])
 def test_prefill_error_level(gh, monkeypatch, n, pos0, nh, nkv, hd):
-    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "bf3")
+    monkeypatch.setenv("GEMMA_HIP_PF_ATTN", "split")
     q, kc, vc = _prefill_inputs(n, pos0, nh, nkv, hd, seed=n)
     args = (n, pos0, nh, nkv, hd, 0, 0.0, False)
     split = _rms(_prefill(gh, q, kc, vc, *args), _prefill_want(q, kc, vc, *args))

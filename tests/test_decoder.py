@@ -404,8 +404,7 @@ def test_prefill_default_attention_is_f32(gh, tmp_path, monkeypatch):
     case is F32_CASES' flip case at gemma-3-4b widths (200 tokens).  With the
     fp32-MFMA kernel (GEMMA_HIP_PF_ATTN=f32) the fp32 and fp64 modes' logits
     part there by the flip level, which shows that the default is not the
-    fp64 mode; the split-bf16 kernel (the default kernel) rounds each 32-key
-    value sum once, and at 200 tokens its logits meet the fp64 mode's, so the
+    fp64 mode; the split-f16 kernel's logits at 200 tokens meet the fp64 mode's, so the
     default is checked against ATTN_F32 under both kernels."""
     name, spec, (_, n) = F32_CASES["4b"]
     model = model_bin.read_bin(model_bin.write_bin(str(tmp_path / "m.bin"), name, seed=11,

@@ -235,7 +235,7 @@ def test_vision_attention_kernels_match_oracle(gh, case, monkeypatch):
     qkv, bias, want = _attention_inputs(n, heads, dim, seed=n + heads)
     dq, db = torch.from_numpy(qkv).cuda(), torch.from_numpy(bias).cuda()
     scale = float(np.abs(want).max())
-    # mode 1 twice: the split-bf16 kernel (the default) and the plain fp32
+    # mode 1 twice: the split-f16 kernel (the default) and the plain fp32
     # matrix-core kernel that GEMMA_HIP_VIS_ATTN=f32 selects per launch
     for mode, kernel, tol in ((0, "f64", ATT_F64_TOL), (1, "split", ATT_F32_TOL),
                               (1, "f32", ATT_F32_TOL)):
