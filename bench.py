@@ -428,8 +428,8 @@ def bench_decoder(torch, gh, name: str, prompt: int, steps: int) -> dict:
     """The prompt and the greedy decode fully on the GPU: `prompt` random token
     ids go through the batched prefill (gemma_hip_decoder_prefill; the median
     of TIMING_RUNS calls after a warm-up call that allocates its row buffers,
-    with the attention on the fp32 matrix cores, the default, and on the fp64
-    ones, the verification mode), then `steps` decode steps from the KV cache
+    with the attention in the fp32 mode, the default, and on the fp64 matrix
+    cores, the verification mode), then `steps` decode steps from the KV cache
     the default prefill filled are timed (one HIP graph launch each, tokens fed back on the device, one
     readback at the end; the median of TIMING_RUNS generations)."""
     import statistics
@@ -508,8 +508,8 @@ def bench_vision(torch, gh) -> dict:
     the whole SigLIP tower (gemma_hip_vision_forward: patch and position
     embedding, 27 encoder layers, post norm, pooling to 256 tokens, RMSNorm,
     projection to the gemma-3-4b width), random weights of that shape; the
-    median of five timed images after one untimed, with the attention on the
-    fp32 matrix cores (the default) and on the fp64 matrix cores (the
+    median of five timed images after one untimed, with the attention in the
+    fp32 mode (the default) and on the fp64 matrix cores (the
     verification mode, equal to the fp64 oracle; gemma_hip_vision_set_attention);
     then the same tower from fp32 weights (an unquantized 'U' file:
     gemma_hip_vision_create_f32, fp32 GEMMs on the split kernel)."""

@@ -374,8 +374,9 @@ int build_jobs(const char *fn, const gemma_hip_job *jobs, int njobs,
 // more with every chunk, and growing waits for the stream), kept for the next
 // call and freed by shutdown; past kAttnWsKeep bytes in all, the other streams'
 // go, and a call that needs more than that by itself, or whose handle names
-// several threads' streams, has its own, freed before it returns.  (Allocated and freed by every call, a 2048-row layer's took 7.5
-// ms beside 0.1 ms of kernels.)
+// several threads' streams, has its own, freed before it returns.  (Allocated
+// and freed by every call, a 2048-row layer's took 7.5 ms beside 0.1 ms of
+// kernels.)
 constexpr size_t kAttnWsKeep = (size_t)1 << 30;
 struct AttnWs {
   char *p = nullptr;

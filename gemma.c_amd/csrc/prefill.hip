@@ -609,8 +609,8 @@ __global__ __launch_bounds__(kNT, 2) void pf_attn_f32_kernel(PfAttn a) {
 // head's q heads at 128 / hn rows), and its tiles are the cache's keys packed by
 // attn_pack_kernel.  At head dim 256 a wave holds its queries' pieces and the
 // value sums in 256 registers, so each SIMD runs one wave and a CU one
-// workgroup (128 KB of LDS for the tiles); the tile loop overlaps its softmax with the next
-// tile's score products by itself.  A tile of 32 keys takes 2.7 us, 2.4 of them
+// workgroup (128 KB of LDS for the tiles); the tile loop overlaps its softmax
+// with the next tile's score products by itself.  A tile of 32 keys takes 2.7 us, 2.4 of them
 // with its loads and LDS reads taken out: the 96 products of a wave at the clock
 // that the chip holds under f16 products on all CUs.  gemma-3-4b, 2048 rows,
 // window 1024: packing 10.4, kernel 62.4, merge 11 us, where three bf16 pieces
@@ -1151,11 +1151,14 @@ int pf_key_split_plan(const PfAttn &b0, int hdim, int qb, int nrb, int kmax, int
 // The fp32 mode's kernel, read at every launch so that one process can time
 // or check both: GEMMA_HIP_PF_ATTN=f32 the fp32-MFMA one, =split (or =bf3, the
 // name of the kernel before it) the split-f16 one; unset, the split-f16 one from
-// kPbMinFlops of score and value products on.  Below, its packing launch and its longer prologue (about 15 us together)
-// outweigh its rate, 2.5 times the other's: whole prompt passes, fp32-MFMA
+// kPbMinFlops of score and value products on.  Below, its packing launch and its
+// longer prologue (about 15 us together) outweigh its rate, 2.5 times the
+// other's: whole prompt passes, fp32-MFMA
 // against split, gemma-3-270m (6 layers) at 512 rows (0.8 GFLOP a layer) 611
 // against 660 us, 700 rows 679 / 694; gemma-3-4b (2 layers) at 400 rows (0.66)
-// 578 / 592, 512 (1.07) 640 / 639, 700 (2.0) 669 / 652.
+// 578 / 592, 512 (1.07) 640 / 639, 700 (2.0) 669 / 652.  A few rows behind a long
+// cache have all of it packed and gain all the same (gemma-3-4b, 2 layers, 32
+// rows behind 8192 keys 506 / 456, behind 32768 988 / 777).
 constexpr double kPbMinFlops = 1.1e9;  // at head dim 256; in proportion below
 enum PfKind { kPfF32, kPfSplit, kPfAuto };
 PfKind pf_attn_kind() {

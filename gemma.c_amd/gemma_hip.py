@@ -128,7 +128,7 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 
 # attention arithmetic of the prompt passes and the vision tower
-# (GEMMA_HIP_ATTN_*): fp32 matrix cores (the default) or fp64 (verification)
+# (GEMMA_HIP_ATTN_*): fp32 (the default) or fp64 matrix cores (verification)
 ATTN_F64, ATTN_F32 = 0, 1
 _SIGS = {
     "gemma_hip_init": (_I, [_I]),

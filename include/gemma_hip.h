@@ -475,7 +475,7 @@ typedef struct {
 /* gemma_hip_vision_create for a 'U' file: forward_vision's !quant branches
  * (gemma.c:4454, 4488, 4562, 4604, 4626, 4709) on the device: pos
  * [npatch][dim] and proj [text_dim][dim] fp32 (registered), every
- * projection an fp32 matrix-core GEMM (gemm_fpx; fp64 in the verification
+ * projection an fp32 GEMM (gemma_hip_matmul_f32's; fp64 in the verification
  * mode of gemma_hip_vision_set_attention), no activation quantize.  Every
  * other vision entry point takes the result as it takes a W8A8 tower. */
 gemma_hip_vision *gemma_hip_vision_create_f32(const gemma_hip_vision_config *cfg,
